@@ -519,6 +519,17 @@ int vgdr_causal_conv1d(int dtype, const void *x, const void *weight, int weight_
                        const int32_t *cu_seqlens, int64_t B, int64_t T, int64_t D, int64_t n_seqs,
                        int kernel_size, int activation, hipStream_t stream);
 
+/* The short conv's gradients over B dense sequences of T tokens: from dy, the
+ * cotangent of vgdr_causal_conv1d's y without caches, dx [B * T, D] and (unless
+ * NULL) dweight [D, K], all in dtype, weight included, and 16-byte aligned.
+ * Sums in fp32, in a fixed order.  What the reference's autograd takes through
+ * ShortConv (opt.py:78-80, :96-100).  dx must not alias x or dy.  workspace:
+ * vgdr_causal_conv1d_bwd_workspace_size bytes, needed with dweight. */
+int64_t vgdr_causal_conv1d_bwd_workspace_size(int dtype, int64_t B, int64_t T, int64_t D, int kernel_size);
+int vgdr_causal_conv1d_bwd(int dtype, const void *x, const void *weight, const void *dy, void *dx,
+                           void *dweight, void *workspace, int64_t workspace_bytes, int64_t B, int64_t T,
+                           int64_t D, int kernel_size, int activation, hipStream_t stream);
+
 /* The output epilogue as one pass over n_rows rows of dv elements (a row per
  * (token, head)): out = epilogue(o, gate).  Replaces rms_norm_gated / the
  * RMSNorm x SiLU expression at linear_attention.py:820-825 after a chunked

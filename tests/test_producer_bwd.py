@@ -1,0 +1,65 @@
+"""The layer's producers and epilogue under autograd on the GPU: the kernels'
+gradients against torch's own autograd of the module's expressions in fp64.
+
+The bars are the repository's parity bars: rel_l2 <= 2e-2 for 16-bit inputs,
+1e-5 for fp32.
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+BARS = {torch.float32: 1e-5, torch.bfloat16: 2e-2, torch.float16: 2e-2}
+
+
+def _rel(x, ref):
+    x, ref = x.double().cpu(), ref.double().cpu()
+    return ((x - ref).norm() / ref.norm().clamp_min(1e-30)).item()
+
+
+def _check(label, got, want, dtype):
+    for name, x, ref in zip(label, got, want):
+        err = _rel(x, ref)
+        print(f'[parity] {name} rel_l2={err:.3e}', flush=True)
+        assert err <= BARS[dtype]
+
+
+def _grads(fn, inputs, cotangent):
+    xs = [t.detach().requires_grad_() for t in inputs]
+    y = fn(*xs)
+    return [y.detach()] + list(torch.autograd.grad(y, xs, cotangent.to(y.dtype)))
+
+
+# 16 x 8 token runs in one workgroup's rows, channel groups of 32 x 4 (the last one
+# partly filled), runs of 8, 16 and 32 tokens with remainders, sequences shorter than
+# the window, and the longest kernel (whose window is wider than the tokens of a step)
+@pytest.mark.gpu
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('B,T,D,K,act', [(1, 1, 8, 4, 'silu'), (3, 2, 40, 4, 'silu'), (2, 70, 192, 1, None),
+                                         (2, 129, 136, 3, 'silu'), (3, 1001, 512, 4, 'silu'), (1, 300, 64, 8, 'silu'),
+                                         (16, 1024, 1024, 4, None)])
+def test_short_conv_gradients(dtype, B, T, D, K, act):
+    from vagus_amd import ops
+    print(f'\n[case] short conv bwd {dtype} B={B} T={T} D={D} K={K} {act}', flush=True)
+    g = torch.Generator().manual_seed(T + D + K)
+    x, w, dy = (torch.randn(*s, generator=g).to(dtype).cuda() for s in ((B, T, D), (D, 1, K), (B, T, D)))
+    got = _grads(lambda x, w: ops.short_conv(x, w, act), (x, w), dy)
+    assert type(got[0]) is torch.Tensor
+    want = _grads(lambda x, w: ops.short_conv_expression(x, w, act), (x.cpu().double(), w.cpu().double()), dy.cpu())
+    _check(('y', 'dx', 'dw'), got, want, dtype)
+
+
+@pytest.mark.gpu
+def test_short_conv_second_derivative():
+    """create_graph: the kernel's backward differentiated again equals torch's."""
+    from vagus_amd import ops
+    g = torch.Generator().manual_seed(3)
+    x, w, dy = (torch.randn(*s, generator=g).cuda() for s in ((2, 9, 8), (8, 1, 4), (2, 9, 8)))
+
+    def second(fn, x, w, dy):
+        x, w = x.requires_grad_(), w.requires_grad_()
+        dx, dw = torch.autograd.grad(fn(x, w, 'silu'), (x, w), dy, create_graph=True)
+        return torch.autograd.grad(dx.square().sum() + dw.square().sum(), (x, w))
+
+    got = second(ops.short_conv, x.clone(), w.clone(), dy)
+    want = second(ops.short_conv_expression, x.cpu().double(), w.cpu().double(), dy.cpu().double())
+    _check(('ddx', 'ddw'), got, want, torch.float32)

@@ -990,6 +990,55 @@ int vgdr_causal_conv1d(int dtype, const void *x, const void *weight, int weight_
     return hip_status(vgdr::causal_conv(dtype, p, stream), "vgdr_causal_conv1d launch");
 }
 
+static int check_conv_bwd(const char *fn, int dtype, int64_t B, int64_t T, int64_t D, int kernel_size) {
+    if (dtype != VGDR_F32 && dtype != VGDR_BF16 && dtype != VGDR_F16)
+        return fail(VGDR_ERR_INVALID, "%s: unknown dtype %d", fn, dtype);
+    if (kernel_size < 1 || kernel_size > 8)
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: kernel_size=%d (supported: 1..8)", fn, kernel_size);
+    if (B < 0 || T < 0 || D <= 0) return fail(VGDR_ERR_INVALID, "%s: bad sizes", fn);
+    const int64_t ve = dtype == VGDR_F32 ? 4 : 8;
+    if (D % ve) return fail(VGDR_ERR_UNSUPPORTED, "%s: D=%lld (must be a multiple of %lld)", fn, (long long)D, (long long)ve);
+    if (T > 0x7fffff00LL || (B > 0 && T > 0 && B > 0x7fffffffffffLL / T / D))
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: sequences too long", fn);
+    return VGDR_OK;
+}
+
+int64_t vgdr_causal_conv1d_bwd_workspace_size(int dtype, int64_t B, int64_t T, int64_t D, int kernel_size) {
+    g_err[0] = 0;
+    if (check_conv_bwd("vgdr_causal_conv1d_bwd_workspace_size", dtype, B, T, D, kernel_size)) return 0;
+    return B * T == 0 ? 0 : 4 * vgdr::conv_bwd_part_floats(B, T, D, kernel_size);
+}
+
+int vgdr_causal_conv1d_bwd(int dtype, const void *x, const void *weight, const void *dy, void *dx, void *dweight,
+                           void *workspace, int64_t workspace_bytes, int64_t B, int64_t T, int64_t D,
+                           int kernel_size, int activation, hipStream_t stream) {
+    g_err[0] = 0;
+    const char *fn = "vgdr_causal_conv1d_bwd";
+    int rc = check_conv_bwd(fn, dtype, B, T, D, kernel_size);
+    if (rc) return rc;
+    if (activation != 0 && activation != 1) return fail(VGDR_ERR_INVALID, "%s: activation %d (0 none, 1 silu)", fn, activation);
+    if (B * T == 0) return VGDR_OK;
+    if (!x || !weight || !dy || !dx) return fail(VGDR_ERR_INVALID, "%s: x, weight, dy and dx are required", fn);
+    if (!aligned16(x) || !aligned16(weight) || !aligned16(dy) || !aligned16(dx) || !aligned16(workspace))
+        return fail(VGDR_ERR_INVALID, "%s: x, weight, dy, dx and workspace must be 16-byte aligned", fn);
+    if (dx == x || dx == dy) return fail(VGDR_ERR_INVALID, "%s: dx must not alias x or dy", fn);
+    if (dweight && (!workspace || workspace_bytes < vgdr_causal_conv1d_bwd_workspace_size(dtype, B, T, D, kernel_size)))
+        return fail(VGDR_ERR_INVALID, "%s: workspace too small", fn);
+    vgdr::ConvBwdParams p{};
+    p.x = x;
+    p.w = weight;
+    p.dy = dy;
+    p.dx = dx;
+    p.dw = dweight;
+    p.part = dweight ? reinterpret_cast<float *>(workspace) : nullptr;
+    p.T = T;
+    p.D = D;
+    p.n_seqs = B;
+    p.K = kernel_size;
+    p.silu = activation;
+    return hip_status(vgdr::causal_conv_bwd(dtype, p, stream), "vgdr_causal_conv1d_bwd launch");
+}
+
 int64_t vgdr_varlen_workspace_size(int64_t n_seqs) {
     return n_seqs < 0 ? 0 : (4 * n_seqs + 1) * (int64_t)sizeof(int32_t);
 }

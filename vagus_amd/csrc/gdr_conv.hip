@@ -36,6 +36,10 @@ __host__ __device__ __forceinline__ int conv_cg_per_group(int64_t ncg) {
     return ncg < CG_PER_GROUP ? (int)ncg : CG_PER_GROUP;
 }
 
+// the backward: channels per thread, and channel groups per workgroup
+constexpr int BWD_VE = 4;
+__host__ __device__ __forceinline__ int conv_bwd_cg(int64_t ncg) { return ncg < 32 ? (int)ncg : 32; }
+
 __device__ __forceinline__ int64_t clamp_tok(int32_t c, int64_t n_tokens) {
     return c < 0 ? 0 : (c > n_tokens ? n_tokens : c);
 }
@@ -259,6 +263,195 @@ hipError_t causal_conv(int dtype, const ConvParams &p, hipStream_t stream) {
     if (dtype == 1) return conv_t<__bf16>(p, stream);
     if (dtype == 2) return conv_t<_Float16>(p, stream);
     return conv_t<float>(p, stream);
+}
+
+// The gradients of the conv + SiLU, dense sequences: with h = conv(x) rounded to E,
+//     dh = dy * silu'(h),  dx[s] = sum_j w[j] dh[s + K - 1 - j],
+//     dw[j] = sum_t dh[t] x[t - K + 1 + j],
+// in one pass over x and dy (h is formed again: it costs K fused multiply-adds,
+// storing it would cost a third of the pass).  Bound by HBM: it reads x and dy
+// and writes dx once.  A thread owns four channels (at K = 4 about 110 VGPRs, four
+// waves per SIMD; eight channels in 16-byte loads take 214, two waves) for `run`
+// tokens of one sequence and slides over them four at a time; behind the run's end
+// it forms the dh of the K - 1 following tokens, which the last dx need.  A workgroup
+// is 32 such units x 8 consecutive runs, so those rows are in the CU's cache.
+// dw: VE x K fp32 sums per thread over the run, added over the workgroup's
+// runs in LDS, one partial row per workgroup, and conv_dw_kernel adds the
+// workgroups' rows in a fixed order: the same result every time, no atomics.
+// Measured at 32,768 tokens, K = 4, bf16: 36 us on average over D = 512, 512, 1024
+// (3.7 TB/s of the 3 x 2 bytes per element), where torch's conv1d + SiLU backward
+// took about 1.2 ms each.
+template <typename E, int K>
+__global__ void __launch_bounds__(256) causal_conv_bwd_kernel(const ConvBwdParams p) {
+    constexpr int VE = BWD_VE, SB = 4;
+    typedef E V __attribute__((ext_vector_type(VE)));
+    const int64_t ncg = p.D / VE;
+    const int cgw = conv_bwd_cg(ncg), rpw = 256 / cgw;
+    const int tid = threadIdx.x;
+    const uint32_t ncb = (uint32_t)((ncg + cgw - 1) / cgw);
+    const int64_t cg0 = (int64_t)(blockIdx.x % ncb) * cgw, cg = cg0 + tid % cgw;
+    const int64_t wgrow = blockIdx.x / ncb;
+    const int64_t run = wgrow * rpw + tid / cgw;
+    const int64_t seq = run / p.runs_per_seq;
+    const int t0 = (int)(run % p.runs_per_seq) * p.run, T = (int)p.T;
+    const bool live = tid < cgw * rpw && cg < ncg && seq < p.n_seqs;
+    const int64_t c0 = cg * VE;
+    float acc[VE * K];
+#pragma unroll
+    for (int i = 0; i < VE * K; ++i) acc[i] = 0.f;
+    if (live) {
+        const E *x = reinterpret_cast<const E *>(p.x) + seq * T * p.D + c0;
+        const E *dy = reinterpret_cast<const E *>(p.dy) + seq * T * p.D + c0;
+        E *dx = reinterpret_cast<E *>(p.dx) + seq * T * p.D + c0;
+        E wb[VE * K];
+        const V *wsrc = reinterpret_cast<const V *>(reinterpret_cast<const E *>(p.w) + c0 * K);
+        unroll<K>([&](auto i) __attribute__((always_inline)) {
+            const V u = wsrc[decltype(i)::value];
+            __builtin_memcpy(wb + VE * decltype(i)::value, &u, sizeof(V));
+        });
+        const int t1 = t0 + p.run < T ? t0 + p.run : T;
+        // rows outside the sequence read a row inside it and are zeroed afterwards
+        auto row = [&](const E *src, int t) __attribute__((always_inline)) -> V {
+            const bool in = t >= 0 && t < T;
+            const V v = *reinterpret_cast<const V *>(src + (int64_t)(in ? t : t0) * p.D);
+            return in ? v : V{};
+        };
+        V xw[K - 1 + SB];                    // inputs t - K + 1 .. t + SB - 1
+        float dh[K - 1 + SB][VE];            // dh of the same tokens
+        unroll<K - 1>([&](auto j) __attribute__((always_inline)) {
+            xw[j] = row(x, t0 - (K - 1) + decltype(j)::value);
+#pragma unroll
+            for (int e = 0; e < VE; ++e) dh[j][e] = 0.f;
+        });
+        for (int t = t0; t < t1 + K - 1; t += SB) {
+            V dyv[SB];
+            unroll<SB>([&](auto i) __attribute__((always_inline)) {
+                xw[K - 1 + i] = row(x, t + decltype(i)::value);
+                dyv[i] = row(dy, t + decltype(i)::value);
+            });
+            unroll<SB>([&](auto ii) __attribute__((always_inline)) {
+                constexpr int i = decltype(ii)::value;
+                const bool in = t + i < T, own = t + i < t1;
+#pragma unroll
+                for (int e = 0; e < VE; ++e) {
+                    float h = 0.f;
+#pragma unroll
+                    for (int j = 0; j < K; ++j) h += (float)wb[e * K + j] * (float)xw[i + j][e];
+                    float d = (float)dyv[i][e];
+                    if (p.silu) {
+                        h = (float)(E)h;
+                        const float s = sigmoidf_(h);
+                        d *= s * (1.f + h * (1.f - s));
+                    }
+                    d = in ? d : 0.f;
+                    dh[K - 1 + i][e] = d;
+                    const float da = own ? d : 0.f;
+#pragma unroll
+                    for (int j = 0; j < K; ++j) acc[e * K + j] += da * (float)xw[i + j][e];
+                }
+                V o;
+#pragma unroll
+                for (int e = 0; e < VE; ++e) {
+                    float s = 0.f;
+#pragma unroll
+                    for (int j = 0; j < K; ++j) s += (float)wb[e * K + j] * dh[i + K - 1 - j][e];
+                    o[e] = (E)s;
+                }
+                const int ts = t + i - (K - 1);                  // dx of the window's oldest token is complete
+                if (ts >= t0 && ts < t1) __builtin_nontemporal_store(o, reinterpret_cast<V *>(dx + (int64_t)ts * p.D));
+            });
+            unroll<K - 1>([&](auto j) __attribute__((always_inline)) {
+                xw[j] = xw[SB + j];
+#pragma unroll
+                for (int e = 0; e < VE; ++e) dh[j][e] = dh[SB + j][e];
+            });
+        }
+    }
+    if (!p.part) return;
+    __shared__ float red[256][VE + 1];
+    const int64_t row0 = wgrow * p.D * K;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < VE; ++e) red[tid][e] = acc[e * K + j];
+        __syncthreads();
+        if (tid < cgw * VE && cg0 + tid / VE < ncg) {
+            float s = 0.f;
+            for (int r = 0; r < rpw; ++r) s += red[r * cgw + tid / VE][tid % VE];
+            p.part[row0 + (cg0 * VE + tid) * K + j] = s;
+        }
+    }
+}
+
+// dw[i] = the sum of the workgroups' partial rows: 64 columns per workgroup, its
+// four waves take every fourth row
+template <typename E>
+__global__ void __launch_bounds__(256) conv_dw_kernel(const float *__restrict__ part, E *__restrict__ dw, int64_t n,
+                                                      int rows) {
+    __shared__ float red[4][64];
+    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x % 64;
+    const int w = threadIdx.x / 64;
+    float s = 0.f;
+    if (i < n)
+        for (int r = w; r < rows; r += 4) s += part[(int64_t)r * n + i];
+    red[w][threadIdx.x % 64] = s;
+    __syncthreads();
+    if (w == 0 && i < n) dw[i] = (E)(red[0][i % 64] + red[1][i % 64] + red[2][i % 64] + red[3][i % 64]);
+}
+
+// tokens per thread of the backward: the longest run (fewest partial rows, least
+// repeated work at its ends) that still gives four workgroups per CU, else 8
+static int conv_bwd_run(int64_t n_seqs, int64_t T, int64_t ncg, int64_t &runs_per_seq, int64_t &rows) {
+    const int cgw = conv_bwd_cg(ncg), rpw = 256 / cgw;
+    const int64_t ncb = (ncg + cgw - 1) / cgw;
+    for (int run = 32;; run /= 2) {
+        runs_per_seq = (T + run - 1) / run;
+        rows = (n_seqs * runs_per_seq + rpw - 1) / rpw;
+        if (run == 8 || rows * ncb >= 1024) return run;
+    }
+}
+
+int64_t conv_bwd_part_floats(int64_t n_seqs, int64_t T, int64_t D, int K) {
+    int64_t rps, rows;
+    conv_bwd_run(n_seqs, T, D / BWD_VE, rps, rows);
+    return rows * D * K;
+}
+
+template <typename E, int K>
+static hipError_t conv_bwd_k(ConvBwdParams p, hipStream_t stream) {
+    const int64_t ncg = p.D / BWD_VE;
+    const int cgw = conv_bwd_cg(ncg);
+    int64_t rows;
+    p.run = conv_bwd_run(p.n_seqs, p.T, ncg, p.runs_per_seq, rows);
+    const int64_t groups = (ncg + cgw - 1) / cgw * rows;
+    if (groups > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((causal_conv_bwd_kernel<E, K>), dim3((unsigned)groups), dim3(256), 0, stream, p);
+    if (p.part)
+        hipLaunchKernelGGL((conv_dw_kernel<E>), dim3((unsigned)((p.D * K + 63) / 64)), dim3(256), 0, stream, p.part,
+                           reinterpret_cast<E *>(p.dw), p.D * K, (int)rows);
+    return hipGetLastError();
+}
+
+template <typename E>
+static hipError_t conv_bwd_t(const ConvBwdParams &p, hipStream_t stream) {
+    switch (p.K) {
+        case 1: return conv_bwd_k<E, 1>(p, stream);
+        case 2: return conv_bwd_k<E, 2>(p, stream);
+        case 3: return conv_bwd_k<E, 3>(p, stream);
+        case 4: return conv_bwd_k<E, 4>(p, stream);
+        case 5: return conv_bwd_k<E, 5>(p, stream);
+        case 6: return conv_bwd_k<E, 6>(p, stream);
+        case 7: return conv_bwd_k<E, 7>(p, stream);
+        case 8: return conv_bwd_k<E, 8>(p, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t causal_conv_bwd(int dtype, const ConvBwdParams &p, hipStream_t stream) {
+    if (dtype == 1) return conv_bwd_t<__bf16>(p, stream);
+    if (dtype == 2) return conv_bwd_t<_Float16>(p, stream);
+    return conv_bwd_t<float>(p, stream);
 }
 
 }  // namespace vgdr

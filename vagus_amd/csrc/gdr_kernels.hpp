@@ -70,6 +70,18 @@ struct ConvParams {
     int n_seqs, K, w_f32, silu;
 };
 
+// The short conv's gradients over dense sequences: x, dy, dx [n_seqs * T, D];
+// w, dw [D, K] in the element type; part: the workgroups' partial dw rows
+// (conv_bwd_part_floats floats; NULL: dw is not wanted).  run, runs_per_seq: set
+// by causal_conv_bwd.
+struct ConvBwdParams {
+    const void *x, *w, *dy;
+    void *dx, *dw;
+    float *part;
+    int64_t T, D, n_seqs, runs_per_seq;
+    int K, silu, run;
+};
+
 struct ChunkParams {
     SeqGeom geo;
     const void *q, *k, *v;        // [n_tokens, H, dk|dv] in the element type
@@ -246,6 +258,8 @@ hipError_t scalar_gates(int dtype, const void *x, const void *w, const float *ne
 hipError_t swiglu(int dtype, const void *x, void *y, int64_t rows, int hidden, hipStream_t stream);
 
 hipError_t causal_conv(int dtype, const ConvParams &p, hipStream_t stream);
+int64_t conv_bwd_part_floats(int64_t n_seqs, int64_t T, int64_t D, int K);
+hipError_t causal_conv_bwd(int dtype, const ConvBwdParams &p, hipStream_t stream);
 
 hipError_t varlen_prepare(const int32_t *cu, int n_seqs, int64_t n_tokens, int chunk,
                           int32_t *ws, hipStream_t stream);

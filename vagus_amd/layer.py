@@ -35,10 +35,10 @@ rows: the continuous batching the reference's Generator cannot do
 
 Projections (W_q, W_k, W_v, W_g, W_o, the gate and beta maps) are torch
 GEMMs, and the scalar gate's softplus is torch elementwise work on the GPU, as
-in the reference.  Training: the scans differentiate through their HIP
-backward kernels; the short conv and the output epilogue have none, so when
-autograd needs their gradients they run as the reference's torch
-expressions on the GPU (inference always runs the kernels).
+in the reference.  Training: the scans and the short conv differentiate through
+their HIP backward kernels; the output epilogue has none, so when autograd
+needs its gradients it runs as the reference's torch expression on the GPU
+(inference always runs the kernels).
 """
 from __future__ import annotations
 
@@ -59,6 +59,15 @@ CONV_IMPLS = ('conv1d', 'shift', 'fla')
 
 def _autograd(*ts) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts)
+
+
+def _plain_module(m, cls) -> bool:
+    """Whether m is a cls whose call is its forward alone: no subclass
+    (parametrisations make one) and no hooks that a kernel in its place would
+    pass by."""
+    return (type(m) is cls and 'forward' not in m.__dict__ and not (
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+        or nn.modules.module._has_any_global_hook()))
 
 
 def parse_fusions(spec) -> frozenset:
@@ -114,7 +123,9 @@ class ShortConv(nn.Module):
         """x (B, L, D) -> (B, L, D), causal.  conv_cache (N, K, D): continue
         from it and advance it in place (a multi-token decode block)."""
         if _autograd(x, self.conv.weight) and cu_seqlens is None and conv_cache is None:
-            # the reference's 'conv1d' path (opt.py:78-80), for its gradients
+            if _plain_module(self.conv, nn.Conv1d):
+                return ops.short_conv(x, self.conv.weight, activation)
+            # a conv with hooks or of another class: its own call (opt.py:78-80)
             y = self.conv(F.pad(x.transpose(1, 2), (self.kernel - 1, 0))).transpose(1, 2)
             return F.silu(y) if activation is not None else y
         y, _ = ops.causal_conv1d(x, self.conv.weight, activation=activation, cu_seqlens=cu_seqlens,

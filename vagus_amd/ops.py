@@ -138,6 +138,22 @@ def _check_grad(*ts):
                                   'chunk_simple_gla, hip_scan, chunk_scan_vec); this call has no backward')
 
 
+def _kernel_autograd(*ts):
+    """Whether an autograd function over a kernel may stand for a torch
+    expression on these tensors: plain GPU tensors of one kernel type, and
+    nothing that has to see the expression itself (autocast, tracing or
+    compiling, a functorch transform, forward-mode AD, a dispatch mode)."""
+    t = ts[0]
+    if not (t.is_cuda and t.dtype in _DTYPES and t.numel() > 0):
+        return False
+    if any(type(x) not in (torch.Tensor, torch.nn.Parameter) or x.dtype != t.dtype or x.device != t.device
+           for x in ts):
+        return False
+    return not (torch.is_autocast_enabled('cuda') or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0)
+
+
 def _gate_activation_rows(f, fz):
     """The per-channel gate from its pre-activation f (B, T, H, dk) in fp32
     (linear_attention.py:722-734): -exp(A_log) softplus(f + dt_bias), or
@@ -1208,6 +1224,62 @@ def causal_conv1d(x, weight, bias=None, residual=None, initial_state=None, outpu
                                                   _ptr(y), _ptr(st_out), _ptr(cu), B, T, D, N, K,
                                                   0 if activation is None else 1, _stream(x.device)))
     return y, (st_out if output_final_state else None)
+
+
+def short_conv_expression(x, weight, activation):
+    """ShortConv in torch (opt.py:78-80, :96-100): the conv, then SiLU."""
+    D, K = x.shape[-1], weight.shape[-1]
+    y = F.conv1d(F.pad(x.transpose(1, 2), (K - 1, 0)), weight.reshape(D, 1, K), groups=D).transpose(1, 2)
+    return F.silu(y) if activation is not None else y
+
+
+class _ShortConvRule(torch.autograd.Function):
+    """causal_conv1d without caches, differentiable: forward
+    vgdr_causal_conv1d, backward vgdr_causal_conv1d_bwd, which forms the
+    pre-activation again from x.  A backward that is itself to be
+    differentiated (create_graph) runs through the torch expression."""
+
+    @staticmethod
+    def forward(ctx, x, weight, activation):
+        ctx.save_for_backward(x, weight)
+        ctx.activation = activation
+        return causal_conv1d(x, weight, activation=None if activation is None else 'silu')[0]
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            need = [t for t, n in zip((x, weight), ctx.needs_input_grad) if n]
+            grads = iter(torch.autograd.grad(short_conv_expression(x, weight, ctx.activation), need, dy,
+                                             create_graph=True))
+            return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:2]) + (None,)
+        B, T, D = x.shape
+        K = weight.shape[-1]
+        xa, wa, dya = _aligned(x), _aligned(weight), _aligned(dy)
+        dx = torch.empty_like(xa)
+        L = _lib.load()
+        dw = ws = None
+        nbytes = 0
+        if ctx.needs_input_grad[1]:
+            dw = torch.empty_like(wa)
+            nbytes = L.vgdr_causal_conv1d_bwd_workspace_size(_DTYPES[x.dtype], B, T, D, K)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        with torch.cuda.device(x.device):
+            _lib.check(L.vgdr_causal_conv1d_bwd(_DTYPES[x.dtype], _ptr(xa), _ptr(wa), _ptr(dya), _ptr(dx), _ptr(dw),
+                                                _ptr(ws), nbytes, B, T, D, K, 0 if ctx.activation is None else 1,
+                                                _stream(x.device)))
+        return dx, dw, None
+
+
+def short_conv(x, weight, activation=None):
+    """The short conv and its activation over x (B, T, D) with weight (D, 1, K),
+    differentiable: one kernel each way where the kernels take the tensors
+    (_kernel_autograd, D in 16-byte units, K <= 8), the torch expression
+    elsewhere."""
+    if (x.dim() == 3 and weight.shape[-1] <= 8 and _kernel_autograd(x, weight)
+            and x.shape[-1] % (16 // x.element_size()) == 0):
+        return _ShortConvRule.apply(x, weight, activation)
+    return short_conv_expression(x, weight, activation)
 
 
 def chunk_write_bwd(q, k, v, w, g, initial_state, do, dht=None, *, scale=None, cu_seqlens=None, chunk_size=64):
