@@ -539,6 +539,17 @@ int vgdr_causal_conv1d_bwd(int dtype, const void *x, const void *weight, const v
 int vgdr_norm_gate(int dtype, const void *o, const vgdr_epilogue *epilogue, void *out, int64_t n_rows,
                    int64_t dv, hipStream_t stream);
 
+/* The epilogue's gradients as one pass: from dy, the cotangent of
+ * vgdr_norm_gate's out, d_o and dgate [n_rows, dv] and dgamma [dv].  Everything in
+ * dtype (gamma included), 16-byte aligned, no gradient aliasing an input; sums in
+ * fp32, in a fixed order.  What the reference's autograd takes through the
+ * expression at linear_attention.py:825.  dv as vgdr_norm_gate's; workspace:
+ * vgdr_norm_gate_bwd_workspace_size bytes. */
+int64_t vgdr_norm_gate_bwd_workspace_size(int dtype, int64_t n_rows, int64_t dv);
+int vgdr_norm_gate_bwd(int dtype, const void *o, const void *gate, const void *gamma, float eps,
+                       const void *dy, void *d_o, void *dgate, void *dgamma, void *workspace,
+                       int64_t workspace_bytes, int64_t n_rows, int64_t dv, hipStream_t stream);
+
 /* The pre-norm blocks' RMSNorm (infra/components/norm_layer.py:15-23) over rows
  * rows of dim elements, with the residual add in front of it that the blocks
  * make before each norm (infra/components/block.py:57-59, :85-87):

@@ -63,3 +63,37 @@ def test_short_conv_second_derivative():
     got = second(ops.short_conv, x.clone(), w.clone(), dy)
     want = second(ops.short_conv_expression, x.cpu().double(), w.cpu().double(), dy.cpu().double())
     _check(('ddx', 'ddw'), got, want, torch.float32)
+
+
+# one row, rows that leave a workgroup's last pass partly filled, more rows than the grid takes
+# in one pass (1024 workgroups x 256 / lanes rows), the shortest and the longest row
+@pytest.mark.gpu
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('rows,dv', [(1, 128), (37, 8), (1001, 256), (20001, 128), (70001, 64), (513, -64)])
+def test_norm_gate_gradients(dtype, rows, dv):
+    from vagus_amd import ops
+    dv = dv if dv > 0 else -dv * (4 if dtype == torch.float32 else 8)       # 64 lanes: the longest
+    print(f'\n[case] epilogue bwd {dtype} rows={rows} dv={dv}', flush=True)
+    g = torch.Generator().manual_seed(rows + dv)
+    o, gate, dy = (torch.randn(rows, dv, generator=g).to(dtype).cuda() for _ in range(3))
+    gamma = (torch.rand(dv, generator=g) + 0.5).to(dtype).cuda()
+    got = _grads(lambda *a: ops.norm_gate(*a, 1e-6), (o, gate, gamma), dy)
+    want = _grads(lambda *a: ops.norm_gate_expression(*a, 1e-6), [t.cpu().double() for t in (o, gate, gamma)], dy.cpu())
+    _check(('y', 'do', 'dgate', 'dgamma'), got, want, dtype)
+
+
+@pytest.mark.gpu
+def test_norm_gate_second_derivative():
+    from vagus_amd import ops
+    g = torch.Generator().manual_seed(4)
+    o, gate, dy = (torch.randn(5, 16, generator=g).cuda() for _ in range(3))
+    gamma = torch.rand(16, generator=g).cuda() + 0.5
+
+    def second(fn, o, gate, gamma, dy):
+        xs = [t.requires_grad_() for t in (o, gate, gamma)]
+        d = torch.autograd.grad(fn(*xs, 1e-6), xs, dy, create_graph=True)
+        return torch.autograd.grad(sum(x.square().sum() for x in d), xs)
+
+    got = second(ops.norm_gate, o.clone(), gate.clone(), gamma.clone(), dy)
+    want = second(ops.norm_gate_expression, *(t.cpu().double() for t in (o, gate, gamma, dy)))
+    _check(('ddo', 'ddgate', 'ddgamma'), got, want, torch.float32)

@@ -876,6 +876,58 @@ int vgdr_norm_gate(int dtype, const void *o, const vgdr_epilogue *epilogue, void
     return hip_status(vgdr::norm_gate(dtype, o, ep, out, n_rows, (int)dv, stream), "vgdr_norm_gate launch");
 }
 
+static int check_norm_gate_rows(const char *fn, int dtype, int64_t n_rows, int64_t dv) {
+    if (dtype != VGDR_F32 && dtype != VGDR_BF16 && dtype != VGDR_F16)
+        return fail(VGDR_ERR_INVALID, "%s: unknown dtype %d", fn, dtype);
+    const int64_t ve = dtype == VGDR_F32 ? 4 : 8, lpr = dv / ve;
+    if (dv <= 0 || dv % ve || lpr > 64 || (lpr & (lpr - 1)))
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: row length %lld (supported: %lld x a power of two, at most %lld)", fn,
+                    (long long)dv, (long long)ve, (long long)(64 * ve));
+    if (n_rows < 0 || n_rows > (int64_t)0x7fffffffLL * 256 / lpr)
+        return fail(VGDR_ERR_INVALID, "%s: n_rows=%lld", fn, (long long)n_rows);
+    return VGDR_OK;
+}
+
+int64_t vgdr_norm_gate_bwd_workspace_size(int dtype, int64_t n_rows, int64_t dv) {
+    g_err[0] = 0;
+    if (check_norm_gate_rows("vgdr_norm_gate_bwd_workspace_size", dtype, n_rows, dv)) return 0;
+    return 4 * (int64_t)vgdr::norm_gate_bwd_blocks(dtype, n_rows, (int)dv) * dv;
+}
+
+int vgdr_norm_gate_bwd(int dtype, const void *o, const void *gate, const void *gamma, float eps, const void *dy,
+                       void *d_o, void *dgate, void *dgamma, void *workspace, int64_t workspace_bytes, int64_t n_rows,
+                       int64_t dv, hipStream_t stream) {
+    g_err[0] = 0;
+    const char *fn = "vgdr_norm_gate_bwd";
+    int rc = check_norm_gate_rows(fn, dtype, n_rows, dv);
+    if (rc) return rc;
+    if (!(eps > 0.f)) return fail(VGDR_ERR_INVALID, "%s: eps must be positive", fn);
+    if (n_rows == 0) return VGDR_OK;
+    if (!o || !gate || !gamma || !dy || !d_o || !dgate || !dgamma)
+        return fail(VGDR_ERR_INVALID, "%s: every tensor is required", fn);
+    if (!aligned16(o) || !aligned16(gate) || !aligned16(gamma) || !aligned16(dy) || !aligned16(d_o) ||
+        !aligned16(dgate) || !aligned16(dgamma))
+        return fail(VGDR_ERR_INVALID, "%s: every tensor must be 16-byte aligned", fn);
+    for (const void *in : {o, gate, gamma, dy})
+        if (in == d_o || in == dgate || in == dgamma)
+            return fail(VGDR_ERR_INVALID, "%s: the gradients must not alias the inputs", fn);
+    if (!workspace || workspace_bytes < vgdr_norm_gate_bwd_workspace_size(dtype, n_rows, dv))
+        return fail(VGDR_ERR_INVALID, "%s: workspace too small", fn);
+    vgdr::NormGateBwd p{};
+    p.o = o;
+    p.gate = gate;
+    p.gamma = gamma;
+    p.dy = dy;
+    p.d_o = d_o;
+    p.dgate = dgate;
+    p.dgamma = dgamma;
+    p.part = reinterpret_cast<float *>(workspace);
+    p.eps = eps;
+    p.n_rows = n_rows;
+    p.dv = (int)dv;
+    return hip_status(vgdr::norm_gate_bwd(dtype, p, stream), "vgdr_norm_gate_bwd launch");
+}
+
 int vgdr_rms_norm(int dtype, const void *x, const void *residual, void *x_out, const void *gamma, void *y,
                   int64_t rows, int64_t dim, float eps, hipStream_t stream) {
     g_err[0] = 0;

@@ -276,7 +276,7 @@ hipError_t causal_conv(int dtype, const ConvParams &p, hipStream_t stream) {
 // it forms the dh of the K - 1 following tokens, which the last dx need.  A workgroup
 // is 32 such units x 8 consecutive runs, so those rows are in the CU's cache.
 // dw: VE x K fp32 sums per thread over the run, added over the workgroup's
-// runs in LDS, one partial row per workgroup, and conv_dw_kernel adds the
+// runs in LDS, one partial row per workgroup, and row_sums_kernel adds the
 // workgroups' rows in a fixed order: the same result every time, no atomics.
 // Measured at 32,768 tokens, K = 4, bf16: 36 us on average over D = 512, 512, 1024
 // (3.7 TB/s of the 3 x 2 bytes per element), where torch's conv1d + SiLU backward
@@ -384,22 +384,6 @@ __global__ void __launch_bounds__(256) causal_conv_bwd_kernel(const ConvBwdParam
     }
 }
 
-// dw[i] = the sum of the workgroups' partial rows: 64 columns per workgroup, its
-// four waves take every fourth row
-template <typename E>
-__global__ void __launch_bounds__(256) conv_dw_kernel(const float *__restrict__ part, E *__restrict__ dw, int64_t n,
-                                                      int rows) {
-    __shared__ float red[4][64];
-    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x % 64;
-    const int w = threadIdx.x / 64;
-    float s = 0.f;
-    if (i < n)
-        for (int r = w; r < rows; r += 4) s += part[(int64_t)r * n + i];
-    red[w][threadIdx.x % 64] = s;
-    __syncthreads();
-    if (w == 0 && i < n) dw[i] = (E)(red[0][i % 64] + red[1][i % 64] + red[2][i % 64] + red[3][i % 64]);
-}
-
 // tokens per thread of the backward: the longest run (fewest partial rows, least
 // repeated work at its ends) that still gives four workgroups per CU, else 8
 static int conv_bwd_run(int64_t n_seqs, int64_t T, int64_t ncg, int64_t &runs_per_seq, int64_t &rows) {
@@ -427,10 +411,9 @@ static hipError_t conv_bwd_k(ConvBwdParams p, hipStream_t stream) {
     const int64_t groups = (ncg + cgw - 1) / cgw * rows;
     if (groups > 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL((causal_conv_bwd_kernel<E, K>), dim3((unsigned)groups), dim3(256), 0, stream, p);
-    if (p.part)
-        hipLaunchKernelGGL((conv_dw_kernel<E>), dim3((unsigned)((p.D * K + 63) / 64)), dim3(256), 0, stream, p.part,
-                           reinterpret_cast<E *>(p.dw), p.D * K, (int)rows);
-    return hipGetLastError();
+    const int dtype = std::is_same<E, float>::value ? 0 : std::is_same<E, __bf16>::value ? 1 : 2;
+    const hipError_t rc = hipGetLastError();
+    return rc != hipSuccess || !p.part ? rc : row_sums(dtype, p.part, p.dw, p.D * K, rows, stream);
 }
 
 template <typename E>

@@ -88,6 +88,140 @@ hipError_t norm_gate(int dtype, const void *o, const Epilogue &ep, void *out, in
     return norm_gate_t<float>(o, ep, out, n_rows, dv, stream);
 }
 
+// The epilogue's gradients: with r = rsqrt(mean o^2 + eps), n = o r and s = SiLU(gate),
+// from dy
+//     do = r (m - n mean(m n)),  m = dy gamma s
+//     dgate = dy n gamma SiLU'(gate),  dgamma = sum over rows of dy n s
+// in one pass that reads o, gate and dy and writes do and dgate: bound by HBM.  The
+// lane layout is the forward's; a workgroup walks over rows (its threads keep the
+// channels they sum dgamma for), writes one partial dgamma row, and row_sums_kernel adds
+// the workgroups' rows in a fixed order.  Measured at 131,072 rows of 256, bf16: 59 us
+// (5.7 TB/s of the five tensors), where torch's expression and its autograd took 0.9 ms.
+template <typename E, int LPR>
+__global__ void __launch_bounds__(256) norm_gate_bwd_kernel(const E *__restrict__ o, const E *__restrict__ gate,
+                                                            const E *__restrict__ gamma, float eps,
+                                                            const E *__restrict__ dy, E *__restrict__ d_o,
+                                                            E *__restrict__ dgate, float *__restrict__ part,
+                                                            int64_t n_rows) {
+    constexpr int VE = 16 / (int)sizeof(E), DV = LPR * VE, RPB = 256 / LPR;
+    typedef E V __attribute__((ext_vector_type(VE)));
+    const int tid = threadIdx.x, lane = tid % LPR;
+    const V wv = reinterpret_cast<const V *>(gamma)[lane];
+    float dw[VE];
+#pragma unroll
+    for (int e = 0; e < VE; ++e) dw[e] = 0.f;
+    for (int64_t row0 = (int64_t)blockIdx.x * RPB; row0 < n_rows; row0 += (int64_t)gridDim.x * RPB) {
+        const int64_t row = row0 + tid / LPR;
+        const bool live = row < n_rows;
+        const int64_t off = (live ? row : n_rows - 1) * DV + lane * VE;      // groups past the end re-read the last row
+        const V ov = __builtin_nontemporal_load(reinterpret_cast<const V *>(o + off));
+        const V gv = __builtin_nontemporal_load(reinterpret_cast<const V *>(gate + off));
+        const V dv = __builtin_nontemporal_load(reinterpret_cast<const V *>(dy + off));
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < VE; ++e) ss += (float)ov[e] * (float)ov[e];
+#pragma unroll
+        for (int k = 1; k < LPR; k <<= 1) ss += __shfl_xor(ss, k);
+        const float r = rsqrtf(ss * (1.f / DV) + eps);
+        float n[VE], m[VE], mn = 0.f;
+        V dg;
+#pragma unroll
+        for (int e = 0; e < VE; ++e) {
+            const float w = (float)wv[e], x = (float)gv[e], d = (float)dv[e], sg = sigmoidf_(x), s = x * sg;
+            n[e] = (float)ov[e] * r;
+            m[e] = d * w * s;
+            mn += m[e] * n[e];
+            dg[e] = (E)(d * n[e] * w * (sg * (1.f + x * (1.f - sg))));
+            dw[e] += live ? d * n[e] * s : 0.f;
+        }
+#pragma unroll
+        for (int k = 1; k < LPR; k <<= 1) mn += __shfl_xor(mn, k);
+        mn *= 1.f / DV;
+        V dx;
+#pragma unroll
+        for (int e = 0; e < VE; ++e) dx[e] = (E)(r * (m[e] - n[e] * mn));
+        if (live) {
+            __builtin_nontemporal_store(dx, reinterpret_cast<V *>(d_o + off));
+            __builtin_nontemporal_store(dg, reinterpret_cast<V *>(dgate + off));
+        }
+    }
+    __shared__ float red[256][VE + 1];
+#pragma unroll
+    for (int e = 0; e < VE; ++e) red[tid][e] = dw[e];
+    __syncthreads();
+    for (int c = tid; c < DV; c += 256) {
+        float s = 0.f;
+        for (int k = 0; k < RPB; ++k) s += red[k * LPR + c / VE][c % VE];
+        part[(int64_t)blockIdx.x * DV + c] = s;
+    }
+}
+
+// out[i] = the sum over the rows of part [rows, n] in a fixed order: 64 columns per
+// workgroup, its 16 waves take every 16th row (with four waves, 64 to 128 rows of
+// 2,048 to 4,096 columns took 17 us of dependent loads)
+template <typename E>
+__global__ void __launch_bounds__(1024) row_sums_kernel(const float *__restrict__ part, E *__restrict__ out, int64_t n,
+                                                        int64_t rows) {
+    __shared__ float red[16][64];
+    const int c = threadIdx.x % 64, w = threadIdx.x / 64;
+    const int64_t i = (int64_t)blockIdx.x * 64 + c;
+    float s = 0.f;
+    if (i < n) {
+#pragma unroll 4
+        for (int64_t r = w; r < rows; r += 16) s += part[r * n + i];
+    }
+    red[w][c] = s;
+    __syncthreads();
+    if (w == 0 && i < n) {
+#pragma unroll
+        for (int k = 1; k < 16; ++k) s += red[k][c];
+        out[i] = (E)s;
+    }
+}
+
+hipError_t row_sums(int dtype, const float *part, void *out, int64_t n, int64_t rows, hipStream_t stream) {
+    const int64_t groups = (n + 63) / 64;
+    if (groups > 0x7fffffff) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)groups), block(1024);
+    if (dtype == 1) hipLaunchKernelGGL((row_sums_kernel<__bf16>), grid, block, 0, stream, part, (__bf16 *)out, n, rows);
+    else if (dtype == 2) hipLaunchKernelGGL((row_sums_kernel<_Float16>), grid, block, 0, stream, part, (_Float16 *)out, n, rows);
+    else hipLaunchKernelGGL((row_sums_kernel<float>), grid, block, 0, stream, part, (float *)out, n, rows);
+    return hipGetLastError();
+}
+
+// workgroups of the epilogue's backward, one partial dgamma row each: four per CU keep
+// HBM busy, and more only lengthen the sum over the partial rows
+int norm_gate_bwd_blocks(int dtype, int64_t n_rows, int dv) {
+    const int64_t rpb = 256 / (dv / (dtype == 0 ? 4 : 8)), need = (n_rows + rpb - 1) / rpb;
+    return (int)(need < 1024 ? need : 1024);
+}
+
+template <typename E>
+static hipError_t norm_gate_bwd_t(int dtype, const NormGateBwd &p, hipStream_t stream) {
+    const int lpr = p.dv / (16 / (int)sizeof(E));
+    const int blocks = norm_gate_bwd_blocks(dtype, p.n_rows, p.dv);
+#define VGDR_NGB(L)                                                                                              \
+    case L:                                                                                                       \
+        hipLaunchKernelGGL((norm_gate_bwd_kernel<E, L>), dim3((unsigned)blocks), dim3(256), 0, stream,            \
+                           reinterpret_cast<const E *>(p.o), reinterpret_cast<const E *>(p.gate),                 \
+                           reinterpret_cast<const E *>(p.gamma), p.eps, reinterpret_cast<const E *>(p.dy),        \
+                           reinterpret_cast<E *>(p.d_o), reinterpret_cast<E *>(p.dgate), p.part, p.n_rows);       \
+        break;
+    switch (lpr) {
+        VGDR_NGB(1) VGDR_NGB(2) VGDR_NGB(4) VGDR_NGB(8) VGDR_NGB(16) VGDR_NGB(32) VGDR_NGB(64)
+        default: return hipErrorInvalidValue;
+    }
+#undef VGDR_NGB
+    const hipError_t rc = hipGetLastError();
+    return rc != hipSuccess ? rc : row_sums(dtype, p.part, p.dgamma, p.dv, blocks, stream);
+}
+
+hipError_t norm_gate_bwd(int dtype, const NormGateBwd &p, hipStream_t stream) {
+    if (dtype == 1) return norm_gate_bwd_t<__bf16>(dtype, p, stream);
+    if (dtype == 2) return norm_gate_bwd_t<_Float16>(dtype, p, stream);
+    return norm_gate_bwd_t<float>(dtype, p, stream);
+}
+
 // The pre-norm blocks' RMSNorm (norm_layer.py:15-23) with the residual add in
 // front of it (block.py:57-59, :85-87): h = x + res rounded to E (the stream's
 // new value, stored to x_out), then y = E(E(h * rsqrt(mean(h^2) + eps)) * gamma),

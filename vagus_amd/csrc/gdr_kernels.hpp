@@ -242,6 +242,22 @@ hipError_t recurrent_fwd(int dtype, int dk, int dv, int gate_vector, const RecPa
 hipError_t norm_gate(int dtype, const void *o, const Epilogue &ep, void *out, int64_t n_rows, int dv,
                      hipStream_t stream);
 
+// out[i] (element type) = the sum over the rows of part [rows, n], in a fixed order
+hipError_t row_sums(int dtype, const float *part, void *out, int64_t n, int64_t rows, hipStream_t stream);
+
+// The epilogue's gradients over n_rows rows: everything in the element type but
+// part, norm_gate_bwd_blocks() rows of dv floats.  dv as norm_gate's.
+struct NormGateBwd {
+    const void *o, *gate, *gamma, *dy;
+    void *d_o, *dgate, *dgamma;
+    float *part;
+    float eps;
+    int64_t n_rows;
+    int dv;
+};
+int norm_gate_bwd_blocks(int dtype, int64_t n_rows, int dv);
+hipError_t norm_gate_bwd(int dtype, const NormGateBwd &p, hipStream_t stream);
+
 // The blocks' RMSNorm with an optional residual add first (res, x_out may be
 // null): x_out = x + res, y = RMSNorm(x + res) * gamma over rows of dim
 // elements.  dim / (16 / sizeof(E)) <= 2048.

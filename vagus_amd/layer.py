@@ -35,10 +35,10 @@ rows: the continuous batching the reference's Generator cannot do
 
 Projections (W_q, W_k, W_v, W_g, W_o, the gate and beta maps) are torch
 GEMMs, and the scalar gate's softplus is torch elementwise work on the GPU, as
-in the reference.  Training: the scans and the short conv differentiate through
-their HIP backward kernels; the output epilogue has none, so when autograd
-needs its gradients it runs as the reference's torch expression on the GPU
-(inference always runs the kernels).
+in the reference.  Training: the scans, the short conv and the output epilogue
+differentiate through their HIP backward kernels; where those do not stand for
+the module's expression (autocast, tracing, functorch transforms, hooks on the
+submodule) the conv and the epilogue run as the reference's torch expressions.
 """
 from __future__ import annotations
 
@@ -357,7 +357,12 @@ class GatedDeltaNet(nn.Module):
         B, L = x.shape[0], x.shape[1]
         gate = self.wg(x).view(B, L, self.head_count, self.value_head_dim)
         if _autograd(o, gate, self.o_norm.gamma):
-            o = (self.o_norm(o.to(gate.dtype)) * F.silu(gate)).reshape(B, L, -1)        # :825
+            o = o.to(gate.dtype)
+            if _plain_module(self.o_norm, RMSNorm):
+                o = ops.norm_gate(o, gate, self.o_norm.gamma, self.o_norm.eps)
+            else:                                               # its own call (:825)
+                o = self.o_norm(o) * F.silu(gate)
+            o = o.reshape(B, L, -1)
         else:
             o = ops.rms_norm_gated(o.to(gate.dtype), gate, self.o_norm.gamma, eps=self.o_norm.eps).reshape(B, L, -1)
         return self.wo(o) if self.out_proj else o

@@ -797,6 +797,63 @@ def rms_norm_gated(x, g, weight, bias=None, activation='swish', residual=None, p
     return _norm_gate(x, _Epilogue(g, weight, eps))
 
 
+def norm_gate_expression(o, gate, gamma, eps):
+    """The output epilogue in torch (linear_attention.py:825, norm_layer.py:15-24)."""
+    h = o.to(torch.promote_types(o.dtype, torch.float32))
+    h = h * torch.rsqrt(h.pow(2).mean(dim=-1, keepdim=True) + eps)
+    return h.to(o.dtype) * gamma * F.silu(gate)
+
+
+def _row_lanes(t):
+    """Whether the row kernels take rows of t's last dim: 16-byte units, a power of two of them up to 64."""
+    n, r = divmod(t.shape[-1] * t.element_size(), 16)
+    return r == 0 and 1 <= n <= 64 and n & (n - 1) == 0
+
+
+class _NormGateRule(torch.autograd.Function):
+    """rms_norm_gated, differentiable: forward vgdr_norm_gate, backward
+    vgdr_norm_gate_bwd, both over o and gate as they are (nothing else is kept
+    for the backward).  A backward that is itself to be differentiated
+    (create_graph) runs through the torch expression."""
+
+    @staticmethod
+    def forward(ctx, o, gate, gamma, eps):
+        ctx.save_for_backward(o, gate, gamma)
+        ctx.eps = eps
+        return _norm_gate(o, _Epilogue(gate, gamma, eps))
+
+    @staticmethod
+    def backward(ctx, dy):
+        o, gate, gamma = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            need = [t for t, n in zip((o, gate, gamma), ctx.needs_input_grad) if n]
+            grads = iter(torch.autograd.grad(norm_gate_expression(o, gate, gamma, ctx.eps), need, dy,
+                                             create_graph=True))
+            return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:3]) + (None,)
+        oa, ga, wa, dya = _aligned(o), _aligned(gate), _aligned(gamma), _aligned(dy)
+        do, dgate, dgamma = torch.empty_like(oa), torch.empty_like(ga), torch.empty_like(wa)
+        dv = o.shape[-1]
+        rows = o.numel() // dv
+        L = _lib.load()
+        nbytes = L.vgdr_norm_gate_bwd_workspace_size(_DTYPES[o.dtype], rows, dv)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=o.device)
+        with torch.cuda.device(o.device):
+            _lib.check(L.vgdr_norm_gate_bwd(_DTYPES[o.dtype], _ptr(oa), _ptr(ga), _ptr(wa), ctx.eps, _ptr(dya),
+                                            _ptr(do), _ptr(dgate), _ptr(dgamma), _ptr(ws), nbytes, rows, dv,
+                                            _stream(o.device)))
+        return do, dgate, dgamma, None
+
+
+def norm_gate(o, gate, gamma, eps):
+    """RMSNorm(o) * gamma * SiLU(gate) over the last dim, differentiable: one
+    kernel each way where the kernels take the tensors (_kernel_autograd,
+    _row_lanes), the torch expression elsewhere."""
+    if (o.shape == gate.shape and gamma.dim() == 1 and gamma.shape[0] == o.shape[-1] and eps > 0
+            and _kernel_autograd(o, gate, gamma) and _row_lanes(o)):
+        return _NormGateRule.apply(o, gate, gamma, eps)
+    return norm_gate_expression(o, gate, gamma, eps)
+
+
 def rms_norm(x, weight, eps: float = 1e-6, residual=None, out_residual=None):
     """The blocks' RMSNorm (infra/components/norm_layer.py:15-23) in one HIP
     pass over the last dim: dtype(dtype(h rsqrt(mean h^2 + eps)) * weight).
