@@ -550,6 +550,13 @@ int vgdr_norm_gate_bwd(int dtype, const void *o, const void *gate, const void *g
                        const void *dy, void *d_o, void *dgate, void *dgamma, void *workspace,
                        int64_t workspace_bytes, int64_t n_rows, int64_t dv, hipStream_t stream);
 
+/* Rows of d elements to unit length, the q, k producer (linear_attention.py:
+ * 703-706): out = x rsqrt(sum x^2 + eps) when dy is NULL, else its gradient
+ * r dy - r^3 x <x, dy>, r = rsqrt(sum x^2 + eps).  x, dy, out [n_rows, d] in dtype,
+ * 16-byte aligned, computed in fp32; d as vgdr_norm_gate's dv. */
+int vgdr_l2norm(int dtype, const void *x, const void *dy, void *out, int64_t n_rows, int64_t d, float eps,
+                hipStream_t stream);
+
 /* The pre-norm blocks' RMSNorm (infra/components/norm_layer.py:15-23) over rows
  * rows of dim elements, with the residual add in front of it that the blocks
  * make before each norm (infra/components/block.py:57-59, :85-87):

@@ -97,3 +97,21 @@ def test_norm_gate_second_derivative():
     got = second(ops.norm_gate, o.clone(), gate.clone(), gamma.clone(), dy)
     want = second(ops.norm_gate_expression, *(t.cpu().double() for t in (o, gate, gamma, dy)))
     _check(('ddo', 'ddgate', 'ddgamma'), got, want, torch.float32)
+
+
+# one row, a partly filled last workgroup, the shortest and the longest row, a row length
+# the kernel does not take (torch's own expression), a strided view
+@pytest.mark.gpu
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('rows,d', [(1, 64), (37, 8), (1001, 128), (513, -64), (65, 100)])
+@pytest.mark.parametrize('view', [False, True])
+def test_l2norm_gradients(dtype, rows, d, view):
+    from vagus_amd import ops
+    d = d if d > 0 else -d * (4 if dtype == torch.float32 else 8)
+    print(f'\n[case] l2norm {dtype} rows={rows} d={d} view={view}', flush=True)
+    g = torch.Generator().manual_seed(rows + d)
+    x, dy = (torch.randn(rows, 2 * d if view else d, generator=g).to(dtype).cuda()[:, :d] for _ in range(2))
+    got = _grads(lambda x: ops.l2norm_rows(x, 1e-6), (x,), dy)
+    want = _grads(lambda x: ops.l2norm_expression(x, 1e-6), (x.cpu().double(),), dy.cpu())
+    _check(('y', 'dx'), got, want, dtype)
+    assert torch.equal(ops.l2norm_rows(x.detach()), got[0])

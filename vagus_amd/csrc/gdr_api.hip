@@ -928,6 +928,20 @@ int vgdr_norm_gate_bwd(int dtype, const void *o, const void *gate, const void *g
     return hip_status(vgdr::norm_gate_bwd(dtype, p, stream), "vgdr_norm_gate_bwd launch");
 }
 
+int vgdr_l2norm(int dtype, const void *x, const void *dy, void *out, int64_t n_rows, int64_t d, float eps,
+                hipStream_t stream) {
+    g_err[0] = 0;
+    int rc = check_norm_gate_rows("vgdr_l2norm", dtype, n_rows, d);
+    if (rc) return rc;
+    if (!(eps >= 0.f)) return fail(VGDR_ERR_INVALID, "vgdr_l2norm: eps must be >= 0");
+    if (n_rows == 0) return VGDR_OK;
+    if (!x || !out) return fail(VGDR_ERR_INVALID, "vgdr_l2norm: x and out are required");
+    if (!aligned16(x) || !aligned16(dy) || !aligned16(out))
+        return fail(VGDR_ERR_INVALID, "vgdr_l2norm: every tensor must be 16-byte aligned");
+    if (out == x || out == dy) return fail(VGDR_ERR_INVALID, "vgdr_l2norm: out must not alias an input");
+    return hip_status(vgdr::l2norm(dtype, x, dy, out, eps, n_rows, (int)d, stream), "vgdr_l2norm launch");
+}
+
 int vgdr_rms_norm(int dtype, const void *x, const void *residual, void *x_out, const void *gamma, void *y,
                   int64_t rows, int64_t dim, float eps, hipStream_t stream) {
     g_err[0] = 0;

@@ -222,6 +222,66 @@ hipError_t norm_gate_bwd(int dtype, const NormGateBwd &p, hipStream_t stream) {
     return norm_gate_bwd_t<float>(dtype, p, stream);
 }
 
+// y = x rsqrt(sum x^2 + eps) over rows of LPR 16-byte units (the q, k producer,
+// linear_attention.py:703-706), and its gradient dx = r (dy - y <y, dy>) with r formed
+// again from x: one pass each, bound by HBM, the epilogue's lane layout.
+template <typename E, int LPR, bool BWD>
+__global__ void __launch_bounds__(256) l2norm_kernel(const E *__restrict__ x, const E *__restrict__ dy,
+                                                     E *__restrict__ out, float eps, int64_t n_rows) {
+    constexpr int VE = 16 / (int)sizeof(E), D = LPR * VE;
+    typedef E V __attribute__((ext_vector_type(VE)));
+    const int64_t gt = (int64_t)blockIdx.x * 256 + threadIdx.x, row = gt / LPR;
+    const bool live = row < n_rows;
+    const int64_t off = (live ? row : n_rows - 1) * D + gt % LPR * VE;       // groups past the end re-read the last row
+    const V xv = *reinterpret_cast<const V *>(x + off);
+    V dv{};
+    if constexpr (BWD) dv = __builtin_nontemporal_load(reinterpret_cast<const V *>(dy + off));
+    float ss = 0.f, xd = 0.f;
+#pragma unroll
+    for (int e = 0; e < VE; ++e) {
+        ss += (float)xv[e] * (float)xv[e];
+        if constexpr (BWD) xd += (float)xv[e] * (float)dv[e];
+    }
+#pragma unroll
+    for (int k = 1; k < LPR; k <<= 1) {
+        ss += __shfl_xor(ss, k);
+        if constexpr (BWD) xd += __shfl_xor(xd, k);
+    }
+    const float r = rsqrtf(ss + eps);
+    V o;
+#pragma unroll
+    for (int e = 0; e < VE; ++e)
+        o[e] = BWD ? (E)(r * ((float)dv[e] - r * r * xd * (float)xv[e])) : (E)((float)xv[e] * r);
+    if (live) *reinterpret_cast<V *>(out + off) = o;
+}
+
+template <typename E>
+static hipError_t l2norm_t(const void *x, const void *dy, void *out, float eps, int64_t n_rows, int d,
+                           hipStream_t stream) {
+    const int lpr = d / (16 / (int)sizeof(E));
+    const dim3 grid((unsigned)((n_rows * lpr + 255) / 256));
+    const E *xp = reinterpret_cast<const E *>(x), *dp = reinterpret_cast<const E *>(dy);
+    E *op = reinterpret_cast<E *>(out);
+#define VGDR_L2(L)                                                                                                \
+    case L:                                                                                                       \
+        if (dy) hipLaunchKernelGGL((l2norm_kernel<E, L, true>), grid, dim3(256), 0, stream, xp, dp, op, eps, n_rows); \
+        else hipLaunchKernelGGL((l2norm_kernel<E, L, false>), grid, dim3(256), 0, stream, xp, dp, op, eps, n_rows);   \
+        break;
+    switch (lpr) {
+        VGDR_L2(1) VGDR_L2(2) VGDR_L2(4) VGDR_L2(8) VGDR_L2(16) VGDR_L2(32) VGDR_L2(64)
+        default: return hipErrorInvalidValue;
+    }
+#undef VGDR_L2
+    return hipGetLastError();
+}
+
+hipError_t l2norm(int dtype, const void *x, const void *dy, void *out, float eps, int64_t n_rows, int d,
+                  hipStream_t stream) {
+    if (dtype == 1) return l2norm_t<__bf16>(x, dy, out, eps, n_rows, d, stream);
+    if (dtype == 2) return l2norm_t<_Float16>(x, dy, out, eps, n_rows, d, stream);
+    return l2norm_t<float>(x, dy, out, eps, n_rows, d, stream);
+}
+
 // The pre-norm blocks' RMSNorm (norm_layer.py:15-23) with the residual add in
 // front of it (block.py:57-59, :85-87): h = x + res rounded to E (the stream's
 // new value, stored to x_out), then y = E(E(h * rsqrt(mean(h^2) + eps)) * gamma),

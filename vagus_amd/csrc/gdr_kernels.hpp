@@ -258,6 +258,11 @@ struct NormGateBwd {
 int norm_gate_bwd_blocks(int dtype, int64_t n_rows, int dv);
 hipError_t norm_gate_bwd(int dtype, const NormGateBwd &p, hipStream_t stream);
 
+// Rows of d elements to unit length, out = x rsqrt(sum x^2 + eps), or with dy the
+// gradient of that; d as norm_gate's dv, n_rows > 0.
+hipError_t l2norm(int dtype, const void *x, const void *dy, void *out, float eps, int64_t n_rows, int d,
+                  hipStream_t stream);
+
 // The blocks' RMSNorm with an optional residual add first (res, x_out may be
 // null): x_out = x + res, y = RMSNorm(x + res) * gamma over rows of dim
 // elements.  dim / (16 / sizeof(E)) <= 2048.

@@ -308,8 +308,7 @@ class GatedDeltaNet(nn.Module):
 
     @staticmethod
     def _l2norm(x, eps: float = 1e-6):
-        h = x.to(torch.promote_types(x.dtype, torch.float32))
-        return (h * torch.rsqrt(h.pow(2).sum(-1, keepdim=True) + eps)).to(x.dtype)
+        return ops.l2norm_rows(x, eps)
 
     def _heads(self, qp, kp, vp, *, l2norm: bool = True, cu_seqlens=None):
         """conv -> SiLU -> per-head view, and (unless the kernel will do it)

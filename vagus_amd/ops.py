@@ -166,32 +166,69 @@ def _gate_activation_rows(f, fz):
     return -a * F.softplus(x)
 
 
+def _row_lanes(t):
+    """Whether the row kernels take rows of t's last dim: 16-byte units, a power of two of them up to 64."""
+    n, r = divmod(t.shape[-1] * t.element_size(), 16)
+    return r == 0 and 1 <= n <= 64 and n & (n - 1) == 0
+
+
+def l2norm_expression(x, eps):
+    """x rsqrt(sum x^2 + eps) over the last dim in >= fp32, cast back (linear_attention.py:703-706)."""
+    h = x.to(torch.promote_types(x.dtype, torch.float32))
+    return (h * torch.rsqrt(h.pow(2).sum(-1, keepdim=True) + eps)).to(x.dtype)
+
+
+def _l2norm_kernel(x, dy, eps):
+    """vgdr_l2norm over the rows of x (dy None), or its gradient for dy."""
+    xa, dya = _aligned(x), _aligned(dy)
+    out = torch.empty_like(xa)
+    d = x.shape[-1]
+    with torch.cuda.device(x.device):
+        _lib.check(_lib.load().vgdr_l2norm(_DTYPES[x.dtype], _ptr(xa), _ptr(dya), _ptr(out), x.numel() // d, d, eps,
+                                           _stream(x.device)))
+    return out
+
+
 class _L2NormRows(torch.autograd.Function):
-    """y = x r, r = rsqrt(sum x^2 + 1e-6) per (token, head), computed in >= fp32
-    and rounded to x's type (linear_attention.py:703-706).  Saves x (its own
-    type) and r (one float per row): autograd through the torch expression
+    """y = x r, r = rsqrt(sum x^2 + eps) per (token, head), computed in >= fp32
+    and rounded to x's type (linear_attention.py:703-706).  Saves x alone (in its
+    own type); r is formed again: autograd through the torch expression
     would keep fp32 copies of the whole (B, T, H, dk) row block.
-    dx = r dy - r^3 x <x, dy>."""
+    dx = r dy - r^3 x <x, dy>.  One kernel each way where the row kernels take
+    the rows, torch elsewhere and for a backward that is itself differentiated."""
 
     @staticmethod
-    def forward(ctx, x):
-        xf = x if x.dtype == torch.float64 else x.float()
-        r = torch.rsqrt((xf * xf).sum(-1, keepdim=True) + 1e-6)
-        ctx.save_for_backward(x, r)
-        return (xf * r).to(x.dtype)
+    def forward(ctx, x, eps):
+        ctx.save_for_backward(x)
+        ctx.eps = eps
+        ctx.kernel = _kernel_autograd(x) and _row_lanes(x)
+        return _l2norm_kernel(x, None, eps) if ctx.kernel else l2norm_expression(x, eps)
 
     @staticmethod
     def backward(ctx, dy):
-        x, r = ctx.saved_tensors
-        xf = x.to(r.dtype)
-        dyf = dy.to(r.dtype)
-        return (r * dyf - r * r * r * xf * (xf * dyf).sum(-1, keepdim=True)).to(x.dtype)
+        x, = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return torch.autograd.grad(l2norm_expression(x, ctx.eps), x, dy, create_graph=True)[0], None
+        if ctx.kernel:
+            return _l2norm_kernel(x, dy, ctx.eps), None
+        xf = x.to(torch.promote_types(x.dtype, torch.float32))
+        dyf = dy.to(xf.dtype)
+        r = torch.rsqrt((xf * xf).sum(-1, keepdim=True) + ctx.eps)
+        return (r * dyf - r * r * r * xf * (xf * dyf).sum(-1, keepdim=True)).to(x.dtype), None
 
 
 def _l2norm_rows(x):
     """x rsqrt(sum x^2 + 1e-6) per (token, head) in >= fp32, cast back
     (linear_attention.py:703-706): the q, k producer, differentiable."""
-    return _L2NormRows.apply(x)
+    return _L2NormRows.apply(x, 1e-6)
+
+
+def l2norm_rows(x, eps: float = 1e-6):
+    """The q, k producer for a layer: one kernel each way where the kernels
+    take the tensor, the module's torch expression elsewhere."""
+    if not (_kernel_autograd(x) and _row_lanes(x) and eps >= 0):
+        return l2norm_expression(x, eps)
+    return _L2NormRows.apply(x, eps) if _wants_grad(x) else _l2norm_kernel(x, None, eps)
 
 
 class _Fusion:
@@ -802,12 +839,6 @@ def norm_gate_expression(o, gate, gamma, eps):
     h = o.to(torch.promote_types(o.dtype, torch.float32))
     h = h * torch.rsqrt(h.pow(2).mean(dim=-1, keepdim=True) + eps)
     return h.to(o.dtype) * gamma * F.silu(gate)
-
-
-def _row_lanes(t):
-    """Whether the row kernels take rows of t's last dim: 16-byte units, a power of two of them up to 64."""
-    n, r = divmod(t.shape[-1] * t.element_size(), 16)
-    return r == 0 and 1 <= n <= 64 and n & (n - 1) == 0
 
 
 class _NormGateRule(torch.autograd.Function):
