@@ -1803,18 +1803,29 @@ __global__ void __launch_bounds__(512) chunk_grad_vec_kernel(const ChunkBwdParam
     }
 }
 
-// dA_log and dt_bias of the fused gate activation: the per-chunk sums
-// chunk_grad_vec_kernel left, added over the chunks in slot order (one
-// workgroup per head, a thread per dt_bias channel and one for A_log), so the
-// result does not depend on scheduling
+// dA_log and ddt_bias: the sums of the per-chunk partials over the chunk slots, in a
+// fixed order, so the result does not depend on scheduling.  A workgroup adds 16
+// columns of one head ([ddt_bias | dA_log]); its 64 thread groups take every 64th slot
+// and meet in LDS.  Bound by latency: one thread per column over all slots was a chain
+// of 512 dependent adds behind their loads at 512 chunks (160 us; the 4 heads' rows are 1 MB).
+constexpr int GPG_COLS = 16, GPG_ROWS = 64;
 template <int DK>
-__global__ void __launch_bounds__(256) gate_param_grad_kernel(const ChunkBwdParams p) {
-    const int h = blockIdx.x, c = threadIdx.x;
-    if (c > DK) return;
+__global__ void __launch_bounds__(GPG_COLS * GPG_ROWS) gate_param_grad_kernel(const ChunkBwdParams p) {
+    __shared__ float red[GPG_ROWS][GPG_COLS + 1];
+    const int h = blockIdx.x, cc = threadIdx.x % GPG_COLS, w = threadIdx.x / GPG_COLS;
+    const int c = blockIdx.y * GPG_COLS + cc;
     int64_t n = p.geo.cu ? (int64_t)p.geo.chunk_offs[p.geo.n_seqs] : (int64_t)p.n_chunk_slots;
     n = n < p.n_chunk_slots ? n : p.n_chunk_slots;
     float acc = 0.f;
-    for (int64_t s = 0; s < n; ++s) acc += p.dpart[(s * p.H + h) * (DK + 1) + c];
+    if (c <= DK) {
+#pragma unroll 4
+        for (int64_t s = w; s < n; s += GPG_ROWS) acc += p.dpart[(s * p.H + h) * (DK + 1) + c];
+    }
+    red[w][cc] = acc;
+    __syncthreads();
+    if (w > 0 || c > DK) return;
+#pragma unroll
+    for (int k = 1; k < GPG_ROWS; ++k) acc += red[k][cc];
     if (c < DK) p.ddt_bias[(int64_t)h * DK + c] = acc;
     else p.dA_log[h] = acc;
 }
@@ -1882,7 +1893,8 @@ static hipError_t run_bwd_vec(ChunkBwdParams p, hipStream_t stream) {
             hipLaunchKernelGGL((chunk_grad_vec_kernel<DK, CH, E>), dim3((unsigned)grad_blocks), dim3(512), 0, stream,
                                p);
         if (p.fz.gate_act)
-            hipLaunchKernelGGL((gate_param_grad_kernel<DK>), dim3((unsigned)p.H), dim3(256), 0, stream, p);
+            hipLaunchKernelGGL((gate_param_grad_kernel<DK>), dim3((unsigned)p.H, (DK + GPG_COLS) / GPG_COLS),
+                               dim3(GPG_COLS * GPG_ROWS), 0, stream, p);
     }
     return hipGetLastError();
 }
