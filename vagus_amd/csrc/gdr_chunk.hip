@@ -554,6 +554,17 @@ chunk_prep_kernel(const ChunkParams p) {
             return s <= wave;
         } else {
             const int job = wave + NW * s;
+            if (GATE == 2 && !fast) {
+                // the diagonal tiles first, one per wave: their exact form is the longest
+                // job (the products on gated operands run 7% slower in this order)
+                I = J = job;
+                if (job >= NB) {
+                    I = 1;
+                    J = job - NB;
+                    while (J >= I) { J -= I; ++I; }
+                }
+                return job < NL;
+            }
             I = 0;
             J = job;
             while (J > I) { J -= I + 1; ++I; }
@@ -688,55 +699,113 @@ chunk_prep_kernel(const ChunkParams p) {
                 if (irow >= clen) bq[kt] = EL::cvt(f32x4{0.f, 0.f, 0.f, 0.f});
             }
         }
-        bool pairwise = false;
-        if constexpr (GATE == 2) {
-            pairwise = (I == J) && flag[I];
-            const int rr = 16 * I;
-#pragma unroll
-            for (int kt = 0; kt < NKB; ++kt) {
-                const int cc = 16 * kt + 4 * g4;
-                const f32x4 gr = ld4(gam + rr * PG + cc);
-                const f32x4 ea = exp4(gr - ld4(gam + jrow * PG + cc));      // <= 1 off the diagonal
-                const f32x4 eb = exp4(ld4(gam + irow * PG + cc) - gr);      // <= 1
-                a[kt] = EL::cvt(EL::tof(a[kt]) * ea);
-                bq[kt] = EL::cvt(EL::tof(bq[kt]) * eb);
-                bk[kt] = EL::cvt(EL::tof(bk[kt]) * eb);
-            }
-        }
         f32x4 accq = {0.f, 0.f, 0.f, 0.f}, acck = {0.f, 0.f, 0.f, 0.f};
+        bool pairwise = false;
+        if constexpr (GATE == 2) pairwise = (I == J) && __builtin_amdgcn_readfirstlane(flag[I]) != 0;
         if (!pairwise) {
+            if constexpr (GATE == 2) {
+                const int rr = 16 * I;
+#pragma unroll
+                for (int kt = 0; kt < NKB; ++kt) {
+                    const int cc = 16 * kt + 4 * g4;
+                    const f32x4 gr = ld4(gam + rr * PG + cc);
+                    const f32x4 ea = exp4(gr - ld4(gam + jrow * PG + cc));      // <= 1 off the diagonal
+                    const f32x4 eb = exp4(ld4(gam + irow * PG + cc) - gr);      // <= 1
+                    a[kt] = EL::cvt(EL::tof(a[kt]) * ea);
+                    bq[kt] = EL::cvt(EL::tof(bq[kt]) * eb);
+                    bk[kt] = EL::cvt(EL::tof(bk[kt]) * eb);
+                }
+            }
 #pragma unroll
             for (int kt = 0; kt < NKB; kt += 2) {
                 accq = mfma_kb2(a[kt], bq[kt], a[kt + 1], bq[kt + 1], accq);
                 acck = mfma_kb2(a[kt], bk[kt], a[kt + 1], bk[kt + 1], acck);
             }
+            // the products' last results pass their wait states before the paths join
+            if constexpr (GATE == 2) asm volatile("s_nop 7\n\ts_nop 7" : "+v"(accq), "+v"(acck));
         } else if constexpr (GATE == 2) {
-            // exact pairwise products for a diagonal block with a large decay range
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-                const int jt = 16 * J + 4 * g4 + jj;
-                float sq = 0.f, sk = 0.f;
-                if (jt <= irow) {
-#pragma unroll 1
-                    for (int cc = 0; cc < DK; cc += 4) {
-                        const f32x4 e = exp4(ld4(gam + irow * PG + cc) - ld4(gam + jt * PG + cc));
-                        const f32x4 kj = EL::tof(ld_frag<E>(Wst + SK::at(jt, cc))) * e;
-                        f32x4 qv;
-                        if constexpr (L::QREG) {                 // as bq above, before the gate
-                            F qf = *reinterpret_cast<const F *>(qsrc + cc);
-                            if (sizeof(E) == 2 && fz.qk_l2norm) qf = EL::cvt(EL::tof(qf) * rqf[irow]);
-                            qv = irow < clen ? EL::tof(qf) : f32x4{0.f, 0.f, 0.f, 0.f};
-                        } else {
-                            qv = EL::tof(ld_frag<E>(Qst + SK::at(irow, cc)));
-                        }
-                        const f32x4 yq = qv * kj;
-                        const f32x4 yk = EL::tof(ld_frag<E>(Kst + SK::at(irow, cc))) * kj;
-                        sq += yq[0] + yq[1] + yq[2] + yq[3];
-                        sk += yk[0] + yk[1] + yk[2] + yk[3];
+            // A diagonal tile whose decay range is too large for one reference row, in
+            // fp32 throughout: the rows in four groups of four.  Row i against the
+            // columns j before its group: reference r = the group's first row, both
+            // factors e^(g_i - g_r), e^(g_r - g_j) <= 1, as fp32 MFMA products (one
+            // per group, of which the group's four rows are kept).  Row i against its
+            // own group: the pairs (i, i - d), d = 0..3, one exponential per channel;
+            // lane (r16, g4) sums its 32 channels of row i and the four g4 lanes add up.
+            // Bound by the exponentials (12 per channel and row with those of the
+            // products, against 8.5 of a loop over every pair, whose lanes read one
+            // pair each from LDS and Q from global memory, 4 channels at a time, with
+            // nothing in flight).  KDA scan of 4 x 8192 tokens, 8 heads, dk = dv = 128, most
+            // chunks flagged: bf16 480 -> 449 us, fp16 921 -> 574 us; 1000 tokens, 4 heads:
+            // prep 48 -> 27 to 38 us.  (The tiles below the diagonal on gated operands too,
+            // as in the fast form, spilled registers: 472 us, and 332 against 305 us
+            // for a call with no flagged block.)
+            const int sub = r16 >> 2, r0 = 16 * I + 4 * sub;
+            // (without it the compiler converts the fragments and reads the decay rows once
+            // ahead of the loops and keeps them: 1,248 bytes of spills per lane)
+            auto opaque_frags = [&](int &c4) __attribute__((always_inline)) {
+                asm volatile("" : "+v"(c4));
+                unroll<NKB>([&](auto kt) __attribute__((always_inline)) {
+                    if constexpr (sizeof(E) == 2) {
+                        u32x2 x = __builtin_bit_cast(u32x2, a[kt]), y = __builtin_bit_cast(u32x2, bq[kt]),
+                              z = __builtin_bit_cast(u32x2, bk[kt]);
+                        asm volatile("" : "+v"(x), "+v"(y), "+v"(z));
+                        a[kt] = __builtin_bit_cast(F, x);
+                        bq[kt] = __builtin_bit_cast(F, y);
+                        bk[kt] = __builtin_bit_cast(F, z);
                     }
+                });
+            };
+#pragma unroll 1
+            for (int si = 1; si < 4; ++si) {
+                f32x4 cq = {0.f, 0.f, 0.f, 0.f}, ck = {0.f, 0.f, 0.f, 0.f};
+                const bool before = r16 < 4 * si;
+                int c4 = 4 * g4;
+                opaque_frags(c4);
+#pragma unroll
+                for (int kt = 0; kt < NKB; ++kt) {
+                    if (kt % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                    const int cc = 16 * kt + c4;
+                    const f32x4 gr = ld4(gam + (16 * I + 4 * si) * PG + cc), gi = ld4(gam + irow * PG + cc);
+                    const f32x4 ea = exp4(gr - gi);                             // row jrow = irow is the j side here
+                    const f32x4 eb = exp4(gi - ld4(gam + r0 * PG + cc));
+                    f32x4 af = EL::tof(a[kt]) * ea;
+                    if (!before) af = f32x4{0.f, 0.f, 0.f, 0.f};
+                    cq = mfma_kb1(af, EL::tof(bq[kt]) * eb, cq);
+                    ck = mfma_kb1(af, EL::tof(bk[kt]) * eb, ck);
                 }
-                accq[jj] = sq;
-                acck[jj] = sk;
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) {
+                    accq[jj] = sub == si && g4 < si ? cq[jj] : accq[jj];
+                    acck[jj] = sub == si && g4 < si ? ck[jj] : acck[jj];
+                }
+            }
+#pragma unroll 1
+            for (int d = 0; d < 4; ++d) {
+                const int jt = irow - d < r0 ? r0 : irow - d;
+                float sq = 0.f, sk = 0.f;
+                int c4 = 4 * g4;
+                opaque_frags(c4);
+#pragma unroll
+                for (int kt = 0; kt < NKB; ++kt) {
+                    if (kt % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                    const int cc = 16 * kt + c4;
+                    const f32x4 kj = EL::tof(ld_frag<E>(Wst + SK::at(jt, cc))) *
+                                     exp4(ld4(gam + irow * PG + cc) - ld4(gam + jt * PG + cc));
+                    const f32x4 yq = EL::tof(bq[kt]) * kj, yk = EL::tof(bk[kt]) * kj;
+                    sq += yq[0] + yq[1] + yq[2] + yq[3];
+                    sk += yk[0] + yk[1] + yk[2] + yk[3];
+                }
+                sq += __shfl_xor(sq, 16);
+                sk += __shfl_xor(sk, 16);
+                sq += __shfl_xor(sq, 32);
+                sk += __shfl_xor(sk, 32);
+                // (i, i - d) is entry jj = (i mod 4) - d of the lane whose columns are i's group
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) {
+                    const bool mine = g4 == sub && jj == (r16 & 3) - d;
+                    accq[jj] = mine ? sq : accq[jj];
+                    acck[jj] = mine ? sk : acck[jj];
+                }
             }
         }
         job_tail(s, I, J, irow, accq, acck);
