@@ -432,60 +432,72 @@ class GatedDeltaNet(nn.Module):
 
     def _decode_weights(self):
         """The one-token decode step's projection weights regrouped, rebuilt
-        whenever a parameter changed (its storage or version): W_q, W_k, W_v
-        and W_g concatenated into one (4 H*dv, dim) weight, so that one GEMM
-        replaces four skinny ones (when H*dk == H*dv); for the
+        whenever a parameter changed (its storage or version): every matrix
+        that multiplies the input (W_q, W_k, W_v, W_g, and without the scalar
+        gate W_a1 and W_b) stacked into one weight, rows padded with zeros to a
+        multiple of 64 (so that the rows of its product stay 16-byte aligned),
+        so that one GEMM replaces up to six skinny ones; for the
         scalar gate [W_a; W_b] as one (2H, dim) weight (W_a alone without the
-        delta rule) and the gate's constants -exp(A_log) and dt_bias in fp32.
-        The copies hold one more set of these weights (4 dim H dv + 2 H dim
-        elements per layer)."""
-        ps = [self.wq.weight, self.wk.weight, self.wv.weight, self.wg.weight]
+        delta rule), which the decode kernel multiplies itself; and the gate's
+        constants in fp32: -exp(A_log) (scalar) or A_log (per channel), and dt_bias.
+        The copies hold one more set of these weights."""
         scalar = self.gate == 'scalar'
+        stacked = [self.wq, self.wk, self.wv, self.wg]
+        if self.gate == 'vector':
+            stacked.append(self.wa1)
+        if self.delta and not scalar:
+            stacked.append(self.wb)
+        ps = [m.weight for m in stacked]
+        n = len(ps)
         if scalar:
-            ps += [self.wa.weight, self.A_log, self.dt_bias]
-        if self.delta:
-            ps.append(self.wb.weight)
+            ps += [self.wa.weight] + ([self.wb.weight] if self.delta else [])
+        if self.gate != 'none':
+            ps += [self.A_log, self.dt_bias]
         key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in ps)
         c = self.__dict__.get('_decode_w')
         if c is None or c[0] != key:
-            same = len({p.shape for p in ps[:4]}) == 1
-            w4 = torch.cat(ps[:4]).contiguous() if same else None
-            wab = gconst = None
-            if scalar:
-                wab = torch.cat([self.wa.weight] + ([self.wb.weight] if self.delta else [])).contiguous()
-                gconst = (-self.A_log.float().exp(), self.dt_bias.float())
-            c = (key, w4, wab, gconst)
+            w = torch.cat(ps[:n])
+            w = F.pad(w, (0, 0, 0, -w.shape[0] % 64)).contiguous()
+            wab = torch.cat(ps[n:-2]).contiguous() if scalar else None
+            gconst = None
+            if self.gate != 'none':
+                gconst = (-self.A_log.float().exp() if scalar else self.A_log.float(), self.dt_bias.float())
+            c = (key, w, wab, gconst)
             self.__dict__['_decode_w'] = c
         return c[1:]
 
     def _decode_inputs(self, x):
-        """(qp, kp, vp, out_gate, g, beta, gate_proj) for the one-token decode
-        kernel: the projections of x (B, 1, dim), the log-decay in fp32 (or the
-        KDA gate's pre-activation) and the beta logits, with the regrouped
-        weights of _decode_weights.  With the scalar gate, g and beta are None
-        and gate_proj = (x, [W_a; W_b], -exp(A_log), dt_bias): the decode
-        kernel forms them itself.  The values are those of the separate
-        projections and of _gates(raw_gate=vector, raw_beta=delta) up to the
-        GEMMs' summation order."""
-        B, L = x.shape[0], x.shape[1]
-        w4, wab, gconst = self._decode_weights()
-        if w4 is not None:
-            # one GEMM over the concatenated weights; for one token the decode
-            # kernel reads the four column blocks of its rows in place, otherwise
-            # one copy makes them four contiguous (B*L, H*dv) blocks
-            y = F.linear(x.reshape(B * L, -1), w4)
-            n = y.shape[-1] // 4
-            if L == 1:
-                qp, kp, vp, og = (y[:, i * n:(i + 1) * n].view(B, L, n) for i in range(4))
-            else:
-                y = y.view(B * L, 4, -1).transpose(0, 1).contiguous()
-                qp, kp, vp, og = (y[i].view(B, L, -1) for i in range(4))
-        else:
-            qp, kp, vp, og = self.wq(x), self.wk(x), self.wv(x), self.wg(x)
-        if wab is None:
+        """(qp, kp, vp, out_gate, g, beta, gate_proj, gate constants) for the
+        one-token decode kernel: the projections of x (B, 1, dim), the KDA gate's
+        pre-activation and the beta logits, from one GEMM over the stacked
+        weight of _decode_weights (W_a2 follows as its own); the kernel reads
+        q, k, v and the output gate in place, as column blocks of the product's rows.
+        With the scalar gate, g and beta are None and gate_proj = (x, [W_a; W_b],
+        -exp(A_log), dt_bias): the decode kernel forms them itself.  The values
+        are those of the separate projections and of _gates(raw_gate=vector,
+        raw_beta=delta) up to the GEMMs' summation order.  A layer whose
+        projections are not plain nn.Linear modules, or whose _gates is
+        overridden, calls them."""
+        B = x.shape[0]
+        H, dk, dv = self.head_count, self.key_head_dim, self.value_head_dim
+        names = ('wq', 'wk', 'wv', 'wg') + {'scalar': (), 'vector': ('wa1',), 'none': ()}[self.gate]
+        if self.delta and self.gate != 'scalar':
+            names += ('wb',)
+        mods = [getattr(self, n) for n in names]
+        if (not all(_plain_module(m, nn.Linear) and m.bias is None and m.weight.dtype == x.dtype for m in mods)
+                or type(self)._gates is not GatedDeltaNet._gates):
             g, beta = self._gates(x, raw_gate=self.gate == 'vector', raw_beta=self.delta)
-            return qp, kp, vp, og, g, beta, None
-        return qp, kp, vp, og, None, None, (x, wab, *gconst)
+            return (self.wq(x), self.wk(x), self.wv(x), self.wg(x), g,
+                    beta if self.delta else None, None, (self.A_log, self.dt_bias) if self.gate == 'vector' else None)
+        w, wab, gconst = self._decode_weights()
+        y = F.linear(x.reshape(B, -1), w)
+        widths = [H * dk, H * dk, H * dv, H * dv] + [m.weight.shape[0] for m in mods[4:]]
+        cols = y[:, :sum(widths)].split(widths, -1)
+        qp, kp, vp, og = (c.unsqueeze(1) for c in cols[:4])
+        if self.gate == 'scalar':
+            return qp, kp, vp, og, None, None, (x, wab, *gconst), None
+        g = self.wa2(cols[4]).view(B, 1, H, dk) if self.gate == 'vector' else None
+        return qp, kp, vp, og, g, cols[-1].unsqueeze(1) if self.delta else None, None, gconst
 
     @torch.no_grad()
     def decode_step(self, x):
@@ -502,12 +514,12 @@ class GatedDeltaNet(nn.Module):
         H, dk, dv = self.head_count, self.key_head_dim, self.value_head_dim
         if L == 1 and type(self)._write is GatedDeltaNet._write and self._decode_kernel_fits():
             vec = self.gate == 'vector'
-            qp, kp, vp, og, g, beta, gp = self._decode_inputs(x)
+            qp, kp, vp, og, g, beta, gp, gc = self._decode_inputs(x)
             o = ops.hip_decode_step(qp, kp, vp, g, beta, self.state, scale=self.scale, delta=self.delta,
                                     gate_proj=gp,
                                     conv_weights=self._conv_weights(), conv_cache=self._caches(), l2norm=True,
                                     beta_logits=self.delta, gate_in_kernel=vec,
-                                    A_log=self.A_log if vec else None, dt_bias=self.dt_bias if vec else None,
+                                    A_log=gc[0] if vec else None, dt_bias=gc[1] if vec else None,
                                     lower_bound=self.gate_lower_bound, out_gate=og,
                                     out_norm_weight=self.o_norm.gamma, out_norm_eps=self.o_norm.eps)
             self.cache_len += L
