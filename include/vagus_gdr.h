@@ -557,6 +557,18 @@ int vgdr_norm_gate_bwd(int dtype, const void *o, const void *gate, const void *g
 int vgdr_l2norm(int dtype, const void *x, const void *dy, void *out, int64_t n_rows, int64_t d, float eps,
                 hipStream_t stream);
 
+/* Weight gradients of n_mats (at most 8) projections y_i = x W_i^T that share
+ * their input: dw[i] [n[i], dim] = dy[i]^T x, summed over the T rows in fp32, in a
+ * fixed order, and rounded once.  x [T, dim] with rows ldx elements apart, dy[i]
+ * [T, n[i]] with rows ld[i] apart; bf16 or fp16; dim, n, ld, ldx multiples of 8,
+ * pointers 16-byte aligned.  The arrays are host arrays.  What the reference's
+ * autograd takes through its nn.Linear projections (linear_attention.py:600-625).
+ * workspace: vgdr_linear_wgrad_workspace_size bytes (0: none needed). */
+int64_t vgdr_linear_wgrad_workspace_size(int dtype, int n_mats, const int64_t *n, int64_t T, int64_t dim);
+int vgdr_linear_wgrad(int dtype, int n_mats, const void *const *dy, const int64_t *ld, const int64_t *n,
+                      const void *x, int64_t ldx, void *const *dw, void *workspace,
+                      int64_t workspace_bytes, int64_t T, int64_t dim, hipStream_t stream);
+
 /* The pre-norm blocks' RMSNorm (infra/components/norm_layer.py:15-23) over rows
  * rows of dim elements, with the residual add in front of it that the blocks
  * make before each norm (infra/components/block.py:57-59, :85-87):

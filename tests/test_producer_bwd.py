@@ -115,3 +115,47 @@ def test_l2norm_gradients(dtype, rows, d, view):
     want = _grads(lambda x: ops.l2norm_expression(x, 1e-6), (x.cpu().double(),), dy.cpu())
     _check(('y', 'dx'), got, want, dtype)
     assert torch.equal(ops.l2norm_rows(x.detach()), got[0])
+
+
+# tiles of 256 x 128 with rows and columns left over, several matrices of one input (widths that
+# are no multiple of 8 or 16 among them), token counts below one step, with a partial last step,
+# with one split and with many
+@pytest.mark.gpu
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('T,dim,widths', [(1, 8, [8]), (31, 40, [4, 264]), (127, 136, [256]), (1003, 1024, [512, 64, 3]),
+                                          (3003, 64, [512]), (8200, 520, [300, 16, 1032]), (70000, 64, [24])])
+@pytest.mark.parametrize('view', [False, True])
+def test_linear_weight_gradients(dtype, T, dim, widths, view):
+    """The sum's bound: fp32 accumulation, one rounding of the result."""
+    from vagus_amd import ops
+    print(f'\n[case] wgrad {dtype} T={T} dim={dim} widths={widths} view={view}', flush=True)
+    g = torch.Generator('cuda').manual_seed(T + dim)
+    # a view: rows of a wider buffer that start on a 16-byte unit
+    mats = [torch.randn(T, d + (16 if view else 0), generator=g, device='cuda').to(dtype)[:, 8 if view else 0:][:, :d]
+            for d in [dim] + widths]
+    got = ops.linear_wgrads(mats[0], mats[1:])
+    for dy, dw in zip(mats[1:], got):
+        ref = dy.double().T.contiguous() @ mats[0].double()
+        err = _rel(dw, ref)
+        print(f'[parity] rel_l2={err:.3e}', flush=True)
+        assert dw.shape == ref.shape and err <= (4e-3 if dtype == torch.bfloat16 else 5e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('frozen', [(), ('x',), (1,), (0, 2)])
+def test_projections_gradients(frozen):
+    from vagus_amd import ops
+    print(f'\n[case] projections frozen={frozen}', flush=True)
+    g = torch.Generator().manual_seed(6)
+    x = torch.randn(2, 65, 128, generator=g).bfloat16().cuda().requires_grad_('x' not in frozen)
+    ws = [(0.1 * torch.randn(n, 128, generator=g)).bfloat16().cuda().requires_grad_(i not in frozen)
+          for i, n in enumerate((256, 64, 4))]
+    dys = [torch.randn(2, 65, n, generator=g).bfloat16().cuda() for n in (256, 64, 4)]
+    leaves = [t for t in [x] + ws if t.requires_grad]
+    got = torch.autograd.grad(ops.projections(x, *ws), leaves, dys)
+    x64, w64 = x.detach().cpu().double(), [w.detach().cpu().double() for w in ws]
+    for t, s in zip([x64] + w64, [x] + ws):
+        t.requires_grad_(s.requires_grad)
+    want = torch.autograd.grad([F.linear(x64, w) for w in w64], [t for t in [x64] + w64 if t.requires_grad],
+                               [d.cpu().double() for d in dys])
+    _check([f'd{i}' for i in range(len(got))], got, want, torch.bfloat16)

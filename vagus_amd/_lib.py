@@ -95,6 +95,9 @@ SIGNATURES = {
     'vgdr_norm_gate_bwd_workspace_size': (_L, [_I, _L, _L]),
     'vgdr_norm_gate_bwd': (_I, [_I, _P, _P, _P, _F, _P, _P, _P, _P, _P, _L, _L, _L, _P]),
     'vgdr_l2norm': (_I, [_I, _P, _P, _P, _L, _L, _F, _P]),
+    'vgdr_linear_wgrad_workspace_size': (_L, [_I, _I, ctypes.POINTER(_L), _L, _L]),
+    'vgdr_linear_wgrad': (_I, [_I, _I, ctypes.POINTER(_P), ctypes.POINTER(_L), ctypes.POINTER(_L), _P, _L,
+                               ctypes.POINTER(_P), _P, _L, _L, _L, _P]),
     'vgdr_rms_norm': (_I, [_I, _P, _P, _P, _P, _P, _L, _L, _F, _P]),
     'vgdr_scalar_gates': (_I, [_I, _P, _P, _P, _P, _P, _P, _L, _L, _L, _P]),
     'vgdr_swiglu': (_I, [_I, _P, _P, _L, _L, _P]),

@@ -942,6 +942,62 @@ int vgdr_l2norm(int dtype, const void *x, const void *dy, void *out, int64_t n_r
     return hip_status(vgdr::l2norm(dtype, x, dy, out, eps, n_rows, (int)d, stream), "vgdr_l2norm launch");
 }
 
+// the plan of one call into p (no pointers); the widths are multiples of 8
+static int plan_wgrad(const char *fn, int dtype, int n_mats, const int64_t *n, int64_t T, int64_t dim,
+                      vgdr::WgradParams &p) {
+    if (dtype != VGDR_BF16 && dtype != VGDR_F16)
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: dtype %d (bf16, fp16)", fn, dtype);
+    if (n_mats < 1 || n_mats > vgdr::WGRAD_MAX || !n)
+        return fail(VGDR_ERR_INVALID, "%s: 1 to %d matrices, got %d", fn, vgdr::WGRAD_MAX, n_mats);
+    if (T < 1 || dim < 8 || dim % 8 || dim > 0x100000)
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: T=%lld dim=%lld (a multiple of 8)", fn, (long long)T, (long long)dim);
+    for (int i = 0; i < n_mats; ++i) {
+        if (n[i] < 8 || n[i] % 8 || n[i] > 0x100000)
+            return fail(VGDR_ERR_UNSUPPORTED, "%s: width %lld (a multiple of 8)", fn, (long long)n[i]);
+        p.g[i].n = (int)n[i];
+    }
+    p.T = T;
+    p.dim = (int)dim;
+    p.n_groups = n_mats;
+    vgdr::wgrad_plan(p);
+    return VGDR_OK;
+}
+
+int64_t vgdr_linear_wgrad_workspace_size(int dtype, int n_mats, const int64_t *n, int64_t T, int64_t dim) {
+    g_err[0] = 0;
+    vgdr::WgradParams p{};
+    if (plan_wgrad("vgdr_linear_wgrad_workspace_size", dtype, n_mats, n, T, dim, p)) return 0;
+    return p.splits > 1 ? 4 * (int64_t)p.splits * p.rows * p.dim : 0;
+}
+
+int vgdr_linear_wgrad(int dtype, int n_mats, const void *const *dy, const int64_t *ld, const int64_t *n, const void *x,
+                      int64_t ldx, void *const *dw, void *workspace, int64_t workspace_bytes, int64_t T, int64_t dim,
+                      hipStream_t stream) {
+    g_err[0] = 0;
+    const char *fn = "vgdr_linear_wgrad";
+    vgdr::WgradParams p{};
+    int rc = plan_wgrad(fn, dtype, n_mats, n, T, dim, p);
+    if (rc) return rc;
+    if (!dy || !ld || !dw || !x || !aligned16(x) || ldx < dim || ldx % 8)
+        return fail(VGDR_ERR_INVALID, "%s: x (rows of a multiple of 8 elements, 16-byte aligned), dy, ld and dw are "
+                    "required", fn);
+    for (int i = 0; i < n_mats; ++i) {
+        if (!dy[i] || !dw[i] || !aligned16(dy[i]) || !aligned16(dw[i]) || ld[i] < n[i] || ld[i] % 8)
+            return fail(VGDR_ERR_INVALID, "%s: matrix %d: rows of a multiple of 8 elements, 16-byte aligned", fn, i);
+        if (dw[i] == dy[i] || dw[i] == x) return fail(VGDR_ERR_INVALID, "%s: dw must not alias an input", fn);
+        p.g[i].dy = dy[i];
+        p.g[i].dw = dw[i];
+        p.g[i].ld = ld[i];
+    }
+    const int64_t need = p.splits > 1 ? 4 * (int64_t)p.splits * p.rows * p.dim : 0;
+    if (need && (!workspace || !aligned16(workspace) || workspace_bytes < need))
+        return fail(VGDR_ERR_INVALID, "%s: workspace too small", fn);
+    p.x = x;
+    p.ldx = ldx;
+    p.part = reinterpret_cast<float *>(workspace);
+    return hip_status(vgdr::wgrad(dtype, p, stream), "vgdr_linear_wgrad launch");
+}
+
 int vgdr_rms_norm(int dtype, const void *x, const void *residual, void *x_out, const void *gamma, void *y,
                   int64_t rows, int64_t dim, float eps, hipStream_t stream) {
     g_err[0] = 0;

@@ -82,6 +82,27 @@ struct ConvBwdParams {
     int K, silu, run;
 };
 
+// Weight gradients of projections that share their input (16-bit elements):
+// dw[n][c] = sum_t dy[t][n] x[t][c], rows of dy and x ld and ldx elements apart, n and
+// dim multiples of 8.  part: splits x rows x dim floats when splits > 1.  row0, tile0
+// and everything from rows on: wgrad_plan.
+constexpr int WGRAD_MAX = 8;
+struct WgradGroup {
+    const void *dy;
+    void *dw;
+    int64_t ld;
+    int n, row0, tile0;
+};
+struct WgradParams {
+    const void *x;
+    float *part;
+    int64_t T, ldx;
+    int dim, n_groups;
+    WgradGroup g[WGRAD_MAX];
+    int64_t split_len;
+    int rows, tiles_m, tiles_n, splits;
+};
+
 struct ChunkParams {
     SeqGeom geo;
     const void *q, *k, *v;        // [n_tokens, H, dk|dv] in the element type
@@ -277,6 +298,9 @@ hipError_t scalar_gates(int dtype, const void *x, const void *w, const float *ne
 
 // SiLU(x[:, :h]) * x[:, h:] over rows of 2h elements; h % (16 / sizeof(E)) == 0.
 hipError_t swiglu(int dtype, const void *x, void *y, int64_t rows, int hidden, hipStream_t stream);
+
+void wgrad_plan(WgradParams &p);
+hipError_t wgrad(int dtype, const WgradParams &p, hipStream_t stream);
 
 hipError_t causal_conv(int dtype, const ConvParams &p, hipStream_t stream);
 int64_t conv_bwd_part_floats(int64_t n_seqs, int64_t T, int64_t D, int K);

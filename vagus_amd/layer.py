@@ -282,18 +282,35 @@ class GatedDeltaNet(nn.Module):
             on = on - {'gate'}
         return on
 
-    def _gates(self, x, *, raw_gate: bool = False, raw_beta: bool = False):
+    def _input_projections(self) -> tuple:
+        """The names of the projections that read the layer's input."""
+        return ('wq', 'wk', 'wv', 'wg') + {'none': (), 'scalar': ('wa',), 'vector': ('wa1',)}[self.gate] \
+            + (('wb',) if self.delta else ())
+
+    def _plain_projections(self) -> bool:
+        """Whether the projections are plain bias-free nn.Linear modules (and the
+        methods that call them this class's own), so that a grouped product may
+        stand for their calls."""
+        names = self._input_projections() + (('wa2',) if self.gate == 'vector' else ()) \
+            + (('wo',) if self.out_proj else ())
+        mods = [getattr(self, n) for n in names]
+        return (type(self)._gates is GatedDeltaNet._gates and type(self)._output is GatedDeltaNet._output
+                and all(_plain_module(m, nn.Linear) and m.bias is None for m in mods))
+
+    def _gates(self, x, *, raw_gate: bool = False, raw_beta: bool = False, proj: dict | None = None):
         """(g, beta): log-decay (fp32) and write strength (fp32), or with
         raw_gate / raw_beta the kernel's inputs (the per-channel pre-activation
-        (B, L, H, dk) and beta logits, in x's dtype) (:708-739)."""
+        (B, L, H, dk) and beta logits, in x's dtype) (:708-739).  proj: the
+        projections of x already formed, by name."""
         g = beta = None
         H, dk = self.head_count, self.key_head_dim
+        out = lambda n: proj[n] if proj else getattr(self, n)(x)  # noqa: E731
         if self.gate == 'scalar':
             assert not raw_gate, 'the fused gate activation is KDA-only (vector gate)'
-            g = -self.A_log.float().exp() * F.softplus(self.wa(x).float() + self.dt_bias.float())
+            g = -self.A_log.float().exp() * F.softplus(out('wa').float() + self.dt_bias.float())
         elif self.gate == 'vector':
             B, L = x.shape[0], x.shape[1]
-            f = self.wa2(self.wa1(x))
+            f = ops.projections(proj['wa1'], self.wa2.weight)[0] if proj else self.wa2(self.wa1(x))
             if raw_gate:
                 g = f.view(B, L, H, dk)
             elif self.gate_lower_bound is not None:
@@ -303,7 +320,7 @@ class GatedDeltaNet(nn.Module):
                 f = f.float() + self.dt_bias.float()
                 g = -self.A_log.float().exp()[:, None] * F.softplus(f).view(B, L, H, dk)
         if self.delta and hasattr(self, 'wb'):
-            beta = self.wb(x) if raw_beta else torch.sigmoid(self.wb(x).float())
+            beta = out('wb') if raw_beta else torch.sigmoid(out('wb').float())
         return g, beta
 
     @staticmethod
@@ -350,11 +367,11 @@ class GatedDeltaNet(nn.Module):
                             disable_recompute=self.disable_recompute,
                             lower_bound=self.gate_lower_bound, cu_seqlens=cu_seqlens)
 
-    def _output(self, o, x):
+    def _output(self, o, x, *, proj: dict | None = None):
         """RMSNorm(o) x SiLU(W_g x) per head, then W_o (:814-825): one HIP pass
-        for the epilogue."""
+        for the epilogue.  proj: the projections of x already formed, by name."""
         B, L = x.shape[0], x.shape[1]
-        gate = self.wg(x).view(B, L, self.head_count, self.value_head_dim)
+        gate = (proj['wg'] if proj else self.wg(x)).view(B, L, self.head_count, self.value_head_dim)
         if _autograd(o, gate, self.o_norm.gamma):
             o = o.to(gate.dtype)
             if _plain_module(self.o_norm, RMSNorm):
@@ -364,19 +381,29 @@ class GatedDeltaNet(nn.Module):
             o = o.reshape(B, L, -1)
         else:
             o = ops.rms_norm_gated(o.to(gate.dtype), gate, self.o_norm.gamma, eps=self.o_norm.eps).reshape(B, L, -1)
-        return self.wo(o) if self.out_proj else o
+        if not self.out_proj:
+            return o
+        return ops.projections(o, self.wo.weight)[0] if proj else self.wo(o)
 
     # --- training / stateless --------------------------------------------
 
     def forward(self, x, is_causal: bool = True):
         assert is_causal, 'linear attention is causal by construction'
-        qp, kp, vp = self.wq(x), self.wk(x), self.wv(x)
+        grouped = _autograd(x, *self.parameters()) and self._plain_projections()
+        if grouped:
+            # one function for the projections of x: _gates and _output take theirs from it
+            names = self._input_projections()
+            y = dict(zip(names, ops.projections(x, *(getattr(self, n).weight for n in names))))
+        else:
+            y = {}
+        qp, kp, vp = (y[n] if grouped else getattr(self, n)(x) for n in ('wq', 'wk', 'wv'))
         on = self._active_fusions(qp)
         q, k, v = self._heads(qp, kp, vp, l2norm='l2norm' not in on)
-        g, beta = self._gates(x, raw_gate='gate' in on, raw_beta='beta' in on)
+        kw = dict(proj=y) if grouped else {}
+        g, beta = self._gates(x, raw_gate='gate' in on, raw_beta='beta' in on, **kw)
         beta, w = self._write(x, k, g, beta)
         o, _ = self._scan(q, k, v, g, beta, None, fusions=on, w=w)
-        return self._output(o, x)
+        return self._output(o, x, **kw)
 
     # --- streaming ---------------------------------------------------------
 

@@ -1370,6 +1370,80 @@ def short_conv(x, weight, activation=None):
     return short_conv_expression(x, weight, activation)
 
 
+def linear_wgrads(x, dys):
+    """dy^T x for each dy (T, n_i) of dys and x (T, dim), 16-bit, in one split-sum
+    kernel (vgdr_linear_wgrad).  Widths that are no multiple of 8 are padded
+    with zero columns."""
+    T, dim = x.shape
+
+    def rows(t):
+        t = t if t.shape[1] % 8 == 0 else F.pad(t, (0, -t.shape[1] % 8))
+        ok = t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1] and t.data_ptr() % 16 == 0
+        return t if ok else _aligned(t)
+
+    x, mats = rows(x), [rows(t) for t in dys]
+    n = [t.shape[1] for t in mats]
+    dws = [torch.empty(m, x.shape[1], dtype=x.dtype, device=x.device) for m in n]
+    c = len(mats)
+    L = _lib.load()
+    ns = (ctypes.c_int64 * c)(*n)
+    with torch.cuda.device(x.device):
+        nbytes = L.vgdr_linear_wgrad_workspace_size(_DTYPES[x.dtype], c, ns, T, x.shape[1])
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+        _lib.check(L.vgdr_linear_wgrad(_DTYPES[x.dtype], c, (ctypes.c_void_p * c)(*(t.data_ptr() for t in mats)),
+                                       (ctypes.c_int64 * c)(*(t.stride(0) for t in mats)), ns, x.data_ptr(), x.stride(0),
+                                       (ctypes.c_void_p * c)(*(t.data_ptr() for t in dws)), _ptr(ws), nbytes, T,
+                                       x.shape[1], _stream(x.device)))
+    return [w[:t.shape[1], :dim] for w, t in zip(dws, dys)]
+
+
+class _Projections(torch.autograd.Function):
+    """F.linear(x, w) for several weights of one input: the products and the
+    input's gradient are the library's (the gradient accumulated by the
+    products themselves, in place of one addition each), the weights'
+    gradients one split-sum kernel.  A backward that is itself to be
+    differentiated (create_graph) runs through torch."""
+
+    @staticmethod
+    def forward(ctx, x, *ws):
+        ctx.save_for_backward(x, *ws)
+        ctx.set_materialize_grads(False)
+        return tuple(F.linear(x, w) for w in ws)
+
+    @staticmethod
+    def backward(ctx, *dys):
+        x, *ws = ctx.saved_tensors
+        used = [i for i, d in enumerate(dys) if d is not None]
+        if torch.is_grad_enabled():
+            need = [t for t, n in zip((x, *ws), ctx.needs_input_grad) if n]
+            out = torch.autograd.grad([F.linear(x, ws[i]) for i in used], need, [dys[i] for i in used],
+                                      create_graph=True, allow_unused=True)
+            out = iter(out)
+            return tuple(next(out) if n else None for n in ctx.needs_input_grad)
+        flat = {i: dys[i].reshape(-1, dys[i].shape[-1]) for i in used}
+        dx = None
+        if ctx.needs_input_grad[0]:
+            # the widest first: its product is rounded before the others add to it
+            for i in sorted(used, key=lambda i: -ws[i].shape[0]):
+                dx = flat[i] @ ws[i] if dx is None else dx.addmm_(flat[i], ws[i])
+            dx = None if dx is None else dx.view(x.shape)
+        dws = [None] * len(ws)
+        want = [i for i in used if ctx.needs_input_grad[1 + i]]
+        if want:
+            for i, w in zip(want, linear_wgrads(x.reshape(-1, x.shape[-1]), [flat[i] for i in want])):
+                dws[i] = w
+        return (dx, *dws)
+
+
+def projections(x, *ws):
+    """[F.linear(x, w) for w in ws], at most 8, differentiable: with 16-bit
+    tensors the weights' gradients come from one kernel (_Projections)."""
+    if (_wants_grad(x, *ws) and x.dtype in (torch.bfloat16, torch.float16) and _kernel_autograd(x, *ws)
+            and len(ws) <= 8):
+        return _Projections.apply(x, *ws)
+    return tuple(F.linear(x, w) for w in ws)
+
+
 def chunk_write_bwd(q, k, v, w, g, initial_state, do, dht=None, *, scale=None, cu_seqlens=None, chunk_size=64):
     """Backward of chunk_scan_vec with explicit write vectors w (B, T, H, dk)
     without autograd (vgdr_chunk_bwd_w; 16-bit q, k, v, w, per-channel g,
