@@ -141,6 +141,10 @@ const char *vgdr_last_error(void);
  * and chunk_size; contents irrelevant): it holds the per-chunk intermediate
  * products and, for a packed batch, the segment table (see
  * vgdr_varlen_prepare).  Calls sharing one workspace must not overlap.
+ * For a dense 16-bit call of few (sequence, head) pairs and 4,096 tokens or
+ * more the size includes the states that split sequences leave between their
+ * segments; a workspace without room for those is accepted down to the
+ * size of the other parts and runs such a call unsplit (equal up to rounding).
  */
 int64_t vgdr_chunk_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
                                   int64_t n_seqs, int varlen, int chunk_size);
@@ -207,7 +211,7 @@ int vgdr_chunk_prep_fused(int dtype, int gate_kind, int use_delta,
  * VGDR_CHUNK_SCRATCH_BYTES long, which exists on every GPU where the library's
  * code object is loaded (its first kernel launch of any entry point there)
  * until the end of the process: every process using the library holds it on
- * each GPU it runs on, whether or not it calls this entry point.  A call whose vgdr_chunk_workspace_size exceeds it
+ * each GPU it runs on, whether or not it calls this entry point.  A call whose vgdr_chunk_workspace_size (without the split sequences' states) exceeds it
  * returns VGDR_ERR_INVALID (use vgdr_chunk_fwd_fused with a workspace).
  * Calls that overlap on one GPU (two streams, two threads) share that array
  * and race; serialise them.  Otherwise the arguments, checks and results are

@@ -160,6 +160,24 @@ ChunkWs chunk_layout(int dtype, int gate_kind, int chunk, int64_t B, int64_t T, 
     return w;
 }
 
+// A split sequence's states follow the `used` bytes of a workspace.  A call splits where the workspace has
+// room for them: the sizes that the *_workspace_size functions return have; a smaller one, down
+// to the call's own need, runs it unsplit.
+int64_t with_segments(int64_t used, int64_t seg_bytes) { return seg_bytes ? (used + 255) / 256 * 256 + seg_bytes : used; }
+void take_segments(vgdr::ChunkParams &p, int dtype, int64_t dk, int64_t dv, int gate_kind, int chunk, void *workspace,
+                   int64_t workspace_bytes, int64_t used) {
+    if (p.geo.cu || !p.use_delta) return;
+    const vgdr::SegPlan s = vgdr::chunk_segments(dtype, (int)dk, gate_kind == VGDR_GATE_VECTOR, p.geo.n_seqs, p.H, dv,
+                                                 p.geo.chunks_per_seq, chunk);
+    if (!s.n_segs || workspace_bytes < with_segments(used, s.bytes)) return;
+    char *at = static_cast<char *>(workspace) + with_segments(used, s.bytes) - s.bytes;
+    p.n_segs = s.n_segs;
+    p.seg_chunks = s.seg_chunks;
+    p.seg_nw = s.nw;
+    p.seg_s = reinterpret_cast<float *>(at);
+    p.seg_m = reinterpret_cast<float *>(at + s.m_off);
+}
+
 // workspace of the backward: the forward's (table, blocks), then each chunk's
 // entry state and exit-state gradient (dk x dv per (chunk, head) in the element
 // type); with the per-channel gate also chunk prep's N (CH x CH fp32 per
@@ -252,6 +270,7 @@ int chunk_call(const char *fn, int phases, int dtype, int gate_kind, int use_del
     p.scale = scale;
     p.fz = fz;
     p.w = w;
+    take_segments(p, dtype, dk, dv, gate_kind, chunk, workspace, workspace_bytes, need);
     int32_t *table = cu_seqlens ? static_cast<int32_t *>(workspace) : nullptr;
     return hip_status(vgdr::chunk_fwd(dtype, (int)dk, chunk, gate_kind == VGDR_GATE_VECTOR, p, table, phases, stream),
                       fn);
@@ -284,7 +303,9 @@ int64_t vgdr_chunk_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T
                                   int64_t n_seqs, int varlen, int chunk_size) {
     if (B < 0 || T < 0 || H <= 0 || n_seqs < 0) return 0;
     const int chunk = effective_chunk(dtype, dk, chunk_size);
-    return chunk_layout(dtype, gate_kind, chunk, B, T, H, dk, n_seqs, varlen).total;
+    const int64_t used = chunk_layout(dtype, gate_kind, chunk, B, T, H, dk, n_seqs, varlen).total;
+    return varlen ? used : with_segments(used, vgdr::chunk_segments_bound(dtype, (int)dk, gate_kind == VGDR_GATE_VECTOR,
+                                                                          n_seqs, H, (T + chunk - 1) / chunk, chunk));
 }
 
 #define VGDR_CHUNK_ARGS                                                                                    \
@@ -338,7 +359,9 @@ int64_t vgdr_chunk_bwd_workspace_size(int dtype, int gate_kind, int64_t B, int64
                                       int64_t dv, int64_t n_seqs, int varlen, int chunk_size) {
     if (B < 0 || T < 0 || H <= 0 || n_seqs < 0 || dv < 0) return 0;
     const int chunk = effective_chunk(dtype, dk, chunk_size);
-    return bwd_layout(dtype, gate_kind, chunk, B, T, H, dk, dv, n_seqs, varlen).total;
+    const int64_t used = bwd_layout(dtype, gate_kind, chunk, B, T, H, dk, dv, n_seqs, varlen).total;
+    return varlen ? used : with_segments(used, vgdr::chunk_segments(dtype, (int)dk, gate_kind == VGDR_GATE_VECTOR, n_seqs,
+                                                                    H, dv, (T + chunk - 1) / chunk, chunk).bytes);
 }
 
 #define VGDR_BWD_ARGS                                                                                        \
@@ -459,6 +482,7 @@ int bwd_call(const char *fn, bool saved, bool delta, VGDR_BWD_ARGS, const vgdr_f
         f.nout = const_cast<float *>(p.nbuf);
         f.h0 = initial_state;
     }
+    if (!saved) take_segments(f, dtype, dk, dv, gate_kind, chunk, workspace, workspace_bytes, ws.total);
     int32_t *table = cu_seqlens ? reinterpret_cast<int32_t *>(wsb) : nullptr;
     if (f.geo.n_seqs == 0) return VGDR_OK;
     if (saved && dtype == VGDR_F32)

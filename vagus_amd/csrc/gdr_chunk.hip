@@ -1505,10 +1505,17 @@ __device__ __forceinline__ typename Elem<E>::frag2 ld_tr_pair(const E *p0, const
 // OUT false (with HS): only those states -- no outputs, so no U~ hand-over,
 // no Q copy and no A, Q loads or products in the output waves; the backward's
 // entry-state walk.
+// OUT false without HS (WALK): the first pass over a split sequence (chunk_segments),
+// its chain alone: every segment but the last, from a zero state and (further
+// columns, with V = 0) from the identity.  No output waves and no hand-over.  The
+// walk is bound by the chain's latency and, with several chain waves on a CU,
+// by their LDS reads of the same K rows, so a wave owns NS strips: two where
+// the columns are many (walk_width), one K operand then serving both.
 template <int DK, int CH, int NW, int NP, typename E, bool VEC, bool DELTA, bool HS = false, bool OUT = true,
-          int NO = 2>
+          int NO = 2, int NS = 1>
 __global__ void __launch_bounds__(64 * (NW + NO + NP))
-__attribute__((amdgpu_waves_per_eu(1, (NW + NO + NP + 3) / 4)))
+__attribute__((amdgpu_waves_per_eu(!OUT && !HS && !VEC && NS == 1 ? 3 : 1,
+                                   !OUT && !HS && !VEC && NS == 1 ? 3 : (NW + NO + NP + 3) / 4)))
 chunk_pipe_kernel(const ChunkParams p) {
     static_assert(sizeof(E) == 2, "transpose reads take 16-bit elements");
     using EL = Elem<E>;
@@ -1516,7 +1523,12 @@ chunk_pipe_kernel(const ChunkParams p) {
     typedef E E4 __attribute__((ext_vector_type(4)));
     using CB = ChunkBlock<E, CH, DK, VEC ? 2 : 1>;
     using KQ = KQRows<DK>;
-    constexpr int NB = CH / 16, NKB = DK / 16, DVT = 16 * NW, NPT = 64 * NP;
+    // WALK: the first pass over a split sequence, its chain alone (no output waves); a chain wave owns
+    // NS column strips
+    constexpr bool WALK = !OUT && !HS;
+    static_assert(WALK ? NO == 0 : NO > 0, "the segment walk has no output waves, the others have");
+    static_assert(WALK || NS == 1, "one strip a wave besides the walk");
+    constexpr int NB = CH / 16, NKB = DK / 16, DVT = 16 * NS * NW, NPT = 64 * NP;
     constexpr int PK = KQ::PITCH, PV = (VEC && NW == 4) ? DVT + 8 : DVT + 16;
     constexpr int SP = DK + 8;                                   // hand-over state row pitch (elements)
     constexpr int TEB = CH * CH * (int)sizeof(E);                // bytes of TE in a slot
@@ -1528,7 +1540,6 @@ chunk_pipe_kernel(const ChunkParams p) {
     // straight from global memory (the whole-row loads and an LDS transpose in
     // the output waves measured no faster there)
     constexpr bool QL = NP >= 4 && OUT;
-    static_assert(OUT || HS, "a walk without outputs stores the entry states");
 
     __shared__ __attribute__((aligned(16))) E K0[CH * PK];
     __shared__ __attribute__((aligned(16))) E K1[CH * PK];
@@ -1538,8 +1549,8 @@ chunk_pipe_kernel(const ChunkParams p) {
     __shared__ __attribute__((aligned(16))) E V1[CH * PV];
     __shared__ __attribute__((aligned(16))) char B0[TEB + FB];
     __shared__ __attribute__((aligned(16))) char B1[TEB + FB];
-    __shared__ __attribute__((aligned(16))) E SH[2 * NW * 16 * SP];
-    __shared__ __attribute__((aligned(16))) E UH[2 * NW * (NB / 2) * 64 * 8];
+    __shared__ __attribute__((aligned(16))) E SH[WALK ? 8 : 2 * NW * 16 * SP];
+    __shared__ __attribute__((aligned(16))) E UH[OUT ? 2 * NW * (NB / 2) * 64 * 8 : 8];
     __shared__ __attribute__((aligned(16))) E QS[QL ? 2 * CH * DK : 8];  // Q (VEC: Q*G), slot c & 1: chunk c
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -1550,18 +1561,33 @@ chunk_pipe_kernel(const ChunkParams p) {
     const int xcd = b & 7, y = b >> 3;
     const int tile = y % p.n_tiles;
     const int pos = (y / p.n_tiles) * 8 + xcd;
-    if (pos >= p.geo.n_seqs * H) return;
+    const int nsegs = WALK ? p.n_segs - 1 : (p.n_segs ? p.n_segs : 1);   // the walk leaves the last segment out
+    if (pos >= p.geo.n_seqs * nsegs * H) return;
     const int h = pos % H;
-    const int spos = pos / H;
+    int spos = pos / H, seg = 0;
+    if (nsegs > 1) {
+        seg = spos % nsegs;
+        spos /= nsegs;
+    }
     const int seq = p.geo.order ? p.geo.order[spos] : spos;
     int64_t bos, eos;
     seq_bounds(p.geo, seq, bos, eos);
-    const int64_t cbase = chunk_base(p.geo, seq);
+    int64_t cbase = chunk_base(p.geo, seq);
+    if (p.n_segs) {                                           // the segment's own tokens and chunks
+        const int64_t step = (int64_t)p.seg_chunks * CH, end = bos + (seg + 1) * step;
+        bos += seg * step;
+        eos = end < eos ? end : eos;
+        cbase += (int64_t)seg * p.seg_chunks;
+    }
     const int col0 = tile * DVT;
+    // WALK: the columns from DV on are the identity's, walked with V = 0: those of seg_m (segment 0 enters
+    // from the call's own state and needs none)
+    const int ncols = WALK && seg > 0 ? DV + DK : DV;
+    if (WALK && col0 >= ncols) return;
     const int64_t sqk = (int64_t)H * DK, sv = (int64_t)H * DV;
     const E *kg = reinterpret_cast<const E *>(p.k) + (int64_t)h * DK;
     const E *qg = reinterpret_cast<const E *>(p.q) + (int64_t)h * DK;
-    const E *vg = reinterpret_cast<const E *>(p.v) + (int64_t)h * DV + col0;
+    const E *vg = reinterpret_cast<const E *>(p.v) + (int64_t)h * DV + (WALK && col0 >= DV ? 0 : col0);
     const char *blocks = reinterpret_cast<const char *>(p.blocks);
     const int64_t len = eos - bos;
     const int nchunks = (int)((len + CH - 1) / CH);
@@ -1673,19 +1699,47 @@ chunk_pipe_kernel(const ChunkParams p) {
 
     // ======================= chain waves ====================================
     if (wave < NW) {
-        const int wcol = 16 * wave;
-        const bool wvalid = col0 + wcol < DV;                  // DV % 16 == 0
-        // entry state (C layout: S[kt][j] = S[16kt + 4g + j][col0 + wcol + r])
-        f32x4 S[NKB];
-        {
+        const int wcol = 16 * NS * wave;
+        const bool wvalid = col0 + wcol < ncols;               // DV % 16 == 0
+        // per strip: its column among its kind's (V's, the identity's), a state row's width, and where
+        // it enters from and leaves to (null: zeros, not wanted)
+        bool ident[NS];
+        int scol[NS], width[NS];
+        const float *enter[NS];
+        float *leave[NS];
+        const int64_t sh0 = ((int64_t)seq * H + h) * DK * DV;
+        auto seg_state = [&](int i) { return p.seg_s + (((int64_t)seq * (p.n_segs - 1) + i) * H + h) * DK * DV; };
+        unroll<NS>([&](auto t) {
+            const int col = col0 + wcol + 16 * (int)t;
+            ident[t] = WALK && col >= DV;
+            scol[t] = ident[t] ? col - DV : col;
+            width[t] = ident[t] ? DK : DV;
+            enter[t] = p.h0 ? p.h0 + sh0 : nullptr;
+            leave[t] = p.ht ? p.ht + sh0 : nullptr;
+            if constexpr (WALK) {
+                if (seg > 0) enter[t] = nullptr;
+                leave[t] = seg_state(seg);
+                if (ident[t]) leave[t] = p.seg_m + (((int64_t)seq * (p.n_segs - 2) + seg - 1) * H + h) * DK * DK;
+                if (col >= ncols) leave[t] = nullptr;
+            } else if (p.n_segs) {
+                if (seg > 0) enter[t] = seg_state(seg - 1);
+                if (seg < p.n_segs - 1) leave[t] = nullptr;
+            }
+        });
+        // entry state (C layout: S[t][kt][j] = S[16kt + 4g + j][scol[t] + r])
+        f32x4 S[NS][NKB];
+        unroll<NS>([&](auto t) {
             const int g4 = lane >> 4, r16 = lane & 15;
-            const int64_t sbase = ((int64_t)seq * H + h) * DK * DV + col0 + wcol + r16;
 #pragma unroll
             for (int kt = 0; kt < NKB; ++kt)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    S[kt][j] = (p.h0 && wvalid) ? p.h0[sbase + (int64_t)(16 * kt + 4 * g4 + j) * DV] : 0.f;
-        }
+                for (int j = 0; j < 4; ++j) {
+                    const int row = 16 * kt + 4 * g4 + j;
+                    if (WALK && ident[t]) S[t][kt][j] = row == scol[t] + r16 ? 1.f : 0.f;
+                    else S[t][kt][j] = (enter[t] && wvalid && (!WALK || scol[t] < DV))
+                                           ? enter[t][(int64_t)row * DV + scol[t] + r16] : 0.f;
+                }
+        });
         for (int c = 0; c < nchunks; ++c) {
             const int z = opaque_s(0);
             lds_barrier();                                    // barrier c
@@ -1711,7 +1765,7 @@ chunk_pipe_kernel(const ChunkParams p) {
             f32x4 gx[NB], gev[NB], gcv[VEC ? NKB : 1];
             float gc = 0.f;
             F2 te[NB][NB / 2];
-            typename EL::frag vf[NB];
+            typename EL::frag vf[NS][NB];
             if constexpr (VEC) {
                 unroll<NKB>([&](auto kt) { gcv[kt] = ld4(gs + 16 * kt + 4 * g4); });     // Gc per key channel
             } else {
@@ -1727,82 +1781,109 @@ chunk_pipe_kernel(const ChunkParams p) {
                         if (2 * q <= I) te[I][q] = ld_pair<E>(TEs + frag_pair_pos<NB>(I, q, 0));
                     });
                 });
-            // V rows in C layout: V[16 I + 4 g + j][wcol + r]
-            unroll<NB>([&](auto I) { vf[I] = ld_tr<E>(Vtr + 16 * I * PV); });
+            // V rows in C layout: V[16 I + 4 g + j][wcol + 16 t + r]
+            unroll<NS>([&](auto t) {
+                unroll<NB>([&](auto I) { vf[t][I] = ld_tr<E>(Vtr + 16 * I * PV + 16 * (int)t); });
+                if constexpr (WALK) {
+                    if (ident[t]) unroll<NB>([&](auto I) { vf[t][I] = typename EL::frag{}; });
+                }
+            });
             __builtin_amdgcn_sched_barrier(0);
 
-            F2 Sb[NKB / 2];
+            F2 Sb[NS][NKB / 2];
 #pragma unroll
-            for (int q = 0; q < NKB / 2; ++q) {
-                Sb[q] = EL::cvt2(S[2 * q], S[2 * q + 1]);
-                // rows 32 q + 4 g .. + 3 and 32 q + 16 + 4 g .. + 3 of column r
-                *reinterpret_cast<E4 *>(sh + 32 * q) = __builtin_shufflevector(Sb[q], Sb[q], 0, 1, 2, 3);
-                *reinterpret_cast<E4 *>(sh + 32 * q + 16) = __builtin_shufflevector(Sb[q], Sb[q], 4, 5, 6, 7);
-            }
-            f32x4 U[NB];
+            for (int t = 0; t < NS; ++t)
+#pragma unroll
+                for (int q = 0; q < NKB / 2; ++q) {
+                    Sb[t][q] = EL::cvt2(S[t][2 * q], S[t][2 * q + 1]);
+                    // rows 32 q + 4 g .. + 3 and 32 q + 16 + 4 g .. + 3 of column r
+                    if constexpr (!WALK) {
+                        *reinterpret_cast<E4 *>(sh + 32 * q) = __builtin_shufflevector(Sb[t][q], Sb[t][q], 0, 1, 2, 3);
+                        *reinterpret_cast<E4 *>(sh + 32 * q + 16) =
+                            __builtin_shufflevector(Sb[t][q], Sb[t][q], 4, 5, 6, 7);
+                    }
+                }
+            f32x4 U[NS][NB];
             if constexpr (DELTA) {
-                // P = K S (C layout), NB independent accumulation chains
-                f32x4 P[NB];
+                // P = K S (C layout), NB independent accumulation chains per strip
+                f32x4 P[NS][NB];
 #pragma unroll
-                for (int I = 0; I < NB; ++I) P[I] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < NS; ++t)
+#pragma unroll
+                    for (int I = 0; I < NB; ++I) P[t][I] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int q = 0; q < NKB / 2; ++q)
 #pragma unroll
-                    for (int I = 0; I < NB; ++I) P[I] = mfma_pair(ld_pair<E>(Krow + 16 * I * PK + 32 * q), Sb[q], P[I]);
+                    for (int I = 0; I < NB; ++I) {
+                        const F2 k = ld_pair<E>(Krow + 16 * I * PK + 32 * q);
+#pragma unroll
+                        for (int t = 0; t < NS; ++t) P[t][I] = mfma_pair(k, Sb[t][q], P[t][I]);
+                    }
                 // X = V - GX P ;  U~ = TE X
-                F2 Xb[NB / 2];
+                F2 Xb[NS][NB / 2];
+#pragma unroll
+                for (int t = 0; t < NS; ++t)
+#pragma unroll
+                    for (int q = 0; q < NB / 2; ++q) {
+                        const f32x4 v0 = EL::tof(vf[t][2 * q]), v1 = EL::tof(vf[t][2 * q + 1]);
+                        if constexpr (VEC) Xb[t][q] = EL::cvt2(v0 - P[t][2 * q], v1 - P[t][2 * q + 1]);
+                        else Xb[t][q] = EL::cvt2(v0 - P[t][2 * q] * gx[2 * q], v1 - P[t][2 * q + 1] * gx[2 * q + 1]);
+                    }
+#pragma unroll
+                for (int I = 0; I < NB; ++I)
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) {
+                        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int q = 0; 2 * q <= I; ++q) acc = mfma_pair(te[I][q], Xb[t][q], acc);
+                        U[t][I] = acc;
+                    }
+            } else {
+                unroll<NS>([&](auto t) { unroll<NB>([&](auto I) { U[t][I] = EL::tof(vf[t][I]); }); });
+            }
+            F2 Wb[NS][NB / 2];
+#pragma unroll
+            for (int t = 0; t < NS; ++t)
 #pragma unroll
                 for (int q = 0; q < NB / 2; ++q) {
-                    if constexpr (VEC) Xb[q] = EL::cvt2(EL::tof(vf[2 * q]) - P[2 * q], EL::tof(vf[2 * q + 1]) - P[2 * q + 1]);
-                    else Xb[q] = EL::cvt2(EL::tof(vf[2 * q]) - P[2 * q] * gx[2 * q],
-                                          EL::tof(vf[2 * q + 1]) - P[2 * q + 1] * gx[2 * q + 1]);
+                    const F2 ub = EL::cvt2(U[t][2 * q], U[t][2 * q + 1]);
+                    if constexpr (OUT) *reinterpret_cast<F2 *>(uh + 512 * q) = ub;
+                    if constexpr (VEC) Wb[t][q] = ub;              // Gend is in the K*Gend tile
+                    else Wb[t][q] = EL::cvt2(U[t][2 * q] * gev[2 * q], U[t][2 * q + 1] * gev[2 * q + 1]);
                 }
-#pragma unroll
-                for (int I = 0; I < NB; ++I) {
-                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int q = 0; 2 * q <= I; ++q) acc = mfma_pair(te[I][q], Xb[q], acc);
-                    U[I] = acc;
-                }
-            } else {
-                unroll<NB>([&](auto I) { U[I] = EL::tof(vf[I]); });
-            }
-            F2 Wb[NB / 2];
-#pragma unroll
-            for (int q = 0; q < NB / 2; ++q) {
-                const F2 ub = EL::cvt2(U[2 * q], U[2 * q + 1]);
-                if constexpr (OUT) *reinterpret_cast<F2 *>(uh + 512 * q) = ub;
-                if constexpr (VEC) Wb[q] = ub;                     // Gend is in the K*Gend tile
-                else Wb[q] = EL::cvt2(U[2 * q] * gev[2 * q], U[2 * q + 1] * gev[2 * q + 1]);
-            }
             // S <- Gc S + (K*Gend)^T U~
-            if constexpr (VEC) {
 #pragma unroll
-                for (int kt = 0; kt < NKB; ++kt) S[kt] *= gcv[kt];
-            } else {
+            for (int t = 0; t < NS; ++t)
 #pragma unroll
-                for (int kt = 0; kt < NKB; ++kt) S[kt] *= gc;
-            }
+                for (int kt = 0; kt < NKB; ++kt) {
+                    if constexpr (VEC) S[t][kt] *= gcv[kt];
+                    else S[t][kt] *= gc;
+                }
 #pragma unroll
             for (int q = 0; q < NB / 2; ++q)
 #pragma unroll
-                for (int kt = 0; kt < NKB; ++kt)
-                    S[kt] = mfma_pair(ld_tr_pair<E>(Ktr + 32 * q * PK + KQ::col(16 * kt),
-                                                    Ktr + (32 * q + 16) * PK + KQ::col(16 * kt)), Wb[q], S[kt]);
+                for (int kt = 0; kt < NKB; ++kt) {
+                    const F2 k = ld_tr_pair<E>(Ktr + 32 * q * PK + KQ::col(16 * kt),
+                                               Ktr + (32 * q + 16) * PK + KQ::col(16 * kt));
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) S[t][kt] = mfma_pair(k, Wb[t][q], S[t][kt]);
+                }
         }
         if (nchunks > 0) lds_barrier();                       // barrier n
-        if (p.ht && wvalid) {
+        unroll<NS>([&](auto t) {
+            if (!leave[t] || !wvalid) return;
             const int g4 = lane >> 4, r16 = lane & 15;
-            const int64_t sbase = ((int64_t)seq * H + h) * DK * DV + col0 + wcol + r16;
 #pragma unroll
             for (int kt = 0; kt < NKB; ++kt)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) p.ht[sbase + (int64_t)(16 * kt + 4 * g4 + j) * DV] = S[kt][j];
-        }
+                for (int j = 0; j < 4; ++j)
+                    leave[t][(int64_t)(16 * kt + 4 * g4 + j) * width[t] + scol[t] + r16] = S[t][kt][j];
+        });
         return;
     }
 
     // ======================= output waves ===================================
+    if constexpr (!WALK) {
     // Output wave o covers token blocks rb(o, 0), rb(o, 1) ({0, 3} and {1, 2} at
     // CH = 64, the same A tile pairs each) of every column strip of the tile.
     // Three register sets of operands: chunk c + 2's loads are issued when chunk
@@ -1968,6 +2049,66 @@ chunk_pipe_kernel(const ChunkParams p) {
         ocompute(o1, c + 1, z);
     }
     __builtin_amdgcn_s_waitcnt(0);                            // no load left in flight at exit
+    }
+}
+
+// ===========================================================================
+// chunk_segment_kernel: the entry states of a split sequence's segments
+// ===========================================================================
+// S_(s+1) = M_s S_s + U_s in fp32, one segment after the other: the walk left U_s (segment s from
+// a zero state; S_1 itself for segment 0) in seg_s[s] and M_s in seg_m[s - 1], and seg_s[s]
+// becomes S_(s+1).  A workgroup owns 16 state columns of one (sequence, head), a wave 16 of their
+// rows; S_s is passed on through LDS.  Bound by latency (a chain of n_segs - 2 products of 0.5
+// MFLOP a workgroup), so M and U are loaded two segments ahead, into three register sets: about
+// 2 us a segment, 4 with M loaded during the products before.
+template <int DK>
+__global__ void __launch_bounds__(4 * DK) __attribute__((amdgpu_waves_per_eu(1, 2)))
+chunk_segment_kernel(const ChunkParams p) {
+    constexpr int NQ = DK / 16, PITCH = DK + 4;
+    __shared__ __attribute__((aligned(16))) float ST[2][16 * PITCH];     // S_s by column
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g4 = lane >> 4, r16 = lane & 15;
+    // the tiles of one (sequence, head) share an XCD, so that its L2 takes M in once
+    const int tiles = p.DV / 16, n = p.n_segs - 2, tile = (blockIdx.x >> 3) % tiles;
+    const int64_t unit = (int64_t)((blockIdx.x >> 3) / tiles) * 8 + (blockIdx.x & 7), seq = unit / p.H, h = unit % p.H;
+    if (seq >= p.geo.n_seqs) return;
+    const int64_t sst = (int64_t)p.H * DK * p.DV, mst = (int64_t)p.H * DK * DK;   // from segment to segment
+    float *s0 = p.seg_s + (seq * (p.n_segs - 1) * p.H + h) * DK * p.DV + 16 * tile;
+    const float *m = p.seg_m + (seq * n * p.H + h) * DK * DK + (16 * wave + r16) * DK + 4 * g4;
+    float *u = s0 + sst + (int64_t)(16 * wave + 4 * g4) * p.DV + r16;              // rows 16 wave + 4 g ..
+    struct Seg {
+        f32x4 a[NQ], u;
+    };
+    Seg x, y, z;
+    auto load = [&](Seg &d, int i) __attribute__((always_inline)) {
+        i = i < n ? i : n - 1;                                // past the end: the last segment again
+        unroll<NQ>([&](auto q) { d.a[q] = ld4(m + i * mst + 16 * q); });
+        unroll<4>([&](auto j) { d.u[(int)j] = u[i * sst + (int64_t)(int)j * p.DV]; });
+    };
+    load(x, 0);
+    load(y, 1);
+    for (int i = tid; i < DK * 16; i += 4 * DK) ST[0][(i & 15) * PITCH + (i >> 4)] = s0[(int64_t)(i >> 4) * p.DV + (i & 15)];
+    auto step = [&](Seg &d, int i) __attribute__((always_inline)) {
+        lds_barrier();
+        f32x4 acc = d.u, acc1 = {0.f, 0.f, 0.f, 0.f};
+        unroll<NQ>([&](auto q) {
+            const f32x4 b = ld4(&ST[i & 1][r16 * PITCH + 16 * q + 4 * g4]);
+            f32x4 &c = (int)q & 1 ? acc1 : acc;
+            unroll<4>([&](auto j) { c = __builtin_amdgcn_mfma_f32_16x16x4f32(d.a[q][(int)j], b[(int)j], c, 0, 0, 0); });
+        });
+        acc += acc1;
+        *reinterpret_cast<f32x4 *>(&ST[(i + 1) & 1][r16 * PITCH + 16 * wave + 4 * g4]) = acc;
+        unroll<4>([&](auto j) { u[i * sst + (int64_t)(int)j * p.DV] = acc[(int)j]; });
+    };
+    for (int i = 0; i < n; i += 3) {
+        load(z, i + 2);
+        step(x, i);
+        if (i + 1 >= n) break;
+        load(x, i + 3);
+        step(y, i + 1);
+        if (i + 2 >= n) break;
+        load(y, i + 4);
+        step(z, i + 2);
+    }
 }
 
 // ===========================================================================
@@ -2000,12 +2141,46 @@ static void launch_pipe(const ChunkParams &p, int nw, int64_t state_blocks, hipS
         hipLaunchKernelGGL((chunk_pipe_kernel<DK, CH, 1, 4, E, VEC, DELTA, HS, OUT>), grid, dim3(64 * 7), 0, stream, p);
 }
 
+// The segment walk's tile (32, 64 or 128 columns): the narrowest that runs all
+// columns at once, one workgroup a CU.  A step takes about 0.9, 1.1 and 1.9 us (dk 128):
+// 16 heads, 512 chunks in 8 segments (28,672 columns): the whole call 536, 408 and
+// 361 us; 8 heads, 64 chunks in 8 (14,336): 71, 61 and 65; 2 heads, 512 chunks in 16 (7,680): 134, 138 and 152.
+static int walk_width(int64_t cols) {
+    const int cus = device_cu_count();
+    return cols <= 32 * cus ? 32 : cols <= 64 * cus ? 64 : 128;
+}
+
+// The passes before the outputs of a split sequence: every segment but the last walked from a zero
+// state (segment 0: from the call's) and, from segment 1 on, from the identity; then the entry states.
+template <int DK, int CH, typename E, bool VEC, int NW, int NS>
+static void launch_walk(ChunkParams p, hipStream_t stream) {
+    const int64_t units = (int64_t)p.geo.n_seqs * p.H;
+    constexpr int COLS = 16 * NW * NS;
+    p.n_tiles = (p.DV + (p.n_segs > 2 ? DK : 0) + COLS - 1) / COLS;
+    const int64_t blocks = (units * (p.n_segs - 1) + 7) / 8 * 8 * p.n_tiles;
+    hipLaunchKernelGGL((chunk_pipe_kernel<DK, CH, NW, 4, E, VEC, true, false, false, 0, NS>), dim3((unsigned)blocks),
+                       dim3(64 * (NW + 4)), 0, stream, p);
+}
+
+template <int DK, int CH, typename E, bool VEC>
+static void launch_segments(const ChunkParams &p, hipStream_t stream) {
+    const int64_t units = (int64_t)p.geo.n_seqs * p.H;
+    const int wide = walk_width(units * (p.n_segs - 1) * (p.DV + (p.n_segs > 2 ? DK : 0)));
+    if (wide == 128) launch_walk<DK, CH, E, VEC, 4, 2>(p, stream);
+    else if (wide == 64) launch_walk<DK, CH, E, VEC, 4, 1>(p, stream);
+    else launch_walk<DK, CH, E, VEC, 2, 1>(p, stream);
+    if (p.n_segs > 2)
+        hipLaunchKernelGGL((chunk_segment_kernel<DK>), dim3((unsigned)((units + 7) / 8 * 8 * (p.DV / 16))),
+                           dim3(4 * DK), 0, stream, p);
+}
+
 template <int DK, int CH, typename E, int GATE, bool DELTA>
 static void launch_state(const ChunkParams &p, int nw, int64_t state_blocks, hipStream_t stream) {
     if constexpr (sizeof(E) == 2) {
         // 16-bit elements: the pipelined kernel (chain, output and producer waves)
         constexpr bool VEC = GATE == 2;
         if constexpr (DELTA) {
+            if (p.n_segs) launch_segments<DK, CH, E, VEC>(p, stream);
             if (p.hs) {                                       // a training forward: entry states saved
                 if (p.states_only)                            // the backward's walk: no outputs
                     launch_pipe<DK, CH, E, VEC, true, true, false>(p, nw, state_blocks, stream);
@@ -2047,7 +2222,7 @@ static hipError_t launch_chunk(const ChunkParams &p, int nw, int phases, hipStre
                                stream, p);
         }
     }
-    const int64_t units = (int64_t)p.geo.n_seqs * p.H;
+    const int64_t units = (int64_t)p.geo.n_seqs * p.H * (p.n_segs ? p.n_segs : 1);
     const int64_t state_blocks = (units + 7) / 8 * 8 * p.n_tiles;
     if ((phases & CHUNK_STATE) && state_blocks > 0) {
         if (p.use_delta) launch_state<DK, CH, E, GATE, true>(p, nw, state_blocks, stream);
@@ -2070,6 +2245,52 @@ static int state_waves(int64_t units, int dv, int cus) {
     }
 }
 
+// A dense call whose state tiles leave CUs idle is a serial chain of its chunks on the
+// others (one 32,768-token sequence of 16 heads: 602 of 680 us, 1.18 us a chunk on 128 CUs).
+// Its sequences are split: the segments' effects on the state are walked side by side
+// (launch_segments), their entry states follow from those, and the outputs run over all
+// segments at once.  That is about 3 state passes' work, so it takes segments enough to
+// pay for it.  dk = dv = 128, whole calls, unsplit -> split, us:
+//   scalar gate: 16 heads 512 chunks 680 -> 361; 128: 153 -> 114; 64: 82 -> 77;
+//   8 heads 64 chunks 77 -> 61, 32 chunks 45 -> 46 (4,096 tokens and up are split);
+//   2 heads 512 chunks 510 -> 134; 24 (sequence, head) pairs, 5 segments: 91 -> 91 (at least 6);
+//   per-channel gate: 8 heads 256 chunks 355 -> 183; 16 heads 128 chunks, 4 segments: 225 -> 174 (at least 4).
+// 32-column output tiles where they give six segments, else (scalar gate) 64-column ones with
+// twice the segments: 16 heads 512 chunks 432 us with 32 columns and 4 segments, 361 with 64 and 8.
+// At most 16 segments: each adds 2 us to the serial chain of entry states (2 heads, 512 chunks: 16
+// segments 134 us, 24: 158), and none under 512 tokens.
+constexpr int64_t SEG_MAX = 16, SEG_TOKENS = 512, SEG_CALL_TOKENS = 4096, SEG_PAYS = 6, SEG_PAYS_VEC = 4;
+
+SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64_t H, int64_t dv, int64_t n_chunks,
+                       int chunk) {
+    SegPlan s{};
+    const int cus = device_cu_count();
+    const int64_t units = n_seqs * H, tokens = n_chunks * chunk;
+    if (dtype == 0 || units <= 0 || dv <= 0 || units > cus || dv > 32 * cus || tokens < SEG_CALL_TOKENS) return s;
+    s.nw = 2;
+    int64_t segs = cus / (units * ((dv + 31) / 32));
+    if (!gate_vector && segs < SEG_PAYS) {
+        s.nw = 4;
+        segs = cus / (units * ((dv + 63) / 64));
+    }
+    if (segs < (gate_vector ? SEG_PAYS_VEC : SEG_PAYS)) return SegPlan{};
+    segs = segs < SEG_MAX ? segs : SEG_MAX;
+    segs = segs < tokens / SEG_TOKENS ? segs : tokens / SEG_TOKENS;
+    s.seg_chunks = (int)((n_chunks + segs - 1) / segs);
+    s.n_segs = (int)((n_chunks + s.seg_chunks - 1) / s.seg_chunks);      // >= 4: 8 chunks a segment or more
+    s.m_off = units * (s.n_segs - 1) * dk * dv * 4;
+    s.bytes = s.m_off + units * (s.n_segs - 2) * dk * dk * 4;
+    return s;
+}
+
+// units * n_segs output tiles of at most 64 columns fit the chip, so that seg_s holds at most 64 columns
+// a CU; seg_m is largest where one tile holds all of dv
+int64_t chunk_segments_bound(int dtype, int dk, int gate_vector, int64_t n_seqs, int64_t H, int64_t n_chunks, int chunk) {
+    const int64_t cus = device_cu_count(), units = n_seqs * H;
+    if (!chunk_segments(dtype, dk, gate_vector, n_seqs, H, 16, n_chunks, chunk).n_segs) return 0;
+    return 4 * dk * (64 * cus + units * (cus / units < SEG_MAX ? cus / units : SEG_MAX) * dk);
+}
+
 int64_t chunk_blocks_bytes(int dtype, int chunk, int64_t chunk_slots, int64_t H, int64_t dk, int gate_vector) {
     const int64_t es = dtype == 0 ? 4 : 2;
     const bool vec = gate_vector && dtype != 0;                            // ChunkBlock<E, chunk, dk, gate>::BYTES
@@ -2079,7 +2300,8 @@ int64_t chunk_blocks_bytes(int dtype, int chunk, int64_t chunk_slots, int64_t H,
 
 template <int DK, int CH, typename E, int GATE>
 static hipError_t run_chunk(ChunkParams p, int phases, hipStream_t stream) {
-    const int nw = state_waves<DK, CH, E, GATE>((int64_t)p.geo.n_seqs * p.H, p.DV, device_cu_count());
+    const int nw = p.n_segs ? p.seg_nw
+                            : state_waves<DK, CH, E, GATE>((int64_t)p.geo.n_seqs * p.H, p.DV, device_cu_count());
     p.n_tiles = (p.DV + 16 * nw - 1) / (16 * nw);
     return launch_chunk<DK, CH, E, GATE>(p, nw, phases, stream);
 }
