@@ -141,8 +141,8 @@ const char *vgdr_last_error(void);
  * and chunk_size; contents irrelevant): it holds the per-chunk intermediate
  * products and, for a packed batch, the segment table (see
  * vgdr_varlen_prepare).  Calls sharing one workspace must not overlap.
- * For a dense 16-bit call of few (sequence, head) pairs and 4,096 tokens or
- * more the size includes the states that split sequences leave between their
+ * For a dense 16-bit call of few (sequence, head) pairs and more than 8,192
+ * tokens (per-channel gate: 4,033 or more) the size includes the states that split sequences leave between their
  * segments; a workspace without room for those is accepted down to the
  * size of the other parts and runs such a call unsplit (equal up to rounding).
  */

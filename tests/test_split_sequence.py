@@ -1,5 +1,5 @@
-"""Dense calls of few (sequence, head) pairs and 4,096 tokens or more, whose
-sequences the chunked scan splits into segments walked side by side: against the
+"""Dense calls of few (sequence, head) pairs and more than 8,192 tokens (per-channel
+gate: 64 chunks or more), whose sequences the chunked scan splits into segments walked side by side: against the
 fp64 oracle, and against the same tokens as a packed batch, which is never
 split.  The decays are weak (a few per cent over a whole sequence), so that
 every segment depends on its entry state.
@@ -46,14 +46,15 @@ def run(x, gate, packed, grads=None):
     return [a.detach() for a in out]
 
 
-# the last chunk of one token; a segment of one chunk; dv past a tile's end and under one; two sequences
+# a last chunk of one token; dv past a tile's end and under one; two sequences; two segments (no entry-state chain)
 @pytest.mark.parametrize('gate,dtype,B,T,H,dk,dv', [
-    ('scalar', torch.bfloat16, 1, 4033, 1, 128, 128),
-    ('scalar', torch.bfloat16, 1, 4100, 16, 128, 128),
-    ('scalar', torch.float16, 2, 4161, 2, 64, 48),
-    ('none', torch.bfloat16, 1, 5000, 3, 64, 16),
-    ('none', torch.float16, 1, 8191, 2, 128, 256),
-    ('vector', torch.bfloat16, 1, 4097, 3, 128, 128),
+    ('scalar', torch.bfloat16, 1, 8193, 1, 128, 128),
+    ('scalar', torch.bfloat16, 1, 8200, 16, 128, 128),
+    ('scalar', torch.float16, 2, 8257, 2, 64, 48),
+    ('none', torch.bfloat16, 1, 9000, 3, 64, 16),
+    ('none', torch.float16, 1, 10001, 2, 128, 256),
+    ('vector', torch.bfloat16, 1, 4033, 3, 128, 128),
+    ('vector', torch.bfloat16, 4, 4100, 8, 128, 128),
     ('vector', torch.float16, 1, 4600, 2, 128, 272),
     ('vector', torch.bfloat16, 2, 4224, 1, 64, 64),
 ])
@@ -82,7 +83,7 @@ def test_split_training_pass(gate, dtype, H, dk, dv):
     Each run is within about a rounding of the element type (2^-8, 2^-11) of the exact gradients, so
     the two are within 2.5 of them of each other."""
     tol = 2.5 * (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11)
-    x = inputs(1, 4200, H, dk, dv, gate, dtype, seed=9)
+    x = inputs(1, 4200 if gate == 'vector' else 8300, H, dk, dv, gate, dtype, seed=9)
     g = torch.Generator().manual_seed(10)
     grads = torch.randn(x.v.shape, generator=g).to(dtype), torch.randn(x.initial_state.shape, generator=g)
     for i, (a, b) in enumerate(zip(run(x, gate, False, grads), run(x, gate, True, grads))):
@@ -94,7 +95,7 @@ def test_split_training_pass(gate, dtype, H, dk, dv):
 def test_workspace_without_room_runs_unsplit():
     """The size a workspace had before sequences were split is still taken: the same result up to rounding,
     and one byte less is refused."""
-    T, H, d = 4096, 2, 128
+    T, H, d = 8256, 2, 128
     x = inputs(1, T, H, d, d, 'scalar', torch.bfloat16, seed=3)
     y = {n: getattr(x, n).cuda() for n in ('q', 'k', 'v', 'g', 'beta', 'initial_state')}
     L = _lib.load()

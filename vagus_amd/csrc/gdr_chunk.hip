@@ -2249,27 +2249,33 @@ static int state_waves(int64_t units, int dv, int cus) {
 // others (one 32,768-token sequence of 16 heads: 602 of 680 us, 1.18 us a chunk on 128 CUs).
 // Its sequences are split: the segments' effects on the state are walked side by side
 // (launch_segments), their entry states follow from those, and the outputs run over all
-// segments at once.  That is about 3 state passes' work, so it takes segments enough to
-// pay for it.  dk = dv = 128, whole calls, unsplit -> split, us:
-//   scalar gate: 16 heads 512 chunks 680 -> 361; 128: 153 -> 114; 64: 82 -> 77;
-//   8 heads 64 chunks 77 -> 61, 32 chunks 45 -> 46 (4,096 tokens and up are split);
-//   2 heads 512 chunks 510 -> 134; 24 (sequence, head) pairs, 5 segments: 91 -> 91 (at least 6);
-//   per-channel gate: 8 heads 256 chunks 355 -> 183; 16 heads 128 chunks, 4 segments: 225 -> 174 (at least 4).
-// 32-column output tiles where they give six segments, else (scalar gate) 64-column ones with
+// segments at once.  That is up to 3 state passes' work (2 with two segments, which need no
+// seg_m), so it takes segments enough to pay for it.  Whole calls, unsplit -> split, us (dk = dv = 128):
+//   scalar gate: 16 heads 512 chunks 680 -> 361; 2 heads 510 -> 134; 32 (sequence, head) pairs
+//   256 chunks, 4 segments 400 -> 344, 3: 355, 2: 445 (at least SEG_PAYS); 24 pairs 129 chunks, 5: 171 -> 146;
+//   per-channel gate: 8 heads 256 chunks 355 -> 183; 16 heads 128 chunks, 4 segments 225 -> 174;
+//   32 pairs, 2 segments: 128 chunks 327 -> 293, 64 chunks 157 -> 152; 20 pairs 64 chunks, 3: 109 -> 110.
+// Scalar-gate sequences up to 8,192 tokens stay whole, though the longer of them gain too (2 heads, 64 chunks
+// 77 -> 57): a sequence of that length gives the same bits alone and in a packed batch, which is
+// never split (its lengths are on the GPU), and callers check one against the other.  Below 64 chunks the passes'
+// fixed cost takes the gain (8 heads, 32 chunks: 45 -> 46).
+// 32-column output tiles where they give SEG_NARROW segments, else (scalar gate) 64-column ones with
 // twice the segments: 16 heads 512 chunks 432 us with 32 columns and 4 segments, 361 with 64 and 8.
-// At most 16 segments: each adds 2 us to the serial chain of entry states (2 heads, 512 chunks: 16
-// segments 134 us, 24: 158), and none under 512 tokens.
-constexpr int64_t SEG_MAX = 16, SEG_TOKENS = 512, SEG_CALL_TOKENS = 4096, SEG_PAYS = 6, SEG_PAYS_VEC = 4;
+// At most SEG_MAX segments: each adds 2 us to the serial chain of entry states (2 heads, 512 chunks: 16
+// segments 134 us, 24: 158), and none under SEG_TOKENS.
+constexpr int64_t SEG_MAX = 16, SEG_TOKENS = 512, SEG_CALL = 8193, SEG_CALL_VEC = 4096;
+constexpr int64_t SEG_NARROW = 6, SEG_PAYS = 4, SEG_PAYS_VEC = 2;
 
 SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64_t H, int64_t dv, int64_t n_chunks,
                        int chunk) {
     SegPlan s{};
     const int cus = device_cu_count();
     const int64_t units = n_seqs * H, tokens = n_chunks * chunk;
-    if (dtype == 0 || units <= 0 || dv <= 0 || units > cus || dv > 32 * cus || tokens < SEG_CALL_TOKENS) return s;
+    if (dtype == 0 || units <= 0 || dv <= 0 || units > cus || dv > 32 * cus) return s;
+    if (tokens < (gate_vector ? SEG_CALL_VEC : SEG_CALL)) return s;
     s.nw = 2;
     int64_t segs = cus / (units * ((dv + 31) / 32));
-    if (!gate_vector && segs < SEG_PAYS) {
+    if (!gate_vector && segs < SEG_NARROW) {
         s.nw = 4;
         segs = cus / (units * ((dv + 63) / 64));
     }
@@ -2277,7 +2283,7 @@ SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64
     segs = segs < SEG_MAX ? segs : SEG_MAX;
     segs = segs < tokens / SEG_TOKENS ? segs : tokens / SEG_TOKENS;
     s.seg_chunks = (int)((n_chunks + segs - 1) / segs);
-    s.n_segs = (int)((n_chunks + s.seg_chunks - 1) / s.seg_chunks);      // >= 4: 8 chunks a segment or more
+    s.n_segs = (int)((n_chunks + s.seg_chunks - 1) / s.seg_chunks);      // >= 2
     s.m_off = units * (s.n_segs - 1) * dk * dv * 4;
     s.bytes = s.m_off + units * (s.n_segs - 2) * dk * dk * 4;
     return s;
