@@ -457,11 +457,11 @@ class GatedDeltaNet(nn.Module):
         return (self.short_conv_size is not None and self.key_head_dim in (64, 128)
                 and (self.value_head_dim in (64, 128) or (self.value_head_dim == 256 and self.short_conv_size == 4)))
 
-    def _decode_weights(self):
+    def _decode_weights(self, stacked):
         """The one-token decode step's projection weights regrouped, rebuilt
-        whenever a parameter changed (its storage or version): every matrix
+        whenever a parameter changed (its storage or version): `stacked`, every matrix
         that multiplies the input (W_q, W_k, W_v, W_g, and without the scalar
-        gate W_a1 and W_b) stacked into one weight, rows padded with zeros to a
+        gate W_a1 and W_b), as one weight, rows padded with zeros to a
         multiple of 64 (so that the rows of its product stay 16-byte aligned),
         so that one GEMM replaces up to six skinny ones; for the
         scalar gate [W_a; W_b] as one (2H, dim) weight (W_a alone without the
@@ -469,13 +469,7 @@ class GatedDeltaNet(nn.Module):
         constants in fp32: -exp(A_log) (scalar) or A_log (per channel), and dt_bias.
         The copies hold one more set of these weights."""
         scalar = self.gate == 'scalar'
-        stacked = [self.wq, self.wk, self.wv, self.wg]
-        if self.gate == 'vector':
-            stacked.append(self.wa1)
-        if self.delta and not scalar:
-            stacked.append(self.wb)
-        ps = [m.weight for m in stacked]
-        n = len(ps)
+        ps, n = list(stacked), len(stacked)
         if scalar:
             ps += [self.wa.weight] + ([self.wb.weight] if self.delta else [])
         if self.gate != 'none':
@@ -510,21 +504,33 @@ class GatedDeltaNet(nn.Module):
         names = ('wq', 'wk', 'wv', 'wg') + {'scalar': (), 'vector': ('wa1',), 'none': ()}[self.gate]
         if self.delta and self.gate != 'scalar':
             names += ('wb',)
-        mods = [getattr(self, n) for n in names]
-        if (not all(_plain_module(m, nn.Linear) and m.bias is None and m.weight.dtype == x.dtype for m in mods)
-                or type(self)._gates is not GatedDeltaNet._gates):
+        mods = [self._modules[n] for n in names]
+        # the modules' own parameter tables: an attribute of a module is a search, and an eager step takes 120 us
+        ws = [m._parameters.get('weight') for m in mods]
+        if not (type(self)._gates is GatedDeltaNet._gates
+                and all(_plain_module(m, nn.Linear) and m._parameters.get('bias') is None
+                        and w is not None and w.dtype == x.dtype for m, w in zip(mods, ws))):
             g, beta = self._gates(x, raw_gate=self.gate == 'vector', raw_beta=self.delta)
             return (self.wq(x), self.wk(x), self.wv(x), self.wg(x), g,
                     beta if self.delta else None, None, (self.A_log, self.dt_bias) if self.gate == 'vector' else None)
-        w, wab, gconst = self._decode_weights()
+        w, wab, gconst = self._decode_weights(ws)
         y = F.linear(x.reshape(B, -1), w)
-        widths = [H * dk, H * dk, H * dv, H * dv] + [m.weight.shape[0] for m in mods[4:]]
-        cols = y[:, :sum(widths)].split(widths, -1)
-        qp, kp, vp, og = (c.unsqueeze(1) for c in cols[:4])
+        # one view per column block (a slice and its reshape are two calls, of the 130 us of an eager step)
+        nk, nv = H * dk, H * dv
+        row, at = y.stride(0), y.storage_offset()
+        qp, kp = y.as_strided((B, 1, nk), (row, nk, 1), at), y.as_strided((B, 1, nk), (row, nk, 1), at + nk)
+        at += 2 * nk
+        vp, og = y.as_strided((B, 1, nv), (row, nv, 1), at), y.as_strided((B, 1, nv), (row, nv, 1), at + nv)
         if self.gate == 'scalar':
             return qp, kp, vp, og, None, None, (x, wab, *gconst), None
-        g = self.wa2(cols[4]).view(B, 1, H, dk) if self.gate == 'vector' else None
-        return qp, kp, vp, og, g, cols[-1].unsqueeze(1) if self.delta else None, None, gconst
+        at += 2 * nv
+        g = beta = None
+        if self.gate == 'vector':
+            g = self.wa2(y.as_strided((B, self.gate_rank), (row, 1), at)).view(B, 1, H, dk)
+            at += self.gate_rank
+        if self.delta:
+            beta = y.as_strided((B, 1, H), (row, H, 1), at)
+        return qp, kp, vp, og, g, beta, None, gconst
 
     @torch.no_grad()
     def decode_step(self, x):
