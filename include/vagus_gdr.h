@@ -508,6 +508,28 @@ int vgdr_decode_step_strided(int dtype, int gate_kind, int use_delta,
                              const vgdr_epilogue *epilogue, const vgdr_gate_proj *gate_proj,
                              hipStream_t stream);
 
+/* vgdr_decode_step_strided with the gate's parameters as the layer's module holds
+ * them, read by the kernel at every call (no copy in another type or layout):
+ *   scalar gate: x [B, dim], w_a and (delta rule) w_b [H, dim] as vgdr_gate_proj's,
+ *       A_log and dt_bias [H]; g and beta are formed as there.
+ *   per-channel gate with fusion.gate_activation: A_log [H] and dt_bias [H * dk] in place of
+ *       the fusion's fp32 ones; x, w_a, w_b and dim are not read.
+ * param_dtype: of A_log and dt_bias. */
+typedef struct vgdr_gate_params {
+    const void *x, *w_a, *w_b;
+    const void *A_log, *dt_bias;
+    int64_t dim;
+    int param_dtype;
+} vgdr_gate_params;
+int vgdr_decode_step_params(int dtype, int gate_kind, int use_delta,
+                            const void *q, const void *k, const void *v,
+                            const float *g, const float *beta,
+                            void *o, const float *initial_state, float *final_state,
+                            int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t ld_qk, int64_t ld_v,
+                            float scale, const vgdr_fusion *fusion, const vgdr_short_conv *conv,
+                            const vgdr_epilogue *epilogue, const vgdr_gate_params *params,
+                            hipStream_t stream);
+
 /* The short conv + SiLU (vgdr_short_conv's semantics) over a whole call's
  * tokens, for prefill: y[t] from x[t - K + 1 .. t] of the same sequence.
  * Replaces the module's ShortConv (opt.py:15-100; fla's causal_conv1d as the
@@ -572,6 +594,19 @@ int64_t vgdr_linear_wgrad_workspace_size(int dtype, int n_mats, const int64_t *n
 int vgdr_linear_wgrad(int dtype, int n_mats, const void *const *dy, const int64_t *ld, const int64_t *n,
                       const void *x, int64_t ldx, void *const *dw, void *workspace,
                       int64_t workspace_bytes, int64_t T, int64_t dim, hipStream_t stream);
+
+/* Projections of a few rows in one launch, y = [W_0 x | W_1 x | ...]: n_mats (at
+ * most 8) weights w[i] [n[i], dim], contiguous, that share the input x [rows, dim]
+ * (rows ldx elements apart); fp32 sums in a fixed order, rounded once.  y's rows are
+ * ldy apart; each block starts at the next multiple of 8 columns after the one
+ * before it.  dim, ldx, ldy multiples of 8, every pointer but beta 16-byte aligned.  The
+ * arrays are host arrays.  beta_mat (-1: none): that matrix's products, rounded to dtype,
+ * go to beta [rows, n[beta_mat]] in fp32 and have no block in y.  The nn.Linear calls of
+ * the reference's one-token step (linear_attention.py:600-625, :918-952); the
+ * weights are read where they lie. */
+int vgdr_project_rows(int dtype, int n_mats, const void *const *w, const int64_t *n, const void *x, int64_t ldx,
+                      void *y, int64_t ldy, int beta_mat, float *beta, int64_t rows, int64_t dim,
+                      hipStream_t stream);
 
 /* The pre-norm blocks' RMSNorm (infra/components/norm_layer.py:15-23) over rows
  * rows of dim elements, with the residual add in front of it that the blocks

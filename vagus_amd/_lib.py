@@ -44,6 +44,13 @@ class GateProj(ctypes.Structure):
                 ('dt_bias', ctypes.c_void_p), ('dim', ctypes.c_int64)]
 
 
+class GateParams(ctypes.Structure):
+    """struct vgdr_gate_params: the gate's parameters as the layer's module holds them."""
+    _fields_ = [('x', ctypes.c_void_p), ('w_a', ctypes.c_void_p), ('w_b', ctypes.c_void_p),
+                ('A_log', ctypes.c_void_p), ('dt_bias', ctypes.c_void_p), ('dim', ctypes.c_int64),
+                ('param_dtype', ctypes.c_int)]
+
+
 # every symbol the header declares, with its ctypes signature
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
 _FZ = ctypes.POINTER(Fusion)
@@ -98,6 +105,8 @@ SIGNATURES = {
     'vgdr_linear_wgrad_workspace_size': (_L, [_I, _I, ctypes.POINTER(_L), _L, _L]),
     'vgdr_linear_wgrad': (_I, [_I, _I, ctypes.POINTER(_P), ctypes.POINTER(_L), ctypes.POINTER(_L), _P, _L,
                                ctypes.POINTER(_P), _P, _L, _L, _L, _P]),
+    'vgdr_project_rows': (_I, [_I, _I, ctypes.POINTER(_P), ctypes.POINTER(_L), _P, _L, _P, _L, _I, _P, _L, _L,
+                               _P]),
     'vgdr_rms_norm': (_I, [_I, _P, _P, _P, _P, _P, _L, _L, _F, _P]),
     'vgdr_scalar_gates': (_I, [_I, _P, _P, _P, _P, _P, _P, _L, _L, _L, _P]),
     'vgdr_swiglu': (_I, [_I, _P, _P, _L, _L, _P]),
@@ -107,6 +116,8 @@ SIGNATURES = {
                               _L, _L, _L, _L, _L, _L, _F, _FZ, _SC, _EP, _P]),
     'vgdr_decode_step_strided': (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P,
                                       _L, _L, _L, _L, _L, _L, _F, _FZ, _SC, _EP, _GP, _P]),
+    'vgdr_decode_step_params': (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P,
+                                     _L, _L, _L, _L, _L, _L, _F, _FZ, _SC, _EP, ctypes.POINTER(GateParams), _P]),
     'vgdr_causal_conv1d': (_I, [_I, _P, _P, _I, _P, _P, _P, _P, _L, _L, _L, _L, _I, _I, _P]),
     'vgdr_causal_conv1d_bwd_workspace_size': (_L, [_I, _L, _L, _L, _I]),
     'vgdr_causal_conv1d_bwd': (_I, [_I, _P, _P, _P, _P, _P, _P, _L, _L, _L, _L, _I, _I, _P]),

@@ -739,12 +739,13 @@ int recurrent_call(int dtype, int gate_kind, int use_delta, const void *q, const
                    float *final_state, const int32_t *cu_seqlens, int64_t B, int64_t T, int64_t H, int64_t dk,
                    int64_t dv, int64_t n_seqs, float scale, const vgdr_fusion *fusion, const vgdr_short_conv *conv,
                    const vgdr_epilogue *epilogue, hipStream_t stream, int64_t ld_qk = 0, int64_t ld_v = 0,
-                   const vgdr_gate_proj *gp = nullptr) {
+                   const vgdr::GateProj *gp = nullptr, int param_dtype = VGDR_F32) {
     g_err[0] = 0;
     // with an explicit write vector, beta is not read; with gate projections
     // (checked by the caller) neither g nor beta is
+    const float *formed = gp ? static_cast<const float *>(gp->dt_bias) : nullptr;
     int rc = check_common("vgdr_recurrent_fwd", dtype, gate_kind, w ? 0 : use_delta, q, k, v,
-                          gp ? gp->neg_exp_a : g, gp ? gp->dt_bias : beta, o, cu_seqlens, B, T, H, dk, dv, n_seqs);
+                          gp ? formed : g, gp ? formed : beta, o, cu_seqlens, B, T, H, dk, dv, n_seqs);
     if (rc) return rc;
     if (w && !use_delta) return fail(VGDR_ERR_INVALID, "vgdr_recurrent_fwd: an explicit write vector needs the delta rule");
     vgdr::Fusion fz;
@@ -791,10 +792,11 @@ int recurrent_call(int dtype, int gate_kind, int use_delta, const void *q, const
     p.w = w;
     p.ld_qk = ld_qk;
     p.ld_v = ld_v;
+    p.param_dtype = param_dtype;
     if (gp) {
         p.g = nullptr;
         p.beta = nullptr;
-        p.gp = vgdr::GateProj{gp->x, gp->w, gp->neg_exp_a, gp->dt_bias, (int)gp->dim};
+        p.gp = *gp;
     }
     return hip_status(vgdr::recurrent_fwd(dtype, (int)dk, (int)dv, gate_kind == VGDR_GATE_VECTOR, p, stream),
                       "vgdr_recurrent_fwd launch");
@@ -811,36 +813,81 @@ int vgdr_decode_step(int dtype, int gate_kind, int use_delta, const void *q, con
                           cu_seqlens, B, T, H, dk, dv, n_seqs, scale, fusion, conv, epilogue, stream);
 }
 
+// what both strided entry points need: the strides reach only the one-token decode kernel, so a state and
+// the four-tap conv with 16-byte aligned weights (any other call would run the token walk, which reads
+// dense rows)
+static int check_strided(const char *fn, int dtype, int gate_kind, int use_delta, int64_t H, int64_t dk, int64_t dv,
+                         int64_t ld_qk, int64_t ld_v, const vgdr_short_conv *conv, const float *initial_state,
+                         const vgdr::GateProj *gp, int64_t dim) {
+    if (ld_qk < H * dk || ld_v < H * dv)
+        return fail(VGDR_ERR_INVALID, "%s: row strides (%lld, %lld) below H*dk = %lld, H*dv = %lld", fn,
+                    (long long)ld_qk, (long long)ld_v, (long long)(H * dk), (long long)(H * dv));
+    if (!conv || conv->kernel_size != 4 || !aligned16(conv->weight_q) || !aligned16(conv->weight_k) ||
+        !aligned16(conv->weight_v) || !initial_state)
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: strided rows need the four-tap short conv with 16-byte aligned weights "
+                    "and an initial state", fn);
+    if (!gp) return VGDR_OK;
+    const int64_t ve = dtype == VGDR_F32 ? 4 : 8, nt = dv > 128 ? 512 : 256;
+    if (gate_kind != VGDR_GATE_SCALAR)
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: gate projections are for the scalar gate", fn);
+    if (!gp->x || !gp->wa || (use_delta && !gp->wb) || (!gp->neg_a && !gp->a_log) || !gp->dt_bias ||
+        !aligned16(gp->x) || !aligned16(gp->wa) || (use_delta && !aligned16(gp->wb)))
+        return fail(VGDR_ERR_INVALID, "%s: gate projections need x and their weights (16-byte aligned), A_log and "
+                    "dt_bias", fn);
+    if (dim <= 0 || dim % ve || dim > 2 * nt * ve)
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: gate projection dim=%lld (a multiple of %lld up to %lld)", fn,
+                    (long long)dim, (long long)ve, (long long)(2 * nt * ve));
+    return VGDR_OK;
+}
+
 int vgdr_decode_step_strided(int dtype, int gate_kind, int use_delta, const void *q, const void *k, const void *v,
                              const float *g, const float *beta, void *o, const float *initial_state,
                              float *final_state, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t ld_qk,
                              int64_t ld_v, float scale, const vgdr_fusion *fusion, const vgdr_short_conv *conv,
                              const vgdr_epilogue *epilogue, const vgdr_gate_proj *gate_proj, hipStream_t stream) {
-    // the strides reach only the one-token decode kernel: it needs a state and the
-    // four-tap conv with 16-byte aligned weights (any other call would run the
-    // token walk, which reads dense rows)
     g_err[0] = 0;
-    if (ld_qk < H * dk || ld_v < H * dv)
-        return fail(VGDR_ERR_INVALID, "vgdr_decode_step_strided: row strides (%lld, %lld) below H*dk = %lld, "
-                    "H*dv = %lld", (long long)ld_qk, (long long)ld_v, (long long)(H * dk), (long long)(H * dv));
-    if (!conv || conv->kernel_size != 4 || !aligned16(conv->weight_q) || !aligned16(conv->weight_k) ||
-        !aligned16(conv->weight_v) || !initial_state)
-        return fail(VGDR_ERR_UNSUPPORTED, "vgdr_decode_step_strided: strided rows need the four-tap short conv "
-                    "with 16-byte aligned weights and an initial state");
+    vgdr::GateProj gp{};
+    int64_t dim = 0;
     if (gate_proj) {
-        const int64_t ve = dtype == VGDR_F32 ? 4 : 8, nt = dv > 128 ? 512 : 256;
-        if (gate_kind != VGDR_GATE_SCALAR)
-            return fail(VGDR_ERR_UNSUPPORTED, "vgdr_decode_step_strided: gate projections are for the scalar gate");
-        if (!gate_proj->x || !gate_proj->w || !gate_proj->neg_exp_a || !gate_proj->dt_bias ||
-            !aligned16(gate_proj->x) || !aligned16(gate_proj->w))
-            return fail(VGDR_ERR_INVALID, "vgdr_decode_step_strided: gate projections need x, w (16-byte aligned), "
-                        "neg_exp_a and dt_bias");
-        if (gate_proj->dim <= 0 || gate_proj->dim % ve || gate_proj->dim > 2 * nt * ve)
-            return fail(VGDR_ERR_UNSUPPORTED, "vgdr_decode_step_strided: gate projection dim=%lld (a multiple of "
-                        "%lld up to %lld)", (long long)gate_proj->dim, (long long)ve, (long long)(2 * nt * ve));
+        dim = gate_proj->dim;
+        const int64_t wb = H * dim * (dtype == VGDR_F32 ? 4 : 2);
+        gp = vgdr::GateProj{gate_proj->x, gate_proj->w, static_cast<const char *>(gate_proj->w) + wb,
+                            gate_proj->neg_exp_a, nullptr, gate_proj->dt_bias, (int)dim};
+    }
+    int rc = check_strided("vgdr_decode_step_strided", dtype, gate_kind, use_delta, H, dk, dv, ld_qk, ld_v, conv,
+                           initial_state, gate_proj ? &gp : nullptr, dim);
+    if (rc) return rc;
+    return recurrent_call(dtype, gate_kind, use_delta, q, k, v, nullptr, g, beta, o, initial_state, final_state,
+                          nullptr, B, 1, H, dk, dv, B, scale, fusion, conv, epilogue, stream, ld_qk, ld_v,
+                          gate_proj ? &gp : nullptr);
+}
+
+int vgdr_decode_step_params(int dtype, int gate_kind, int use_delta, const void *q, const void *k, const void *v,
+                            const float *g, const float *beta, void *o, const float *initial_state,
+                            float *final_state, int64_t B, int64_t H, int64_t dk, int64_t dv, int64_t ld_qk,
+                            int64_t ld_v, float scale, const vgdr_fusion *fusion, const vgdr_short_conv *conv,
+                            const vgdr_epilogue *epilogue, const vgdr_gate_params *params, hipStream_t stream) {
+    g_err[0] = 0;
+    const char *fn = "vgdr_decode_step_params";
+    if (!params || params->param_dtype < VGDR_F32 || params->param_dtype > VGDR_F16 || !params->A_log || !params->dt_bias)
+        return fail(VGDR_ERR_INVALID, "%s: A_log and dt_bias (fp32, bf16 or fp16) are required", fn);
+    const bool scalar = gate_kind == VGDR_GATE_SCALAR;
+    if (!scalar && !(gate_kind == VGDR_GATE_VECTOR && fusion && fusion->gate_activation))
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: the scalar gate's parameters, or those of the fused gate activation", fn);
+    const vgdr::GateProj gp{params->x, params->w_a, params->w_b, nullptr, params->A_log, params->dt_bias,
+                            (int)params->dim};
+    int rc = check_strided(fn, dtype, gate_kind, use_delta, H, dk, dv, ld_qk, ld_v, conv, initial_state,
+                           scalar ? &gp : nullptr, params->dim);
+    if (rc) return rc;
+    vgdr_fusion fz{};
+    if (fusion) fz = *fusion;
+    if (!scalar) {                                             // their own type: param_dtype
+        fz.A_log = static_cast<const float *>(params->A_log);
+        fz.dt_bias = static_cast<const float *>(params->dt_bias);
     }
     return recurrent_call(dtype, gate_kind, use_delta, q, k, v, nullptr, g, beta, o, initial_state, final_state,
-                          nullptr, B, 1, H, dk, dv, B, scale, fusion, conv, epilogue, stream, ld_qk, ld_v, gate_proj);
+                          nullptr, B, 1, H, dk, dv, B, scale, fusion ? &fz : nullptr, conv, epilogue, stream, ld_qk,
+                          ld_v, scalar ? &gp : nullptr, params->param_dtype);
 }
 
 int vgdr_recurrent_fwd_w(int dtype, int gate_kind, const void *q, const void *k, const void *v, const void *w,
@@ -1020,6 +1067,54 @@ int vgdr_linear_wgrad(int dtype, int n_mats, const void *const *dy, const int64_
     p.ldx = ldx;
     p.part = reinterpret_cast<float *>(workspace);
     return hip_status(vgdr::wgrad(dtype, p, stream), "vgdr_linear_wgrad launch");
+}
+
+int vgdr_project_rows(int dtype, int n_mats, const void *const *w, const int64_t *n, const void *x, int64_t ldx,
+                      void *y, int64_t ldy, int beta_mat, float *beta, int64_t rows, int64_t dim,
+                      hipStream_t stream) {
+    g_err[0] = 0;
+    const char *fn = "vgdr_project_rows";
+    if (dtype != VGDR_F32 && dtype != VGDR_BF16 && dtype != VGDR_F16)
+        return fail(VGDR_ERR_INVALID, "%s: unknown dtype %d", fn, dtype);
+    if (n_mats < 1 || n_mats > vgdr::PROJ_MAX || !w || !n)
+        return fail(VGDR_ERR_INVALID, "%s: 1 to %d matrices, got %d", fn, vgdr::PROJ_MAX, n_mats);
+    if (dim < 8 || dim % 8 || dim > 0x100000)
+        return fail(VGDR_ERR_UNSUPPORTED, "%s: dim=%lld (a multiple of 8, at most 1048576)", fn, (long long)dim);
+    if (rows < 0 || rows > 0xffff * 16LL) return fail(VGDR_ERR_INVALID, "%s: rows=%lld", fn, (long long)rows);
+    if (beta_mat < -1 || beta_mat >= n_mats || (beta_mat >= 0 && !beta))
+        return fail(VGDR_ERR_INVALID, "%s: beta_mat=%d", fn, beta_mat);
+    vgdr::ProjectParams p{};
+    int64_t cols = 0;
+    for (int i = 0; i < n_mats; ++i) {
+        if (n[i] < 1 || n[i] > 0x1000000) return fail(VGDR_ERR_INVALID, "%s: width %lld", fn, (long long)n[i]);
+        p.m[i].w = w[i];
+        p.m[i].n = (int)n[i];
+        if (i == beta_mat) continue;
+        cols = (cols + 7) / 8 * 8;
+        p.m[i].col0 = (int)cols;
+        cols += n[i];
+    }
+    if (rows == 0) return VGDR_OK;
+    if (!x || !aligned16(x) || ldx % 8 || ldx < dim)
+        return fail(VGDR_ERR_INVALID, "%s: x: 16-byte aligned rows of a multiple of 8 elements", fn);
+    if (cols && (!y || !aligned16(y) || ldy % 8 || ldy < cols))
+        return fail(VGDR_ERR_INVALID, "%s: y: 16-byte aligned rows of a multiple of 8 elements, at least %lld", fn,
+                    (long long)cols);
+    for (int i = 0; i < n_mats; ++i) {
+        if (!w[i] || !aligned16(w[i])) return fail(VGDR_ERR_INVALID, "%s: weight %d must be 16-byte aligned", fn, i);
+        if (w[i] == y) return fail(VGDR_ERR_INVALID, "%s: y must not alias an input", fn);
+    }
+    if (x == y) return fail(VGDR_ERR_INVALID, "%s: y must not alias an input", fn);
+    p.x = x;
+    p.y = y;
+    p.ldx = ldx;
+    p.ldy = ldy;
+    p.rows = (int)rows;
+    p.dim = (int)dim;
+    p.n_mats = n_mats;
+    p.beta_mat = beta_mat;
+    p.beta = beta;
+    return hip_status(vgdr::project_rows(dtype, p, stream), "vgdr_project_rows launch");
 }
 
 int vgdr_rms_norm(int dtype, const void *x, const void *residual, void *x_out, const void *gamma, void *y,

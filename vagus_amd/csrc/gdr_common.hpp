@@ -212,6 +212,13 @@ __device__ __forceinline__ float gate_activation(float f, float a_log, float dt,
     return lb_set ? lb * sigmoidf_(a * z) : -a * softplusf_(z);
 }
 
+// element i of a parameter in the element type `dtype` (0 fp32, 1 bf16, 2 fp16)
+__device__ __forceinline__ float param_f(const void *p, int dtype, int64_t i) {
+    if (dtype == 1) return (float)reinterpret_cast<const __bf16 *>(p)[i];
+    if (dtype == 2) return (float)reinterpret_cast<const _Float16 *>(p)[i];
+    return reinterpret_cast<const float *>(p)[i];
+}
+
 // 16-byte global access
 struct alignas(16) Vec16 { uint32_t w[4]; };
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

@@ -103,6 +103,24 @@ struct WgradParams {
     int rows, tiles_m, tiles_n, splits;
 };
 
+// Projections of a few rows: y[b] = [W_0 x[b] | W_1 x[b] | ...], W_i [n, dim]
+// contiguous and as its module holds it, rows of x and y ldx and ldy elements
+// apart; matrix i's outputs start at column col0 of y and (set by project_rows) at tile tile0.
+constexpr int PROJ_MAX = 8;
+struct ProjectMat {
+    const void *w;
+    int n, col0, tile0;
+};
+struct ProjectParams {
+    const void *x;
+    void *y;
+    int64_t ldx, ldy;
+    int rows, dim, n_mats;
+    int beta_mat;                 // -1, or the matrix whose products, rounded to the element type, go
+    float *beta;                  // here in fp32 [rows, n] and not to y
+    ProjectMat m[PROJ_MAX];
+};
+
 struct ChunkParams {
     SeqGeom geo;
     const void *q, *k, *v;        // [n_tokens, H, dk|dv] in the element type
@@ -207,13 +225,14 @@ struct ScanBwdParams {
 // The scalar gate and the beta logits of a one-token decode step formed in the
 // decode kernel from the layer's input row (GatedDeltaNet._gates,
 // linear_attention.py:719-721, :734-735): p = W_a x and W_b x rounded to the
-// element type (nn.Linear's output), g = neg_a softplus(p + dt_bias), beta = the
+// element type (nn.Linear's output), g = -exp(A_log) softplus(p + dt_bias), beta = the
 // rounded W_b x (logits).  x NULL: g and beta come in as tensors.
 struct GateProj {
     const void *x;                // [n_tokens, dim] in the element type, 16-byte aligned rows
-    const void *w;                // [H, dim] W_a, then [H, dim] W_b (delta rule), 16-byte aligned rows
-    const float *neg_a;           // [H]: -exp(A_log)
-    const float *dt_bias;         // [H]
+    const void *wa, *wb;          // [H, dim] each (wb: delta rule), 16-byte aligned rows
+    const float *neg_a;           // [H]: -exp(A_log); NULL: formed from a_log
+    const void *a_log;            // [H], of type RecParams::param_dtype
+    const void *dt_bias;          // [H], of type RecParams::param_dtype
     int dim;                      // a multiple of 8
 };
 
@@ -230,6 +249,7 @@ struct RecParams {
     int H, n_seqs;
     int use_delta;
     float scale;
+    int param_dtype;              // decode step: of gp.a_log, gp.dt_bias, fz.A_log and fz.dt_bias (0 fp32, 1 bf16, 2 fp16)
     Fusion fz;
     Epilogue ep;                  // applied to o before it is stored
     ShortConv cv;                 // applied to q, k, v where they are read
@@ -312,6 +332,8 @@ hipError_t rms_norm(int dtype, const void *x, const void *res, void *x_out, cons
 // beta [rows, H] (fp32, with_beta).  dim % (16 / sizeof(E)) == 0.
 hipError_t scalar_gates(int dtype, const void *x, const void *w, const float *neg_a, const float *dt_bias, float *g,
                         float *beta, int64_t rows, int dim, int H, bool with_beta, hipStream_t stream);
+
+hipError_t project_rows(int dtype, const ProjectParams &p, hipStream_t stream);
 
 // SiLU(x[:, :h]) * x[:, h:] over rows of 2h elements; h % (16 / sizeof(E)) == 0.
 hipError_t swiglu(int dtype, const void *x, void *y, int64_t rows, int hidden, hipStream_t stream);

@@ -445,11 +445,14 @@ decode_conv_kernel(const RecParams p) {
     constexpr int GVE = 16 / (int)sizeof(E), GU = 2;
     typedef E GV __attribute__((ext_vector_type(GVE)));
     GV gxv[GU], gav[GU], gbv[GU];
+    float ga = 0.f, gd = 0.f;                                 // -exp(A_log) (its A_log), dt_bias
     if (gproj) {
+        ga = p.gp.neg_a ? p.gp.neg_a[h] : param_f(p.gp.a_log, p.param_dtype, h);
+        gd = param_f(p.gp.dt_bias, p.param_dtype, h);
         const int nu = p.gp.dim / GVE;
         const E *xr = reinterpret_cast<const E *>(p.gp.x) + t * (int64_t)p.gp.dim;
-        const E *wa = reinterpret_cast<const E *>(p.gp.w) + (int64_t)h * p.gp.dim;
-        const E *wb = wa + (int64_t)H * p.gp.dim;
+        const E *wa = reinterpret_cast<const E *>(p.gp.wa) + (int64_t)h * p.gp.dim;
+        const E *wb = reinterpret_cast<const E *>(p.gp.wb) + (int64_t)h * p.gp.dim;
         const bool wbeta = !WR && p.use_delta;
 #pragma unroll
         for (int i = 0; i < GU; ++i) {
@@ -520,9 +523,11 @@ decode_conv_kernel(const RecParams p) {
         float a = 1.f;
         if constexpr (GATE == 2) {
             const float gf = p.fz.gate_act && p.fz.gate_16 ? bits_to_f<E>(gr) : __uint_as_float(gr);
-            const float gl = p.fz.gate_act ? gate_activation(gf, p.fz.A_log[h], p.fz.dt_bias[(int64_t)h * DK + tid],
-                                                             p.fz.lb_set, p.fz.lb)
-                                           : gf;
+            const float gl = p.fz.gate_act
+                                 ? gate_activation(gf, param_f(p.fz.A_log, p.param_dtype, h),
+                                                   param_f(p.fz.dt_bias, p.param_dtype, (int64_t)h * DK + tid),
+                                                   p.fz.lb_set, p.fz.lb)
+                                 : gf;
             a = __expf(gl);
             gv[tid] = a;
             kr[tid] = kv;
@@ -547,7 +552,7 @@ decode_conv_kernel(const RecParams p) {
                 sb += gpart[w][1];
             }
             // nn.Linear's outputs in the element type, then the gate (fp32)
-            gsc = p.gp.neg_a[h] * softplus_acc(EL::to_f(EL::from_f(sa)) + p.gp.dt_bias[h]);
+            gsc = (p.gp.neg_a ? ga : -expf(ga)) * softplus_acc(EL::to_f(EL::from_f(sa)) + gd);
             bsc = EL::to_f(EL::from_f(sb));
         }
         sc[0] = (GATE == 1 && (p.g || gproj)) ? __expf(gsc) : 1.f;

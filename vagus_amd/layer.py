@@ -457,80 +457,45 @@ class GatedDeltaNet(nn.Module):
         return (self.short_conv_size is not None and self.key_head_dim in (64, 128)
                 and (self.value_head_dim in (64, 128) or (self.value_head_dim == 256 and self.short_conv_size == 4)))
 
-    def _decode_weights(self, stacked):
-        """The one-token decode step's projection weights regrouped, rebuilt
-        whenever a parameter changed (its storage or version): `stacked`, every matrix
-        that multiplies the input (W_q, W_k, W_v, W_g, and without the scalar
-        gate W_a1 and W_b), as one weight, rows padded with zeros to a
-        multiple of 64 (so that the rows of its product stay 16-byte aligned),
-        so that one GEMM replaces up to six skinny ones; for the
-        scalar gate [W_a; W_b] as one (2H, dim) weight (W_a alone without the
-        delta rule), which the decode kernel multiplies itself; and the gate's
-        constants in fp32: -exp(A_log) (scalar) or A_log (per channel), and dt_bias.
-        The copies hold one more set of these weights."""
-        scalar = self.gate == 'scalar'
-        ps, n = list(stacked), len(stacked)
-        if scalar:
-            ps += [self.wa.weight] + ([self.wb.weight] if self.delta else [])
-        if self.gate != 'none':
-            ps += [self.A_log, self.dt_bias]
-        key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in ps)
-        c = self.__dict__.get('_decode_w')
-        if c is None or c[0] != key:
-            w = torch.cat(ps[:n])
-            w = F.pad(w, (0, 0, 0, -w.shape[0] % 64)).contiguous()
-            wab = torch.cat(ps[n:-2]).contiguous() if scalar else None
-            gconst = None
-            if self.gate != 'none':
-                gconst = (-self.A_log.float().exp() if scalar else self.A_log.float(), self.dt_bias.float())
-            c = (key, w, wab, gconst)
-            self.__dict__['_decode_w'] = c
-        return c[1:]
-
     def _decode_inputs(self, x):
-        """(qp, kp, vp, out_gate, g, beta, gate_proj, gate constants) for the
-        one-token decode kernel: the projections of x (B, 1, dim), the KDA gate's
-        pre-activation and the beta logits, from one GEMM over the stacked
-        weight of _decode_weights (W_a2 follows as its own); the kernel reads
-        q, k, v and the output gate in place, as column blocks of the product's rows.
-        With the scalar gate, g and beta are None and gate_proj = (x, [W_a; W_b],
-        -exp(A_log), dt_bias): the decode kernel forms them itself.  The values
-        are those of the separate projections and of _gates(raw_gate=vector,
-        raw_beta=delta) up to the GEMMs' summation order.  A layer whose
-        projections are not plain nn.Linear modules, or whose _gates is
-        overridden, calls them."""
+        """(qp, kp, vp, out_gate, g, beta, gate_proj) for the one-token decode kernel,
+        from x (B, 1, dim): the projections, the KDA gate's pre-activation and the beta
+        logits.  One launch forms them (ops.project_rows; W_a2 follows as its own)
+        from the weights where they lie, and the kernel reads q, k, v and the output gate in
+        place, as column blocks of its result.  With the scalar gate, g and
+        beta are None and gate_proj = (x, W_a, W_b, A_log, dt_bias): the decode kernel
+        forms them itself.  The values are those of the separate projections and of
+        _gates(raw_gate=vector, raw_beta=delta) up to the sums' order.
+        Projections that are not plain bias-free nn.Linear modules of x's type, an
+        overridden _gates, and batches that the launch does not take are called one
+        by one."""
         B = x.shape[0]
         H, dk, dv = self.head_count, self.key_head_dim, self.value_head_dim
-        names = ('wq', 'wk', 'wv', 'wg') + {'scalar': (), 'vector': ('wa1',), 'none': ()}[self.gate]
-        if self.delta and self.gate != 'scalar':
-            names += ('wb',)
-        mods = [self._modules[n] for n in names]
+        vec, scalar = self.gate == 'vector', self.gate == 'scalar'
+        names = self._input_projections()
+        mods = [self._modules.get(n) for n in names]
+        x2 = x.reshape(B, -1)
         # the modules' own parameter tables: an attribute of a module is a search, and an eager step takes 120 us
-        ws = [m._parameters.get('weight') for m in mods]
-        if not (type(self)._gates is GatedDeltaNet._gates
-                and all(_plain_module(m, nn.Linear) and m._parameters.get('bias') is None
-                        and w is not None and w.dtype == x.dtype for m, w in zip(mods, ws))):
-            g, beta = self._gates(x, raw_gate=self.gate == 'vector', raw_beta=self.delta)
-            return (self.wq(x), self.wk(x), self.wv(x), self.wg(x), g,
-                    beta if self.delta else None, None, (self.A_log, self.dt_bias) if self.gate == 'vector' else None)
-        w, wab, gconst = self._decode_weights(ws)
-        y = F.linear(x.reshape(B, -1), w)
-        # one view per column block (a slice and its reshape are two calls, of the 130 us of an eager step)
-        nk, nv = H * dk, H * dv
-        row, at = y.stride(0), y.storage_offset()
-        qp, kp = y.as_strided((B, 1, nk), (row, nk, 1), at), y.as_strided((B, 1, nk), (row, nk, 1), at + nk)
-        at += 2 * nk
-        vp, og = y.as_strided((B, 1, nv), (row, nv, 1), at), y.as_strided((B, 1, nv), (row, nv, 1), at + nv)
-        if self.gate == 'scalar':
-            return qp, kp, vp, og, None, None, (x, wab, *gconst), None
-        at += 2 * nv
-        g = beta = None
-        if self.gate == 'vector':
-            g = self.wa2(y.as_strided((B, self.gate_rank), (row, 1), at)).view(B, 1, H, dk)
-            at += self.gate_rank
-        if self.delta:
-            beta = y.as_strided((B, 1, H), (row, H, 1), at)
-        return qp, kp, vp, og, g, beta, None, gconst
+        if (type(self)._gates is GatedDeltaNet._gates
+                and all(_plain_module(m, nn.Linear) and m._parameters.get('bias') is None for m in mods)):
+            w = {n: m._parameters.get('weight') for n, m in zip(names, mods)}
+            if (all(t is not None for t in w.values()) and not torch.is_autocast_enabled('cuda')
+                    and ops.project_rows_fits(x2, list(w.values()))):
+                y, at, beta = ops.project_rows(x2, [w[n] for n in names if n not in ('wa', 'wb')],
+                                               None if scalar else w.get('wb'))
+                # one view per column block (a slice and its reshape are two calls)
+                ld, off = y.stride(0), y.storage_offset()
+                qp, kp, vp, og = (y.as_strided((B, 1, n), (ld, n, 1), off + c)
+                                  for n, c in zip((H * dk, H * dk, H * dv, H * dv), at))
+                if scalar:
+                    return qp, kp, vp, og, None, None, (x, w['wa'], w.get('wb'), self.A_log, self.dt_bias)
+                g = None
+                if vec:
+                    f = y.as_strided((B, w['wa1'].shape[0]), (ld, 1), off + at[4])
+                    g = self.wa2(f).view(B, 1, H, dk)
+                return qp, kp, vp, og, g, None if beta is None else beta.view(B, 1, H), None
+        g, beta = self._gates(x, raw_gate=vec, raw_beta=self.delta)
+        return self.wq(x), self.wk(x), self.wv(x), self.wg(x), g, beta if self.delta else None, None
 
     @torch.no_grad()
     def decode_step(self, x):
@@ -547,12 +512,12 @@ class GatedDeltaNet(nn.Module):
         H, dk, dv = self.head_count, self.key_head_dim, self.value_head_dim
         if L == 1 and type(self)._write is GatedDeltaNet._write and self._decode_kernel_fits():
             vec = self.gate == 'vector'
-            qp, kp, vp, og, g, beta, gp, gc = self._decode_inputs(x)
+            qp, kp, vp, og, g, beta, gp = self._decode_inputs(x)
             o = ops.hip_decode_step(qp, kp, vp, g, beta, self.state, scale=self.scale, delta=self.delta,
                                     gate_proj=gp,
                                     conv_weights=self._conv_weights(), conv_cache=self._caches(), l2norm=True,
                                     beta_logits=self.delta, gate_in_kernel=vec,
-                                    A_log=gc[0] if vec else None, dt_bias=gc[1] if vec else None,
+                                    A_log=self.A_log if vec else None, dt_bias=self.dt_bias if vec else None,
                                     lower_bound=self.gate_lower_bound, out_gate=og,
                                     out_norm_weight=self.o_norm.gamma, out_norm_eps=self.o_norm.eps)
             self.cache_len += L

@@ -323,16 +323,12 @@ class RaggedGenerator:
     def _fingerprint(self) -> tuple:
         """What a recorded decode step holds by address: every parameter
         (storage and version: load_state_dict, an optimizer step or .to()
-        change one of them), each layer's state and conv-cache buffers, and
-        the regrouped decode weights.  A replay is valid only while this is
-        unchanged."""
+        change one of them) and each layer's state and conv-cache buffers.  A
+        replay is valid only while the addresses are unchanged."""
         key = [(p.data_ptr(), p._version) for p in self.model.parameters()]
         for blk in self.model.blocks:
             att = blk.att
             key += [(t.data_ptr(), t.dtype) for t in (att.state,) + (att._caches() if att.short_conv_size else ())]
-            c = att.__dict__.get('_decode_w')
-            key.append(None if c is None else tuple(None if t is None else t.data_ptr()
-                                                    for t in (c[1], c[2]) + (c[3] or ())))
         return tuple(key)
 
     @torch.no_grad()

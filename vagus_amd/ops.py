@@ -43,6 +43,7 @@ _DTYPES = {torch.float32: _lib.VGDR_F32, torch.bfloat16: _lib.VGDR_BF16, torch.f
 _CHUNK_TILE_DV = 16          # the chunk kernel takes dv in multiples of 16
 _REC_DVS = (64, 128)         # the recurrent kernel's column widths
 _DEC_DVS = (64, 128, 256)    # the one-token decode step with the short conv (one kernel)
+_PROJECT_ROWS = 256          # rows that project_rows takes
 
 
 def _ptr(t):
@@ -231,6 +232,12 @@ def l2norm_rows(x, eps: float = 1e-6):
     return _L2NormRows.apply(x, eps) if _wants_grad(x) else _l2norm_kernel(x, None, eps)
 
 
+def _constants_fit(c, A_log, dt_bias):
+    """Whether a kernel reads these gate constants as they are, beside c (a tensor or a call)."""
+    return (A_log.dtype == dt_bias.dtype and A_log.dtype in _DTYPES and A_log.device == dt_bias.device == c.device
+            and A_log.is_contiguous() and dt_bias.is_contiguous())
+
+
 class _Fusion:
     """The producer fusions of one call (linear_attention.py:457-497 flags)."""
 
@@ -246,11 +253,22 @@ class _Fusion:
     def any(self):
         return self.l2norm or self.beta or self.gate
 
-    def struct(self, c):
-        """(the C struct, tensors it points into) for the padded operands of call c."""
+    def in_place(self, c):
+        """Whether the decode step of call c reads A_log and dt_bias where they lie
+        (vgdr_decode_step_params): in one kernel type, contiguous, unpadded."""
+        return (self.gate and not c.padded and _constants_fit(c, self.A_log, self.dt_bias)
+                and self.A_log.numel() == c.H and self.dt_bias.numel() == c.H * c.dk)
+
+    def struct(self, c, params=True):
+        """(the C struct, tensors it points into) for the padded operands of call c.
+        params=False: A_log and dt_bias go beside it (in_place)."""
         keep = []
         fz = _lib.Fusion(int(self.l2norm), int(self.beta), int(self.gate), _lib.VGDR_F32, None, None, 0, 0.0)
-        if self.gate:
+        if self.gate and not params:
+            fz.gate_dtype = _DTYPES[c.g.dtype]
+            if self.lower_bound is not None:
+                fz.lower_bound_set, fz.lower_bound = 1, float(self.lower_bound)
+        elif self.gate:
             a_log = self.A_log.detach().float().reshape(c.H).contiguous()
             dt = self.dt_bias.detach().float().reshape(c.H, c.dk)
             dt = _aligned(_pad_to(dt, {1: c.dkp}))
@@ -965,6 +983,44 @@ def swiglu(x):
     return y
 
 
+def project_rows_fits(x, ws):
+    """Whether project_rows takes these: GPU tensors of one kernel type, x (rows,
+    dim) of 1 to _PROJECT_ROWS rows, up to eight contiguous weights (n, dim),
+    rows in 16-byte units."""
+    dim = x.shape[-1]
+    return (x.is_cuda and x.dtype in _DTYPES and dim % 8 == 0 and 0 < x.shape[0] <= _PROJECT_ROWS
+            and len(ws) <= 8 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= dim
+            and x.data_ptr() % 16 == 0
+            and all(type(w) in (torch.Tensor, torch.nn.Parameter) and w.dtype == x.dtype and w.device == x.device
+                    and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.shape[1] == dim for w in ws))
+
+
+def project_rows(x, ws, w_b=None):
+    """[F.linear(x, w) for w in ws] for a few rows x (rows, dim) in one launch
+    (vgdr_project_rows; project_rows_fits), as column blocks of one (rows, n)
+    tensor whose first columns are multiples of 8 apart; with w_b also beta
+    (rows, H) = W_b x in fp32 (the logits, rounded to x's type first).  Returns (y, first
+    columns, beta or None).  The weights are read where they lie, at every call.
+    No autograd."""
+    _check_grad(x, *ws, w_b)
+    rows, dim = x.shape
+    dev = x.device
+    at, cols = [], 0
+    for w in ws:
+        at.append(cols)
+        cols += -(-w.shape[0] // 8) * 8
+    y = torch.empty(rows, cols, dtype=x.dtype, device=dev)
+    beta = None if w_b is None else torch.empty(rows, w_b.shape[0], dtype=torch.float32, device=dev)
+    mats = ws if w_b is None else [*ws, w_b]
+    c = len(mats)
+    with torch.cuda.device(dev):
+        _lib.check(_lib.load().vgdr_project_rows(
+            _DTYPES[x.dtype], c, (ctypes.c_void_p * c)(*[w.data_ptr() for w in mats]),
+            (ctypes.c_int64 * c)(*[w.shape[0] for w in mats]), x.data_ptr(), x.stride(0), y.data_ptr(), cols,
+            -1 if beta is None else c - 1, _ptr(beta), rows, dim, _stream(dev)))
+    return y, at, beta
+
+
 class _ShortConv:
     """The q, k, v short conv + SiLU (opt.py:15-93) and its decode caches
     (linear_attention.py:929-941) for one decode call."""
@@ -1060,18 +1116,31 @@ def _recurrent(q, k, v, g, beta, *, gate, delta, scale, initial_state, output_fi
                  and conv.K == 4 and q.shape[1] == 1)
     rows = rows and one_token and (epilogue is None or _row_stride(epilogue.gate.reshape(v.shape)) is not None)
     if gate_proj is not None:
-        # (x, W_ab, -exp(A_log), dt_bias): the decode kernel forms the scalar gate and
-        # beta from x; any other call takes them from the gate kernel first
-        x_, w_, na_, db_ = gate_proj
+        # (x, W_ab, -exp(A_log), dt_bias) or (x, W_a, W_b, A_log, dt_bias): the decode kernel
+        # forms the scalar gate and beta from x; any other call takes them from the gate kernel first
+        live = None
+        if len(gate_proj) == 5:
+            x_, wa_, wb_, A_, db_ = gate_proj
+            ws_ = [wa_, wb_] if delta else [wa_]
+            if (_constants_fit(q, A_, db_)
+                    and all(w.dtype == q.dtype and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in ws_)):
+                live, w_, na_ = (*ws_, A_, db_), wa_, None
+            else:
+                w_, na_ = torch.cat(ws_), -A_.float().exp()
+        else:
+            x_, w_, na_, db_ = gate_proj
         dim = x_.shape[-1]
         fits = (one_token and gate == 'scalar' and x_.dtype == q.dtype and w_.dtype == q.dtype
                 and dim % (16 // q.element_size()) == 0
                 and dim <= 2 * (512 if dv > 128 else 256) * (16 // q.element_size()))
         if fits:
             gp_x = _aligned(x_.reshape(-1, dim))
-            gp_w = _aligned(w_)
-            gp_na, gp_db = na_.float().contiguous(), db_.float().contiguous()
+            if live is None:
+                gp_w = _aligned(w_)
+                gp_na, gp_db = na_.float().contiguous(), db_.float().contiguous()
         else:
+            if live is not None:
+                w_, na_ = torch.cat(live[:-2]), -live[-2].float().exp()
             g, beta = scalar_gates(x_, w_, na_, db_, with_beta=delta)
             g, beta = g.reshape(q.shape[:3]), (beta.reshape(q.shape[:3]) if delta else None)
             gate_proj = None
@@ -1104,7 +1173,15 @@ def _recurrent(q, k, v, g, beta, *, gate, delta, scale, initial_state, output_fi
                                               None if fz is None else ctypes.byref(fz), _stream(c.device)))
             del keep
         elif conv is not None:
-            fz, keep = fusion.struct(c) if fusion.any else (None, None)
+            pm = None
+            if gate_proj is not None and live is not None:
+                pm = _lib.GateParams(x=_ptr(gp_x), w_a=_ptr(live[0]), w_b=_ptr(live[1]) if delta else None,
+                                     A_log=_ptr(live[-2]), dt_bias=_ptr(live[-1]), dim=dim,
+                                     param_dtype=_DTYPES[live[-1].dtype])
+            elif c.ld_qk and fusion.in_place(c):
+                pm = _lib.GateParams(A_log=_ptr(fusion.A_log), dt_bias=_ptr(fusion.dt_bias),
+                                     param_dtype=_DTYPES[fusion.A_log.dtype])
+            fz, keep = fusion.struct(c, params=pm is None) if fusion.any else (None, None)
             ep, keep_ep = (None, None)
             if epilogue is not None:
                 assert epilogue.gate.shape == (c.B, c.T, c.H, c.dv), \
@@ -1114,15 +1191,18 @@ def _recurrent(q, k, v, g, beta, *, gate, delta, scale, initial_state, output_fi
             fzp, scp, epp = (None if fz is None else ctypes.byref(fz)), ctypes.byref(sc), \
                 (None if ep is None else ctypes.byref(ep))
             if c.ld_qk or gate_proj is not None:
-                gp = None
-                if gate_proj is not None:
-                    gp = _lib.GateProj(x=_ptr(gp_x), w=_ptr(gp_w), neg_exp_a=_ptr(gp_na), dt_bias=_ptr(gp_db),
-                                       dim=dim)
-                _lib.check(L.vgdr_decode_step_strided(
-                    _DTYPES[c.dtype], c.gate_kind, int(delta), _ptr(c.q), _ptr(c.k), _ptr(c.v), _ptr(c.g),
-                    _ptr(c.beta), _ptr(o), _ptr(h0), _ptr(S), c.B, c.H, c.dkp, c.dvp, c.ld_qk or c.H * c.dkp,
-                    c.ld_v or c.H * c.dvp, scale, fzp, scp, epp, None if gp is None else ctypes.byref(gp),
-                    _stream(c.device)))
+                args = (_DTYPES[c.dtype], c.gate_kind, int(delta), _ptr(c.q), _ptr(c.k), _ptr(c.v), _ptr(c.g),
+                        _ptr(c.beta), _ptr(o), _ptr(h0), _ptr(S), c.B, c.H, c.dkp, c.dvp, c.ld_qk or c.H * c.dkp,
+                        c.ld_v or c.H * c.dvp, scale, fzp, scp, epp)
+                if pm is not None:
+                    _lib.check(L.vgdr_decode_step_params(*args, ctypes.byref(pm), _stream(c.device)))
+                else:
+                    gp = None
+                    if gate_proj is not None:
+                        gp = _lib.GateProj(x=_ptr(gp_x), w=_ptr(gp_w), neg_exp_a=_ptr(gp_na), dt_bias=_ptr(gp_db),
+                                           dim=dim)
+                    _lib.check(L.vgdr_decode_step_strided(*args, None if gp is None else ctypes.byref(gp),
+                                                          _stream(c.device)))
             else:
                 _lib.check(L.vgdr_decode_step(*head, fzp, scp, epp, _stream(c.device)))
             del keep, keep_ep, keep_sc
@@ -1229,7 +1309,8 @@ def hip_decode_step(qp, kp, vp, g, beta, state, *, scale: float, delta: bool = T
     then reads them in place (vgdr_decode_step_strided) instead of from copies.
     gate_proj (x, W_ab, -exp(A_log), dt_bias), for the scalar gate in place of g
     and beta: x (B, 1, dim) is the layer's input, W_ab [W_a; W_b] (W_a alone
-    without the delta rule); the kernel forms g = -exp(A_log) softplus(W_a x +
+    without the delta rule); or (x, W_a, W_b, A_log, dt_bias), the parameters as the
+    module holds them; the kernel forms g = -exp(A_log) softplus(W_a x +
     dt_bias) and the beta logits W_b x itself (linear_attention.py:719-721,
     :734-735), with nn.Linear's rounding of W_a x and W_b x.  conv_weights (w_q, w_k, w_v): the
     ShortConv weights, (D, 1, K) or (D, K); conv_cache (qp_cache, kp_cache,

@@ -194,7 +194,9 @@ class DecodeGraph:
     receive each replay's outputs (``outputs``).  Run `step` once eagerly
     before recording (that step loads the kernels), as its first real
     decode step.  The kernels issue no memset, so the recorded graph holds
-    kernel launches only."""
+    kernel launches only.  It reads a layer's parameters where they lie: a
+    change in place, however written, reaches the next replay; one that moves a
+    parameter (`p.data = new`, `.to()`) needs a new recording."""
 
     def __init__(self, step):
         self.graph = torch.cuda.CUDAGraph()
