@@ -190,6 +190,19 @@ def _l2norm_kernel(x, dy, eps):
     return out
 
 
+def _differentiable_grads(expression, inputs, needed, cotangents):
+    """The gradients of expression(*inputs) for the inputs that need one (None for the
+    others), differentiable: what a rule's backward returns under create_graph.  The
+    expression runs on aliases of the inputs and is differentiated with respect to
+    those, so that the pass ends there: with respect to the inputs themselves it would go
+    on through their own history, and where one input was computed from another
+    (a weight used twice) count that path here and again upstream."""
+    alias = [t.view_as(t) if n else t for t, n in zip(inputs, needed)]
+    got = iter(torch.autograd.grad(expression(*alias), [a for a, n in zip(alias, needed) if n], cotangents,
+                                   create_graph=True, allow_unused=True))
+    return tuple(next(got) if n else None for n in needed)
+
+
 class _L2NormRows(torch.autograd.Function):
     """y = x r, r = rsqrt(sum x^2 + eps) per (token, head), computed in >= fp32
     and rounded to x's type (linear_attention.py:703-706).  Saves x alone (in its
@@ -209,7 +222,7 @@ class _L2NormRows(torch.autograd.Function):
     def backward(ctx, dy):
         x, = ctx.saved_tensors
         if torch.is_grad_enabled():
-            return torch.autograd.grad(l2norm_expression(x, ctx.eps), x, dy, create_graph=True)[0], None
+            return _differentiable_grads(lambda x: l2norm_expression(x, ctx.eps), (x,), (True,), dy) + (None,)
         if ctx.kernel:
             return _l2norm_kernel(x, dy, ctx.eps), None
         xf = x.to(torch.promote_types(x.dtype, torch.float32))
@@ -875,10 +888,8 @@ class _NormGateRule(torch.autograd.Function):
     def backward(ctx, dy):
         o, gate, gamma = ctx.saved_tensors
         if torch.is_grad_enabled():
-            need = [t for t, n in zip((o, gate, gamma), ctx.needs_input_grad) if n]
-            grads = iter(torch.autograd.grad(norm_gate_expression(o, gate, gamma, ctx.eps), need, dy,
-                                             create_graph=True))
-            return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:3]) + (None,)
+            return _differentiable_grads(lambda *t: norm_gate_expression(*t, ctx.eps), (o, gate, gamma),
+                                         ctx.needs_input_grad[:3], dy) + (None,)
         oa, ga, wa, dya = _aligned(o), _aligned(gate), _aligned(gamma), _aligned(dy)
         do, dgate, dgamma = torch.empty_like(oa), torch.empty_like(ga), torch.empty_like(wa)
         dv = o.shape[-1]
@@ -1418,10 +1429,8 @@ class _ShortConvRule(torch.autograd.Function):
     def backward(ctx, dy):
         x, weight = ctx.saved_tensors
         if torch.is_grad_enabled():
-            need = [t for t, n in zip((x, weight), ctx.needs_input_grad) if n]
-            grads = iter(torch.autograd.grad(short_conv_expression(x, weight, ctx.activation), need, dy,
-                                             create_graph=True))
-            return tuple(next(grads) if n else None for n in ctx.needs_input_grad[:2]) + (None,)
+            return _differentiable_grads(lambda *t: short_conv_expression(*t, ctx.activation), (x, weight),
+                                         ctx.needs_input_grad[:2], dy) + (None,)
         B, T, D = x.shape
         K = weight.shape[-1]
         xa, wa, dya = _aligned(x), _aligned(weight), _aligned(dy)
@@ -1496,11 +1505,10 @@ class _Projections(torch.autograd.Function):
         x, *ws = ctx.saved_tensors
         used = [i for i, d in enumerate(dys) if d is not None]
         if torch.is_grad_enabled():
-            need = [t for t, n in zip((x, *ws), ctx.needs_input_grad) if n]
-            out = torch.autograd.grad([F.linear(x, ws[i]) for i in used], need, [dys[i] for i in used],
-                                      create_graph=True, allow_unused=True)
-            out = iter(out)
-            return tuple(next(out) if n else None for n in ctx.needs_input_grad)
+            if not used:
+                return (None,) * len(ctx.needs_input_grad)
+            return _differentiable_grads(lambda x, *ws: [F.linear(x, ws[i]) for i in used], (x, *ws),
+                                         ctx.needs_input_grad, [dys[i] for i in used])
         flat = {i: dys[i].reshape(-1, dys[i].shape[-1]) for i in used}
         dx = None
         if ctx.needs_input_grad[0]:
