@@ -8,7 +8,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from vagus_amd import ops
-from vagus_amd.layer import GatedDeltaNet
+from vagus_amd.layer import GatedDeltaNet, ShortConv
 
 
 def _layer(gate='scalar', dtype=torch.float32, device='cpu', **kw):
@@ -100,3 +100,32 @@ def test_decode_inputs_call_a_module_that_is_not_plain(change, gate, name, monke
             assert torch.equal(y, w(x))
         assert (g is None) if gate == 'none' else torch.equal(g, want_g)
         assert torch.equal(beta, want_beta)
+
+
+def _conv_bias(conv):
+    conv.bias = nn.Parameter(torch.full((conv.weight.shape[0],), 0.5))
+
+
+def _conv_padding(conv):
+    """A module that pads by itself."""
+    conv.padding = (2,)
+
+
+def _conv_dilation(conv):
+    conv.dilation = (2,)
+
+
+def _conv_stride(conv):
+    conv.stride = (2,)
+
+
+@pytest.mark.parametrize('change', [_conv_bias, _conv_padding, _conv_dilation, _conv_stride], ids=lambda f: f.__name__)
+def test_short_conv_calls_a_conv_of_other_settings(change):
+    """Under autograd the short conv is the module's own call (opt.py:78-80) unless that is
+    the plain causal conv of its weight."""
+    conv = ShortConv(8, 4)
+    x = torch.randn(2, 9, 8, generator=torch.Generator().manual_seed(1))
+    change(conv.conv)
+    want = F.silu(conv.conv(F.pad(x.transpose(1, 2), (3, 0))).transpose(1, 2))
+    got = conv(x, 'silu')
+    assert got.shape == want.shape and torch.equal(got, want)

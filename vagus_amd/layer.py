@@ -123,9 +123,11 @@ class ShortConv(nn.Module):
         """x (B, L, D) -> (B, L, D), causal.  conv_cache (N, K, D): continue
         from it and advance it in place (a multi-token decode block)."""
         if _autograd(x, self.conv.weight) and cu_seqlens is None and conv_cache is None:
-            if _plain_module(self.conv, nn.Conv1d):
-                return ops.short_conv(x, self.conv.weight, activation)
-            # a conv with hooks or of another class: its own call (opt.py:78-80)
+            c = self.conv
+            if (_plain_module(c, nn.Conv1d) and c.bias is None and c.weight.shape == (c.groups, 1, self.kernel)
+                    and (c.stride, c.padding, c.dilation) == ((1,), (0,), (1,))):
+                return ops.short_conv(x, c.weight, activation)
+            # a conv with hooks, of another class or of other settings: its own call (opt.py:78-80)
             y = self.conv(F.pad(x.transpose(1, 2), (self.kernel - 1, 0))).transpose(1, 2)
             return F.silu(y) if activation is not None else y
         y, _ = ops.causal_conv1d(x, self.conv.weight, activation=activation, cu_seqlens=cu_seqlens,
