@@ -129,3 +129,29 @@ def test_short_conv_calls_a_conv_of_other_settings(change):
     want = F.silu(conv.conv(F.pad(x.transpose(1, 2), (3, 0))).transpose(1, 2))
     got = conv(x, 'silu')
     assert got.shape == want.shape and torch.equal(got, want)
+
+
+def test_training_pass_of_a_layer_without_write_strengths(monkeypatch):
+    """A subclass that writes by itself and has no W_b: the training pass groups the projections
+    that are there."""
+    class OwnWrite(GatedDeltaNet):
+        def __init__(self, *args, **kw):
+            super().__init__(*args, **kw)
+            del self.wb
+
+        def _write(self, x, k, g, beta):
+            assert beta is None
+            return None, 0.5 * k
+
+    torch.manual_seed(0)
+    m = OwnWrite(64, 2, 64, 64)
+    monkeypatch.setattr(OwnWrite, '_pick_impl', lambda self, q: 'hip')
+    scans = []
+
+    def scan(q, k, v, g, beta, S0, *, w, **kw):
+        scans.append(w)
+        return v + w.sum(-1, keepdim=True) + g.sum(-1, keepdim=True), S0
+
+    monkeypatch.setattr(ops, 'chunk_scan_vec', scan)
+    m(torch.randn(2, 5, 64)).sum().backward()
+    assert len(scans) == 1 and all(p.grad is not None for n, p in m.named_parameters() if not n.startswith('wq'))

@@ -287,7 +287,7 @@ class GatedDeltaNet(nn.Module):
     def _input_projections(self) -> tuple:
         """The names of the projections that read the layer's input."""
         return ('wq', 'wk', 'wv', 'wg') + {'none': (), 'scalar': ('wa',), 'vector': ('wa1',)}[self.gate] \
-            + (('wb',) if self.delta else ())
+            + (('wb',) if self.delta and hasattr(self, 'wb') else ())
 
     def _plain_projections(self) -> bool:
         """Whether the projections are plain bias-free nn.Linear modules (and the
