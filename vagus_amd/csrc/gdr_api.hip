@@ -176,6 +176,7 @@ void take_segments(vgdr::ChunkParams &p, int dtype, int64_t dk, int64_t dv, int 
     p.seg_nw = s.nw;
     p.seg_s = reinterpret_cast<float *>(at);
     p.seg_m = reinterpret_cast<float *>(at + s.m_off);
+    p.seg_whole = reinterpret_cast<int *>(at + s.whole_off);
 }
 
 // workspace of the backward: the forward's (table, blocks), then each chunk's

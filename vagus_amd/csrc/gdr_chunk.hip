@@ -1460,6 +1460,10 @@ __device__ __forceinline__ typename Elem<E>::frag2 ld_tr_pair(const E *p0, const
     return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// what the walk of a split sequence starts the identity's columns from: they are operands in the element type
+// like the state's, and fp16's normal range ends at 6e-5, where a state of 1,000s still has e^-16 below it
+template <typename E> constexpr float SEG_UNIT = std::is_same<E, _Float16>::value ? 1024.f : 1.f;
+
 // ===========================================================================
 // chunk_pipe_kernel: the chunk recurrence for 16-bit elements, with the
 // outputs computed one chunk behind by waves of their own
@@ -1573,13 +1577,24 @@ chunk_pipe_kernel(const ChunkParams p) {
     int64_t bos, eos;
     seq_bounds(p.geo, seq, bos, eos);
     int64_t cbase = chunk_base(p.geo, seq);
-    if (p.n_segs) {                                           // the segment's own tokens and chunks
+    const int col0 = tile * DVT;
+    bool split = p.n_segs > 0;
+    if (!WALK && p.n_segs > 2) {                              // columns that chunk_segment_kernel could not chain
+        const int *fl = p.seg_whole + ((int64_t)seq * H + h) * (DV / 16) + col0 / 16;
+        int whole = 0;
+#pragma unroll
+        for (int i = 0; i < DVT / 16; ++i) whole |= col0 + 16 * i < DV ? fl[i] : 0;
+        if (__builtin_amdgcn_readfirstlane(whole)) {
+            if (seg > 0) return;
+            split = false;
+        }
+    }
+    if (split) {                                              // the segment's own tokens and chunks
         const int64_t step = (int64_t)p.seg_chunks * CH, end = bos + (seg + 1) * step;
         bos += seg * step;
         eos = end < eos ? end : eos;
         cbase += (int64_t)seg * p.seg_chunks;
     }
-    const int col0 = tile * DVT;
     // WALK: the columns from DV on are the identity's, walked with V = 0: those of seg_m (segment 0 enters
     // from the call's own state and needs none)
     const int ncols = WALK && seg > 0 ? DV + DK : DV;
@@ -1721,7 +1736,7 @@ chunk_pipe_kernel(const ChunkParams p) {
                 leave[t] = seg_state(seg);
                 if (ident[t]) leave[t] = p.seg_m + (((int64_t)seq * (p.n_segs - 2) + seg - 1) * H + h) * DK * DK;
                 if (col >= ncols) leave[t] = nullptr;
-            } else if (p.n_segs) {
+            } else if (split) {
                 if (seg > 0) enter[t] = seg_state(seg - 1);
                 if (seg < p.n_segs - 1) leave[t] = nullptr;
             }
@@ -1735,7 +1750,7 @@ chunk_pipe_kernel(const ChunkParams p) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int row = 16 * kt + 4 * g4 + j;
-                    if (WALK && ident[t]) S[t][kt][j] = row == scol[t] + r16 ? 1.f : 0.f;
+                    if (WALK && ident[t]) S[t][kt][j] = row == scol[t] + r16 ? SEG_UNIT<E> : 0.f;
                     else S[t][kt][j] = (enter[t] && wvalid && (!WALK || scol[t] < DV))
                                            ? enter[t][(int64_t)row * DV + scol[t] + r16] : 0.f;
                 }
@@ -1877,7 +1892,8 @@ chunk_pipe_kernel(const ChunkParams p) {
             for (int kt = 0; kt < NKB; ++kt)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    leave[t][(int64_t)(16 * kt + 4 * g4 + j) * width[t] + scol[t] + r16] = S[t][kt][j];
+                    leave[t][(int64_t)(16 * kt + 4 * g4 + j) * width[t] + scol[t] + r16] =
+                        WALK && ident[t] ? S[t][kt][j] * (1.f / SEG_UNIT<E>) : S[t][kt][j];
         });
         return;
     }
@@ -2061,6 +2077,11 @@ chunk_pipe_kernel(const ChunkParams p) {
 // rows; S_s is passed on through LDS.  Bound by latency (a chain of n_segs - 2 products of 0.5
 // MFLOP a workgroup), so M and U are loaded two segments ahead, into three register sets: about
 // 2 us a segment, 4 with M loaded during the products before.
+// S <- M S + U stands for the serial chain only where M and U are in range: a map that expands
+// (keys or writes of more than a contraction's size) can leave fp32, or an operand's 16 bits in the
+// walk, where the state itself, zero or small, does not. An entry of M above 2 in size (a contraction's are at
+// most 1), or one of M or U that is not finite, marks the workgroup's 16 columns as whole, and the output pass
+// walks those through all segments from the call's own state, as an unsplit call does.
 template <int DK>
 __global__ void __launch_bounds__(4 * DK) __attribute__((amdgpu_waves_per_eu(1, 2)))
 chunk_segment_kernel(const ChunkParams p) {
@@ -2087,7 +2108,12 @@ chunk_segment_kernel(const ChunkParams p) {
     load(x, 0);
     load(y, 1);
     for (int i = tid; i < DK * 16; i += 4 * DK) ST[0][(i & 15) * PITCH + (i >> 4)] = s0[(int64_t)(i >> 4) * p.DV + (i & 15)];
+    int ok = 1;
     auto step = [&](Seg &d, int i) __attribute__((always_inline)) {
+        unroll<NQ>([&](auto q) {
+            unroll<4>([&](auto j) { ok &= fabsf(d.a[q][(int)j]) <= 2.f; });
+        });
+        unroll<4>([&](auto j) { ok &= fabsf(d.u[(int)j]) <= __FLT_MAX__; });
         lds_barrier();
         f32x4 acc = d.u, acc1 = {0.f, 0.f, 0.f, 0.f};
         unroll<NQ>([&](auto q) {
@@ -2109,6 +2135,10 @@ chunk_segment_kernel(const ChunkParams p) {
         load(y, i + 4);
         step(z, i + 2);
     }
+    // segment 0's state enters the chain as it is
+    for (int i = tid; i < DK * 16; i += 4 * DK) ok &= fabsf(s0[(int64_t)(i >> 4) * p.DV + (i & 15)]) <= __FLT_MAX__;
+    ok = __syncthreads_and(ok);
+    if (tid == 0) p.seg_whole[(seq * p.H + h) * tiles + tile] = !ok;
 }
 
 // ===========================================================================
@@ -2285,16 +2315,17 @@ SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64
     s.seg_chunks = (int)((n_chunks + segs - 1) / segs);
     s.n_segs = (int)((n_chunks + s.seg_chunks - 1) / s.seg_chunks);      // >= 2
     s.m_off = units * (s.n_segs - 1) * dk * dv * 4;
-    s.bytes = s.m_off + units * (s.n_segs - 2) * dk * dk * 4;
+    s.whole_off = s.m_off + units * (s.n_segs - 2) * dk * dk * 4;
+    s.bytes = s.whole_off + (s.n_segs > 2 ? units * (dv / 16) * 4 : 0);
     return s;
 }
 
 // units * n_segs output tiles of at most 64 columns fit the chip, so that seg_s holds at most 64 columns
-// a CU; seg_m is largest where one tile holds all of dv
+// a CU and seg_whole an entry for 16 of them; seg_m is largest where one tile holds all of dv
 int64_t chunk_segments_bound(int dtype, int dk, int gate_vector, int64_t n_seqs, int64_t H, int64_t n_chunks, int chunk) {
     const int64_t cus = device_cu_count(), units = n_seqs * H;
     if (!chunk_segments(dtype, dk, gate_vector, n_seqs, H, 16, n_chunks, chunk).n_segs) return 0;
-    return 4 * dk * (64 * cus + units * (cus / units < SEG_MAX ? cus / units : SEG_MAX) * dk);
+    return 4 * dk * (64 * cus + units * (cus / units < SEG_MAX ? cus / units : SEG_MAX) * dk) + 4 * 4 * cus;
 }
 
 int64_t chunk_blocks_bytes(int dtype, int chunk, int64_t chunk_slots, int64_t H, int64_t dk, int gate_vector) {

@@ -147,17 +147,19 @@ struct ChunkParams {
                                   // no outputs (o is not written): the backward's entry-state walk
     // a split sequence (SegPlan): n_segs runs of seg_chunks chunks each, walked side by side.
     // seg_s [n_seqs, n_segs - 1, H, dk, dv]: the entry states of segments 1 ..; seg_m [n_seqs,
-    // n_segs - 2, H, dk, dk]: what segment 1 .. n_segs - 2 makes of its entry state.  seg_nw: the outputs'
-    // tile (16 seg_nw columns).  n_segs 0: not split.
+    // n_segs - 2, H, dk, dk]: what segment 1 .. n_segs - 2 makes of its entry state.  seg_whole [n_seqs, H,
+    // dv / 16]: whether those 16 columns run unsplit after all.  seg_nw: the outputs' tile (16 seg_nw
+    // columns).  n_segs 0: not split.
     int n_segs, seg_chunks, seg_nw;
     float *seg_s, *seg_m;
+    int *seg_whole;
 };
 
 // How a dense 16-bit call with the delta rule splits its sequences (n_segs 0: it does not);
-// m_off, bytes: where seg_m starts after seg_s, and the size of both.
+// m_off, whole_off, bytes: where seg_m and seg_whole start after seg_s, and the size of all three.
 struct SegPlan {
     int n_segs, seg_chunks, nw;
-    int64_t m_off, bytes;
+    int64_t m_off, whole_off, bytes;
 };
 SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64_t H, int64_t dv, int64_t n_chunks,
                        int chunk);
