@@ -141,13 +141,19 @@ const char *vgdr_last_error(void);
  * and chunk_size; contents irrelevant): it holds the per-chunk intermediate
  * products and, for a packed batch, the segment table (see
  * vgdr_varlen_prepare).  Calls sharing one workspace must not overlap.
- * For a dense 16-bit call of few (sequence, head) pairs and more than 8,192
- * tokens (per-channel gate: 4,033 or more) the size includes the states that split sequences leave between their
- * segments; a workspace without room for those is accepted down to the
- * size of the other parts and runs such a call unsplit (equal up to rounding).
+ *
+ * Split sequences.  A dense 16-bit call with the delta rule, of few (sequence,
+ * head) pairs and more than 8,192 tokens a sequence, may walk its sequences in
+ * segments, whose number depends on the sizes, the batch and the GPU: the same
+ * result up to rounding.  Every other call gives each sequence the same bits
+ * alone, in any dense batch and in a packed one.  vgdr_chunk_workspace_size has room for
+ * the segments' states; a workspace of vgdr_chunk_whole_workspace_size, or any
+ * without that room, runs the call unsplit: the caller's choice, call by call.
  */
 int64_t vgdr_chunk_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
                                   int64_t n_seqs, int varlen, int chunk_size);
+int64_t vgdr_chunk_whole_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
+                                        int64_t n_seqs, int varlen, int chunk_size);
 
 int vgdr_chunk_fwd(int dtype, int gate_kind, int use_delta,
                    const void *q, const void *k, const void *v,
@@ -211,7 +217,7 @@ int vgdr_chunk_prep_fused(int dtype, int gate_kind, int use_delta,
  * VGDR_CHUNK_SCRATCH_BYTES long, which exists on every GPU where the library's
  * code object is loaded (its first kernel launch of any entry point there)
  * until the end of the process: every process using the library holds it on
- * each GPU it runs on, whether or not it calls this entry point.  A call whose vgdr_chunk_workspace_size (without the split sequences' states) exceeds it
+ * each GPU it runs on, whether or not it calls this entry point.  A call whose vgdr_chunk_whole_workspace_size exceeds it
  * returns VGDR_ERR_INVALID (use vgdr_chunk_fwd_fused with a workspace).
  * Calls that overlap on one GPU (two streams, two threads) share that array
  * and race; serialise them.  Otherwise the arguments, checks and results are
@@ -263,6 +269,10 @@ int vgdr_chunk_fwd_w(int dtype, const void *q, const void *k, const void *v, con
  */
 int64_t vgdr_chunk_bwd_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
                                       int64_t dv, int64_t n_seqs, int varlen, int chunk_size);
+/* the same without room for split sequences' states (vgdr_chunk_whole_workspace_size): what the saved
+ * backward needs, and the walk of a sequence as a whole in the others and in vgdr_chunk_fwd_saving */
+int64_t vgdr_chunk_bwd_whole_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
+                                            int64_t dv, int64_t n_seqs, int varlen, int chunk_size);
 int vgdr_chunk_bwd(int dtype, int gate_kind,
                    const void *q, const void *k, const void *v, const float *g, const float *beta,
                    const float *initial_state, const void *grad_o, const float *grad_final_state,

@@ -1,5 +1,5 @@
-"""Dense calls of few (sequence, head) pairs and more than 8,192 tokens (per-channel
-gate: 64 chunks or more), whose sequences the chunked scan splits into segments walked side by side: against the
+"""Dense calls of few (sequence, head) pairs and more than 8,192 tokens, whose
+sequences the chunked scan splits into segments walked side by side: against the
 fp64 oracle, and against the same tokens as a packed batch, which is never
 split.  The decays are weak (a few per cent over a whole sequence), so that
 every segment depends on its entry state.
@@ -7,8 +7,6 @@ every segment depends on its entry state.
 Split and unsplit runs round the same quantities to the element type in the
 same places, so their errors are of one size: the split run's may be at most
 1.25 times the unsplit run's."""
-import math
-
 import pytest
 import torch
 
@@ -28,6 +26,15 @@ def inputs(B, T, H, dk, dv, gate, dtype, seed):
                               seed=seed)
     x.g = None if gate == 'none' else 1e-3 * x.g
     return x
+
+
+def segment_bytes(gate, dtype, B, T, H, dk, dv):
+    """What this very call keeps between segments (the backward's workspace size takes dv, and has the plan's own
+    bytes); 0 when it is not split."""
+    L = _lib.load()
+    kind = {'none': _lib.VGDR_GATE_NONE, 'scalar': _lib.VGDR_GATE_SCALAR, 'vector': _lib.VGDR_GATE_VECTOR}[gate]
+    call = ops._DTYPES[dtype], kind, B, T, H, dk, dv, B, 0, 64
+    return L.vgdr_chunk_bwd_workspace_size(*call) - L.vgdr_chunk_bwd_whole_workspace_size(*call)
 
 
 def run(x, gate, packed, grads=None):
@@ -53,20 +60,22 @@ def run(x, gate, packed, grads=None):
     ('scalar', torch.float16, 2, 8257, 2, 64, 48),
     ('none', torch.bfloat16, 1, 9000, 3, 64, 16),
     ('none', torch.float16, 1, 10001, 2, 128, 256),
-    ('vector', torch.bfloat16, 1, 4033, 3, 128, 128),
+    ('vector', torch.bfloat16, 1, 8193, 3, 128, 128),
+    ('vector', torch.bfloat16, 4, 8200, 8, 128, 128),
     ('vector', torch.bfloat16, 4, 4100, 8, 128, 128),
-    ('vector', torch.float16, 1, 4600, 2, 128, 272),
-    ('vector', torch.bfloat16, 2, 4224, 1, 64, 64),
+    ('vector', torch.bfloat16, 1, 4033, 3, 128, 128),
+    ('vector', torch.float16, 1, 8600, 2, 128, 272),
+    ('vector', torch.bfloat16, 2, 8224, 1, 64, 64),
 ])
 def test_split_against_oracle_and_packed(gate, dtype, B, T, H, dk, dv):
-    L = _lib.load()
-    kind = {'none': _lib.VGDR_GATE_NONE, 'scalar': _lib.VGDR_GATE_SCALAR, 'vector': _lib.VGDR_GATE_VECTOR}[gate]
-    size = lambda t: L.vgdr_chunk_workspace_size(1, kind, 1, t, H, dk, 1, 0, 64) / math.ceil(t / 64)  # noqa: E731
-    assert size(T) > size(64), 'this call is not split'
+    assert segment_bytes(gate, dtype, B, T, H, dk, dv) > 0, 'this call is not split'
     x = inputs(B, T, H, dk, dv, gate, dtype, seed=T)
     up = lambda a: None if a is None else a.double()  # noqa: E731
     ref = gdr.recurrent(up(x.q), up(x.k), up(x.v), up(x.g), up(x.beta), x.initial_state.double(), scale=dk ** -0.5)
     split, whole = run(x, gate, False), run(x, gate, True)
+    # two segments have no M and are the unsplit chain in two places at once: the same bits
+    two = segment_bytes(gate, dtype, B, T, H, dk, dv) < 2 * 4 * B * H * dk * dv
+    assert two == (T <= 8192 or B * H == 32) and torch.equal(split[0], whole[0]) == two
     for name, a, b, r in zip(('o', 'S'), split, whole, ref):
         ea, eb = rel(a, r), rel(b, r)
         print(f'[split] {gate} {dtype} {B}x{T}x{H} {dk}/{dv}: {name} {ea:.2e}, unsplit {eb:.2e}', flush=True)
@@ -83,7 +92,8 @@ def test_split_training_pass(gate, dtype, H, dk, dv):
     Each run is within about a rounding of the element type (2^-8, 2^-11) of the exact gradients, so
     the two are within 2.5 of them of each other."""
     tol = 2.5 * (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11)
-    x = inputs(1, 4200 if gate == 'vector' else 8300, H, dk, dv, gate, dtype, seed=9)
+    x = inputs(1, 8300, H, dk, dv, gate, dtype, seed=9)
+    assert segment_bytes(gate, dtype, 1, 8300, H, dk, dv) > 0, 'this call is not split'
     g = torch.Generator().manual_seed(10)
     grads = torch.randn(x.v.shape, generator=g).to(dtype), torch.randn(x.initial_state.shape, generator=g)
     for i, (a, b) in enumerate(zip(run(x, gate, False, grads), run(x, gate, True, grads))):
@@ -100,8 +110,8 @@ def test_workspace_without_room_runs_unsplit():
     y = {n: getattr(x, n).cuda() for n in ('q', 'k', 'v', 'g', 'beta', 'initial_state')}
     L = _lib.load()
     full = L.vgdr_chunk_workspace_size(1, 1, 1, T, H, d, 1, 0, 64)
-    least = T // 64 * L.vgdr_chunk_workspace_size(1, 1, 1, 64, H, d, 1, 0, 64)
-    assert least < full
+    least = L.vgdr_chunk_whole_workspace_size(1, 1, 1, T, H, d, 1, 0, 64)
+    assert least == T // 64 * L.vgdr_chunk_workspace_size(1, 1, 1, 64, H, d, 1, 0, 64) < full
 
     def call(nbytes):
         o, S = torch.empty_like(y['v']), torch.empty_like(y['initial_state'])

@@ -61,6 +61,7 @@ SIGNATURES = {
     'vgdr_version': (_I, []),
     'vgdr_last_error': (ctypes.c_char_p, []),
     'vgdr_chunk_workspace_size': (_L, [_I, _I, _L, _L, _L, _L, _L, _I, _I]),
+    'vgdr_chunk_whole_workspace_size': (_L, [_I, _I, _L, _L, _L, _L, _L, _I, _I]),
     'vgdr_chunk_fwd': (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L,
                             _L, _L, _L, _L, _L, _L, _F, _I, _P]),
     'vgdr_chunk_prep': (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L,
@@ -76,6 +77,7 @@ SIGNATURES = {
     'vgdr_chunk_fwd_w': (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L,
                               _L, _L, _L, _L, _L, _L, _F, _I, _FZ, _P]),
     'vgdr_chunk_bwd_workspace_size': (_L, [_I, _I, _L, _L, _L, _L, _L, _L, _I, _I]),
+    'vgdr_chunk_bwd_whole_workspace_size': (_L, [_I, _I, _L, _L, _L, _L, _L, _L, _I, _I]),
     'vgdr_chunk_bwd': (_I, [_I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L,
                             _L, _L, _L, _L, _L, _L, _F, _I, _P]),
     'vgdr_chunk_bwd_saved': (_I, [_I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L,

@@ -300,6 +300,13 @@ int vgdr_version(void) { return 100; }
 
 const char *vgdr_last_error(void) { return g_err; }
 
+int64_t vgdr_chunk_whole_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
+                                        int64_t n_seqs, int varlen, int chunk_size) {
+    if (B < 0 || T < 0 || H <= 0 || n_seqs < 0) return 0;
+    const int chunk = effective_chunk(dtype, dk, chunk_size);
+    return chunk_layout(dtype, gate_kind, chunk, B, T, H, dk, n_seqs, varlen).total;
+}
+
 int64_t vgdr_chunk_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
                                   int64_t n_seqs, int varlen, int chunk_size) {
     if (B < 0 || T < 0 || H <= 0 || n_seqs < 0) return 0;
@@ -355,6 +362,13 @@ int vgdr_chunk_fwd_w(int dtype, const void *q, const void *k, const void *v, con
                       dv, n_seqs, scale, chunk_size, fusion, stream, w ? w : dummy);
 }
 
+
+int64_t vgdr_chunk_bwd_whole_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
+                                            int64_t dv, int64_t n_seqs, int varlen, int chunk_size) {
+    if (B < 0 || T < 0 || H <= 0 || n_seqs < 0 || dv < 0) return 0;
+    const int chunk = effective_chunk(dtype, dk, chunk_size);
+    return bwd_layout(dtype, gate_kind, chunk, B, T, H, dk, dv, n_seqs, varlen).total;
+}
 
 int64_t vgdr_chunk_bwd_workspace_size(int dtype, int gate_kind, int64_t B, int64_t T, int64_t H, int64_t dk,
                                       int64_t dv, int64_t n_seqs, int varlen, int chunk_size) {

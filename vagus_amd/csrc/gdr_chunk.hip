@@ -2280,20 +2280,23 @@ static int state_waves(int64_t units, int dv, int cus) {
 // Its sequences are split: the segments' effects on the state are walked side by side
 // (launch_segments), their entry states follow from those, and the outputs run over all
 // segments at once.  That is up to 3 state passes' work (2 with two segments, which need no
-// seg_m), so it takes segments enough to pay for it.  Whole calls, unsplit -> split, us (dk = dv = 128):
-//   scalar gate: 16 heads 512 chunks 680 -> 361; 2 heads 510 -> 134; 32 (sequence, head) pairs
-//   256 chunks, 4 segments 400 -> 344, 3: 355, 2: 445 (at least SEG_PAYS); 24 pairs 129 chunks, 5: 171 -> 146;
-//   per-channel gate: 8 heads 256 chunks 355 -> 183; 16 heads 128 chunks, 4 segments 225 -> 174;
-//   32 pairs, 2 segments: 128 chunks 327 -> 293, 64 chunks 157 -> 152; 20 pairs 64 chunks, 3: 109 -> 110.
-// Scalar-gate sequences up to 8,192 tokens stay whole, though the longer of them gain too (2 heads, 64 chunks
-// 77 -> 57): a sequence of that length gives the same bits alone and in a packed batch, which is
-// never split (its lengths are on the GPU), and callers check one against the other.  Below 64 chunks the passes'
-// fixed cost takes the gain (8 heads, 32 chunks: 45 -> 46).
+// seg_m), so it takes segments enough to pay for it.  Whole calls by events, unsplit -> split, us (dk = dv = 128;
+// pairs: (sequence, head) pairs):
+//   scalar gate: 512 chunks, 16 pairs 703 -> 394, 2 pairs 529 -> 164; 256 chunks, 32 pairs (4 segments) 436 -> 371, 3
+//   segments 384, 2: 474 (at least SEG_PAYS); 129 chunks, 24 pairs 190 -> 172, 16: 179 -> 143, 8: 168 -> 112;
+//   per-channel gate: 512 chunks, 2 pairs 533 -> 175; 256 chunks, 8 pairs 379 -> 208, 24 (2 segments) 546 -> 499,
+//   32: 613 -> 566; 129 chunks, 32 pairs 340 -> 314, 24: 302 -> 273, 20: 275 -> 238, 16: 248 -> 191, 4: 176 -> 125.
+// A sequence of up to SEG_WHOLE tokens gives the same bits alone, in any batch and in a packed one, which is never
+// split (its lengths are on the GPU), without the caller asking for it. Two segments keep the bits: the walk over
+// the first is the unsplit chain as far as it goes, and only a third needs M. So per-channel calls from SEG_TWO
+// tokens on take two (32 pairs: 128 chunks 339 -> 315, 64 chunks 183 -> 175; 8 pairs, 128 chunks 184 -> 181, 64: 109 ->
+// 110), and scalar-gate ones, where two do not pay, stay whole, though more segments would gain (2 pairs, 64 chunks 77 -> 57;
+// per channel, 16 pairs, 128 chunks in 4: 225 -> 174). Above, the caller's workspace says (take_segments).
 // 32-column output tiles where they give SEG_NARROW segments, else (scalar gate) 64-column ones with
-// twice the segments: 16 heads 512 chunks 432 us with 32 columns and 4 segments, 361 with 64 and 8.
-// At most SEG_MAX segments: each adds 2 us to the serial chain of entry states (2 heads, 512 chunks: 16
+// twice the segments: 16 pairs 512 chunks 432 us with 32 columns and 4 segments, 361 with 64 and 8.
+// At most SEG_MAX segments: each adds 2 us to the serial chain of entry states (2 pairs, 512 chunks: 16
 // segments 134 us, 24: 158), and none under SEG_TOKENS.
-constexpr int64_t SEG_MAX = 16, SEG_TOKENS = 512, SEG_CALL = 8193, SEG_CALL_VEC = 4096;
+constexpr int64_t SEG_MAX = 16, SEG_TOKENS = 512, SEG_WHOLE = 8192, SEG_TWO = 4096;
 constexpr int64_t SEG_NARROW = 6, SEG_PAYS = 4, SEG_PAYS_VEC = 2;
 
 SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64_t H, int64_t dv, int64_t n_chunks,
@@ -2302,7 +2305,7 @@ SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64
     const int cus = device_cu_count();
     const int64_t units = n_seqs * H, tokens = n_chunks * chunk;
     if (dtype == 0 || units <= 0 || dv <= 0 || units > cus || dv > 32 * cus) return s;
-    if (tokens < (gate_vector ? SEG_CALL_VEC : SEG_CALL)) return s;
+    if (tokens < (gate_vector ? SEG_TWO : SEG_WHOLE + 1)) return s;
     s.nw = 2;
     int64_t segs = cus / (units * ((dv + 31) / 32));
     if (!gate_vector && segs < SEG_NARROW) {
@@ -2311,6 +2314,7 @@ SegPlan chunk_segments(int dtype, int dk, int gate_vector, int64_t n_seqs, int64
     }
     if (segs < (gate_vector ? SEG_PAYS_VEC : SEG_PAYS)) return SegPlan{};
     segs = segs < SEG_MAX ? segs : SEG_MAX;
+    if (tokens <= SEG_WHOLE) segs = 2;
     segs = segs < tokens / SEG_TOKENS ? segs : tokens / SEG_TOKENS;
     s.seg_chunks = (int)((n_chunks + segs - 1) / segs);
     s.n_segs = (int)((n_chunks + s.seg_chunks - 1) / s.seg_chunks);      // >= 2

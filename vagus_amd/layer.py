@@ -139,7 +139,7 @@ class GatedDeltaNet(nn.Module):
     """Gated delta-rule linear attention (GDN: gate='scalar'; KDA:
     gate='vector'; DeltaNet: gate='none'; simple GLA: delta=False) on the HIP
     kernels.  Arguments as the reference's (linear_attention.py:570-592);
-    `impl` also takes 'hip'."""
+    `impl` also takes 'hip', and whole_sequences is the scans' (ops)."""
 
     def __init__(
             self,
@@ -163,6 +163,7 @@ class GatedDeltaNet(nn.Module):
             A_init_range: tuple[float, float] = (1.0, 16.0),
             dt_init_range: tuple[float, float] = (1e-3, 1e-1),
             out_proj: bool = True,
+            whole_sequences: bool = False,
     ):
         super().__init__()
         if isinstance(gate, bool):                     # legacy spelling: True = scalar (GDN)
@@ -191,6 +192,7 @@ class GatedDeltaNet(nn.Module):
         self.impl = impl
         self.fusions = parse_fusions(fused)
         self.disable_recompute = disable_recompute
+        self.whole_sequences = whole_sequences        # ops: no sequence walked in segments
         self.gate_lower_bound = gate_lower_bound
         self.scale = key_head_dim ** -0.5
         self.out_proj = out_proj
@@ -357,7 +359,8 @@ class GatedDeltaNet(nn.Module):
             assert self.delta, 'an explicit write vector needs the delta rule'
             assert g is not None and g.dim() == 4, 'the asymmetric chunk form is implemented for the vector gate'
             return ops.chunk_scan_vec(q, k, v, g, None, S0, scale=self.scale, delta=True,
-                                      chunk_size=self.chunk_size, w=w, cu_seqlens=cu_seqlens)
+                                      chunk_size=self.chunk_size, w=w, cu_seqlens=cu_seqlens,
+                                      whole_sequences=self.whole_sequences)
         self._pick_impl(q)
         return ops.hip_scan(q, k, v, g, beta, S0, scale=self.scale, delta=self.delta,
                             chunk_size=self.chunk_size,
@@ -367,7 +370,8 @@ class GatedDeltaNet(nn.Module):
                             A_log=self.A_log if self.gate != 'none' else None,
                             dt_bias=self.dt_bias if self.gate != 'none' else None,
                             disable_recompute=self.disable_recompute,
-                            lower_bound=self.gate_lower_bound, cu_seqlens=cu_seqlens)
+                            lower_bound=self.gate_lower_bound, cu_seqlens=cu_seqlens,
+                            whole_sequences=self.whole_sequences)
 
     def _output(self, o, x, *, proj: dict | None = None):
         """RMSNorm(o) x SiLU(W_g x) per head, then W_o (:814-825): one HIP pass

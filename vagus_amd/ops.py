@@ -15,6 +15,14 @@ Layouts: q, k (B, T, H, dk); v (B, T, H, dv); g (B, T, H) scalar log-decay
 states (N, H, dk, dv) fp32 with N = B (dense) or the segment count.  o comes
 back in q's dtype.
 
+A sequence gives the same bits alone, in any dense batch and in a packed one, with
+one exception: a dense 16-bit delta-rule call of few (sequence, head) pairs and
+more than 8,192 tokens a sequence is walked in segments whose number depends on the
+batch and the GPU, the same result up to rounding.  whole_sequences=True, on the
+chunked scans that take it and on the layer, leaves it out: every sequence is one
+chain of chunks, at the price of the speed (one 32,768-token sequence of 16
+heads: 674 against 364 us).
+
 The fla flags use_qk_l2norm_in_kernel, use_beta_sigmoid_in_kernel and (KDA)
 use_gate_in_kernel with A_log / dt_bias / lower_bound move the producers'
 elementwise work into the kernels (struct vgdr_fusion): q, k arrive
@@ -402,6 +410,16 @@ def _gate_of(g):
 _VEC_BWD_CHUNK = 64
 
 
+def _workspace(c: _Call, gate_kind, chunk_size, *, bwd: bool, whole: bool):
+    """(a workspace, its bytes) of a chunked call; whole: without room for split
+    sequences' states, so that no sequence is split."""
+    fn = f'vgdr_chunk{"_bwd" if bwd else ""}{"_whole" if whole else ""}_workspace_size'
+    with torch.cuda.device(c.device):
+        nbytes = getattr(_lib.load(), fn)(_DTYPES[c.dtype], gate_kind, c.B, c.T, c.H, c.dkp, *([c.dvp] if bwd else []),
+                                          c.N, int(c.cu is not None), int(chunk_size))
+    return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=c.device), nbytes
+
+
 def _chunk_bwd_covers(q, g, chunk_size):
     """Whether vgdr_chunk_bwd takes this delta-rule call: a scalar gate or
     none at any dtype, a per-channel gate with 16-bit q, k, v (in 64-token
@@ -416,7 +434,8 @@ def _bwd_chunk(q, g, chunk_size):
 
 
 def chunk_gated_delta_rule_bwd(q, k, v, g, beta, initial_state, do, dht=None, *, scale=None, cu_seqlens=None,
-                               chunk_size=64, saved_workspace=None, fusion: _Fusion = _NO_FUSION, delta=True):
+                               chunk_size=64, saved_workspace=None, fusion: _Fusion = _NO_FUSION, delta=True,
+                               whole_sequences=False):
     """Backward of chunk_gated_delta_rule / chunk_kda without autograd
     (vgdr_chunk_bwd): the gradients of (o, final_state) under the cotangents
     do (and dht, None = zero) with respect to q, k, v, g, beta and
@@ -459,13 +478,11 @@ def chunk_gated_delta_rule_bwd(q, k, v, g, beta, initial_state, do, dht=None, *,
     dS0 = new(c.N, c.H, c.dkp, c.dvp) if initial_state is not None else None
     L = _lib.load()
     dtype = _DTYPES[c.dtype]
-    nbytes = L.vgdr_chunk_bwd_workspace_size(dtype, c.gate_kind, c.B, c.T, c.H, c.dkp, c.dvp, c.N,
-                                             int(c.cu is not None), int(chunk_size))
-    if saved_workspace is not None:
-        assert saved_workspace.numel() >= nbytes, 'saved_workspace is smaller than this backward needs'
-        ws, saved = saved_workspace, True
+    saved = saved_workspace is not None
+    if saved:                                                  # nothing is walked again: no segments
+        ws, nbytes = saved_workspace, saved_workspace.numel()
     else:
-        ws, saved = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=c.device), False
+        ws, nbytes = _workspace(c, c.gate_kind, chunk_size, bwd=True, whole=whole_sequences)
     head = (dtype, c.gate_kind, _ptr(c.q), _ptr(c.k), _ptr(c.v), _ptr(c.g), _ptr(c.beta), _ptr(c.h0), _ptr(dop),
             _ptr(dSp), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dg), _ptr(db), _ptr(dS0), _ptr(c.cu), _ptr(ws), nbytes,
             c.B, c.T, c.H, c.dkp, c.dvp, c.N, scale, int(chunk_size))
@@ -500,7 +517,7 @@ def chunk_gated_delta_rule_bwd(q, k, v, g, beta, initial_state, do, dht=None, *,
 
 
 def _chunk_fwd_saving(q, k, v, g, beta, initial_state, *, scale, cu_seqlens, chunk_size,
-                      fusion: _Fusion = _NO_FUSION):
+                      fusion: _Fusion = _NO_FUSION, whole_sequences=False):
     """vgdr_chunk_fwd_saving: the chunked forward (16-bit, any gate, delta
     rule) run in a backward workspace, which keeps the chunk blocks and every
     chunk's entry state for vgdr_chunk_bwd_saved.  fusion: beta logits and
@@ -512,9 +529,7 @@ def _chunk_fwd_saving(q, k, v, g, beta, initial_state, *, scale, cu_seqlens, chu
     o, S = c.new_output(), c.new_state()
     L = _lib.load()
     dtype = _DTYPES[c.dtype]
-    nbytes = L.vgdr_chunk_bwd_workspace_size(dtype, c.gate_kind, c.B, c.T, c.H, c.dkp, c.dvp, c.N,
-                                             int(c.cu is not None), int(chunk_size))
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=c.device)
+    ws, nbytes = _workspace(c, c.gate_kind, chunk_size, bwd=True, whole=whole_sequences)
     head = (dtype, c.gate_kind, _ptr(c.q), _ptr(c.k), _ptr(c.v), _ptr(c.g), _ptr(c.beta), _ptr(o), _ptr(c.h0),
             _ptr(S), _ptr(c.cu), _ptr(ws), nbytes, c.B, c.T, c.H, c.dkp, c.dvp, c.N, float(scale), int(chunk_size))
     with torch.cuda.device(c.device):
@@ -624,12 +639,12 @@ class _ChunkDeltaRule(torch.autograd.Function):
     [0, 1] and g the log-decay."""
 
     @staticmethod
-    def forward(ctx, q, k, v, g, beta, S0, A_log, dt_bias, scale, cu, chunk_size, fusion):
+    def forward(ctx, q, k, v, g, beta, S0, A_log, dt_bias, scale, cu, chunk_size, fusion, whole=False):
         ctx.ws = None
         chunk_size = _bwd_chunk(q, g, chunk_size)
         if q.dtype != torch.float32:
             o, S, ctx.ws = _chunk_fwd_saving(q, k, v, g, beta, S0, scale=scale, cu_seqlens=cu,
-                                             chunk_size=chunk_size, fusion=fusion)
+                                             chunk_size=chunk_size, fusion=fusion, whole_sequences=whole)
         else:
             assert not fusion.any, 'the kernel fusions take 16-bit q, k, v'
             o, S = chunk_scan(q, k, v, g, beta, gate=_gate_of(g), delta=True,
@@ -651,7 +666,7 @@ class _ChunkDeltaRule(torch.autograd.Function):
                                            chunk_size=ctx.chunk_size, saved_workspace=ctx.ws, fusion=fz)
         ctx.ws = None
         dA, ddt = grads[6:] if fz.gate else (None, None)
-        return grads[:6] + (dA, ddt, None, None, None, None)
+        return grads[:6] + (dA, ddt, None, None, None, None, None)
 
 
 class _ChunkPlain(torch.autograd.Function):
@@ -681,7 +696,8 @@ class _ChunkPlain(torch.autograd.Function):
 
 
 def chunk_scan(q, k, v, g, beta, *, gate, delta, scale=None, initial_state=None, output_final_state=False,
-               cu_seqlens=None, chunk_size=64, phase_event=None, fusion: _Fusion = _NO_FUSION):
+               cu_seqlens=None, chunk_size=64, phase_event=None, fusion: _Fusion = _NO_FUSION,
+               whole_sequences=False):
     """Chunkwise prefill, the general form behind chunk_gated_delta_rule,
     chunk_kda and chunk_simple_gla: gate in {'none', 'scalar', 'vector'},
     delta selects the delta rule.  Returns (o, final_state or None).
@@ -690,6 +706,7 @@ def chunk_scan(q, k, v, g, beta, *, gate, delta, scale=None, initial_state=None,
     between the chunk-prep and the chunk-state kernels (the same two launches
     either way), so that a caller can time the two phases separately.
     fusion: the producer fusions (_Fusion).
+    whole_sequences: the module's docstring.
 
     With grads enabled and an input that requires grad, the scan runs through
     _ChunkDeltaRule (delta rule: scalar gate or none, or the per-channel gate
@@ -710,7 +727,7 @@ def chunk_scan(q, k, v, g, beta, *, gate, delta, scale=None, initial_state=None,
             kf = _Fusion(beta=fusion.beta, gate=fusion.gate, A_log=fusion.A_log, dt_bias=fusion.dt_bias,
                          lower_bound=fusion.lower_bound)
             o, S = _ChunkDeltaRule.apply(q, k, v, gk, beta, initial_state, fusion.A_log, fusion.dt_bias, scale,
-                                         cu_seqlens, chunk_size, kf)
+                                         cu_seqlens, chunk_size, kf, whole_sequences)
             return o, (S if output_final_state else None)
         if fusion.beta:
             beta = torch.sigmoid(beta.float())
@@ -724,7 +741,7 @@ def chunk_scan(q, k, v, g, beta, *, gate, delta, scale=None, initial_state=None,
                                    chunk_size, delta)
         else:
             o, S = _ChunkDeltaRule.apply(q, k, v, gk, beta, initial_state, None, None, scale, cu_seqlens, chunk_size,
-                                         _NO_FUSION)
+                                         _NO_FUSION, whole_sequences)
         return o, (S if output_final_state else None)
     c = _Call(q, k, v, g, beta, initial_state, cu_seqlens, gate=gate, delta=delta,
               dv_to=lambda d: -(-d // _CHUNK_TILE_DV) * _CHUNK_TILE_DV, fusion=fusion)
@@ -732,10 +749,7 @@ def chunk_scan(q, k, v, g, beta, *, gate, delta, scale=None, initial_state=None,
     o = c.new_output()
     S = c.new_state() if output_final_state else None
     L = _lib.load()
-    varlen = c.cu is not None
-    nbytes = L.vgdr_chunk_workspace_size(_DTYPES[c.dtype], c.gate_kind, c.B, c.T, c.H, c.dkp, c.N, int(varlen),
-                                         int(chunk_size))
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=c.device)
+    ws, nbytes = _workspace(c, c.gate_kind, chunk_size, bwd=False, whole=whole_sequences)
     with torch.cuda.device(c.device):
         head = (_DTYPES[c.dtype], c.gate_kind, int(delta), _ptr(c.q), _ptr(c.k), _ptr(c.v), _ptr(c.g),
                 _ptr(c.beta), _ptr(o), _ptr(c.h0), _ptr(S), _ptr(c.cu), _ptr(ws), nbytes,
@@ -773,7 +787,8 @@ def _kda_fusion(use_qk_l2norm_in_kernel, use_beta_sigmoid_in_kernel, use_gate_in
 
 def chunk_gated_delta_rule(q, k, v, g, beta, scale=None, initial_state=None,
                            output_final_state=False, cu_seqlens=None, chunk_size=64,
-                           use_qk_l2norm_in_kernel=False, use_beta_sigmoid_in_kernel=False):
+                           use_qk_l2norm_in_kernel=False, use_beta_sigmoid_in_kernel=False, *,
+                           whole_sequences=False):
     """GDN chunkwise prefill (the call at linear_attention.py:487-491).
 
     g: (B, T, H) log-decay (None for DeltaNet, a = 1).  Returns (o, final_state),
@@ -782,13 +797,13 @@ def chunk_gated_delta_rule(q, k, v, g, beta, scale=None, initial_state=None,
     fz = _Fusion(l2norm=use_qk_l2norm_in_kernel, beta=use_beta_sigmoid_in_kernel)
     return chunk_scan(q, k, v, g, beta, gate='scalar' if g is not None else 'none', delta=True,
                   scale=scale, initial_state=initial_state, output_final_state=output_final_state,
-                  cu_seqlens=cu_seqlens, chunk_size=chunk_size, fusion=fz)
+                  cu_seqlens=cu_seqlens, chunk_size=chunk_size, fusion=fz, whole_sequences=whole_sequences)
 
 
 def chunk_kda(q, k, v, g, beta, scale=None, initial_state=None, output_final_state=False,
               cu_seqlens=None, chunk_size=64, use_qk_l2norm_in_kernel=False,
               use_beta_sigmoid_in_kernel=False, use_gate_in_kernel=False, A_log=None, dt_bias=None,
-              safe_gate=False, lower_bound=None, disable_recompute=False):
+              safe_gate=False, lower_bound=None, disable_recompute=False, *, whole_sequences=False):
     """KDA chunkwise prefill (the call at linear_attention.py:474-479).
 
     g: (B, T, H, dk) per-channel log-decay, or with use_gate_in_kernel the gate
@@ -800,7 +815,7 @@ def chunk_kda(q, k, v, g, beta, scale=None, initial_state=None, output_final_sta
                      safe_gate, lower_bound)
     return chunk_scan(q, k, v, g, beta, gate='vector', delta=True, scale=scale,
                   initial_state=initial_state, output_final_state=output_final_state,
-                  cu_seqlens=cu_seqlens, chunk_size=chunk_size, fusion=fz)
+                  cu_seqlens=cu_seqlens, chunk_size=chunk_size, fusion=fz, whole_sequences=whole_sequences)
 
 
 def chunk_simple_gla(q, k, v, g, scale=None, initial_state=None, output_final_state=False,
@@ -1269,7 +1284,7 @@ def fused_recurrent_kda(q, k, v, g, beta, scale=None, initial_state=None, output
 def hip_scan(q, k, v, g, beta, S0, *, scale: float, delta: bool, chunk_size: int = 64,
              l2norm_in_kernel: bool = False, gate_in_kernel: bool = False, beta_in_kernel: bool = False,
              A_log=None, dt_bias=None, disable_recompute: bool = False, lower_bound: float | None = None,
-             cu_seqlens=None):
+             cu_seqlens=None, whole_sequences: bool = False):
     """The contract of fla_scan (linear_attention.py:428-498), flags included:
     chunked scan from entry state S0 (or zeros), always returning (o in
     q.dtype, final S fp32).  g: None, (B, L, H) or (B, L, H, dk) (with
@@ -1284,7 +1299,7 @@ def hip_scan(q, k, v, g, beta, S0, *, scale: float, delta: bool, chunk_size: int
                  dt_bias=dt_bias, lower_bound=lower_bound if gate_in_kernel else None)
     return chunk_scan(q, k, v, g, beta, gate=gate, delta=delta, scale=scale,
                   initial_state=S0, output_final_state=True, cu_seqlens=cu_seqlens,
-                  chunk_size=chunk_size, fusion=fz)
+                  chunk_size=chunk_size, fusion=fz, whole_sequences=whole_sequences)
 
 
 def hip_recurrent(q, k, v, g, beta, S0, *, scale: float, delta: bool, cu_seqlens=None,
@@ -1533,7 +1548,8 @@ def projections(x, *ws):
     return tuple(F.linear(x, w) for w in ws)
 
 
-def chunk_write_bwd(q, k, v, w, g, initial_state, do, dht=None, *, scale=None, cu_seqlens=None, chunk_size=64):
+def chunk_write_bwd(q, k, v, w, g, initial_state, do, dht=None, *, scale=None, cu_seqlens=None, chunk_size=64,
+                    whole_sequences=False):
     """Backward of chunk_scan_vec with explicit write vectors w (B, T, H, dk)
     without autograd (vgdr_chunk_bwd_w; 16-bit q, k, v, w, per-channel g,
     run in 64-token chunks whatever chunk_size asks): the gradients of (o,
@@ -1556,9 +1572,7 @@ def chunk_write_bwd(q, k, v, w, g, initial_state, do, dht=None, *, scale=None, c
     dS0 = new(c.N, c.H, c.dkp, c.dvp) if initial_state is not None else None
     L = _lib.load()
     dtype = _DTYPES[c.dtype]
-    nbytes = L.vgdr_chunk_bwd_workspace_size(dtype, _lib.VGDR_GATE_VECTOR, c.B, c.T, c.H, c.dkp, c.dvp, c.N,
-                                             int(c.cu is not None), int(chunk_size))
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=c.device)
+    ws, nbytes = _workspace(c, _lib.VGDR_GATE_VECTOR, chunk_size, bwd=True, whole=whole_sequences)
     with torch.cuda.device(c.device):
         _lib.check(L.vgdr_chunk_bwd_w(dtype, _ptr(c.q), _ptr(c.k), _ptr(c.v), _ptr(wk), _ptr(c.g), _ptr(c.h0),
                                       _ptr(dop), _ptr(dSp), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dw), _ptr(dg),
@@ -1580,11 +1594,11 @@ class _ChunkWrite(torch.autograd.Function):
     states, in 64-token chunks).  16-bit q, k, v, w, per-channel g."""
 
     @staticmethod
-    def forward(ctx, q, k, v, g, S0, w, scale, cu, chunk_size):
+    def forward(ctx, q, k, v, g, S0, w, scale, cu, chunk_size, whole):
         o, S = chunk_scan_vec(q, k, v, g, None, S0, scale=scale, delta=True, chunk_size=chunk_size, w=w,
-                              cu_seqlens=cu)
+                              cu_seqlens=cu, whole_sequences=whole)
         ctx.save_for_backward(q, k, v, g, S0, w, cu)
-        ctx.scale, ctx.chunk_size = scale, chunk_size
+        ctx.scale, ctx.chunk_size, ctx.whole = scale, chunk_size, whole
         return o, S
 
     @staticmethod
@@ -1593,12 +1607,12 @@ class _ChunkWrite(torch.autograd.Function):
         if do is None:
             do = torch.zeros(*v.shape, dtype=q.dtype, device=q.device)
         dq, dk, dv, dw, dg, dS0 = chunk_write_bwd(q, k, v, w, g, S0, do, dS, scale=ctx.scale, cu_seqlens=cu,
-                                                  chunk_size=_VEC_BWD_CHUNK)
-        return dq, dk, dv, dg, dS0, dw, None, None, None
+                                                  chunk_size=_VEC_BWD_CHUNK, whole_sequences=ctx.whole)
+        return dq, dk, dv, dg, dS0, dw, None, None, None, None
 
 
 def chunk_scan_vec(q, k, v, g, beta, S0, *, scale: float, delta: bool, chunk_size: int = 64, w=None,
-                   cu_seqlens=None):
+                   cu_seqlens=None, whole_sequences: bool = False):
     """The reference's chunk_scan_vec (linear_attention.py:312-425) on the GPU,
     including its explicit write vectors: returns (o in q's dtype, final S fp32).
 
@@ -1620,10 +1634,11 @@ def chunk_scan_vec(q, k, v, g, beta, S0, *, scale: float, delta: bool, chunk_siz
     elif g.dim() == 3:
         g = g.float().unsqueeze(-1).expand(B, T, H, dk)
     if w is not None and _wants_grad(q, k, v, g, beta, S0, w):
-        return _ChunkWrite.apply(q, k, v, g, S0, w, scale, cu_seqlens, chunk_size)
+        return _ChunkWrite.apply(q, k, v, g, S0, w, scale, cu_seqlens, chunk_size, whole_sequences)
     if w is None:
         return chunk_scan(q, k, v, g, beta, gate='vector', delta=delta, scale=scale, initial_state=S0,
-                          output_final_state=True, cu_seqlens=cu_seqlens, chunk_size=chunk_size)
+                          output_final_state=True, cu_seqlens=cu_seqlens, chunk_size=chunk_size,
+                          whole_sequences=whole_sequences)
     assert delta, 'an explicit write vector needs the delta rule'
     assert w.shape == q.shape, f'w must be {tuple(q.shape)} (B, T, H, dk); got {tuple(w.shape)}'
     if q.dtype == torch.float32:
@@ -1636,10 +1651,7 @@ def chunk_scan_vec(q, k, v, g, beta, S0, *, scale: float, delta: bool, chunk_siz
     o = c.new_output()
     S = c.new_state()
     L = _lib.load()
-    varlen = c.cu is not None
-    nbytes = L.vgdr_chunk_workspace_size(_DTYPES[c.dtype], _lib.VGDR_GATE_VECTOR, c.B, c.T, c.H, c.dkp, c.N,
-                                         int(varlen), int(chunk_size))
-    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=c.device)
+    ws, nbytes = _workspace(c, _lib.VGDR_GATE_VECTOR, chunk_size, bwd=False, whole=whole_sequences)
     with torch.cuda.device(c.device):
         _lib.check(L.vgdr_chunk_fwd_w(_DTYPES[c.dtype], _ptr(c.q), _ptr(c.k), _ptr(c.v), _ptr(wk), _ptr(c.g), _ptr(o),
                                       _ptr(c.h0), _ptr(S), _ptr(c.cu), _ptr(ws), nbytes, c.B, c.T, c.H, c.dkp, c.dvp,
