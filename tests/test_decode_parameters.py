@@ -20,9 +20,9 @@ from vagus_amd.layer import GatedDeltaNet
 SIZES = [(64, 128), (128, 128), (128, 256)]
 
 
-def _layer(gate, dk, dv, dtype, device, *, delta=True, H=2, dim=256, seed=0):
+def _layer(gate, dk, dv, dtype, device, *, delta=True, H=2, dim=256, seed=0, rank=20):
     torch.manual_seed(seed)
-    m = GatedDeltaNet(dim=dim, head_count=H, key_head_dim=dk, value_head_dim=dv, gate=gate, delta=delta, gate_rank=20)
+    m = GatedDeltaNet(dim=dim, head_count=H, key_head_dim=dk, value_head_dim=dv, gate=gate, delta=delta, gate_rank=rank)
     for lin in (m.wq, m.wk, m.wv, m.wg):
         torch.nn.init.normal_(lin.weight, std=dim ** -0.5)
     return m.to(device=device, dtype=dtype).eval()
@@ -35,29 +35,37 @@ def _rewrite(m, seed):
         p.data.copy_(p.data.cpu().float() * (0.5 + torch.rand(p.shape, generator=g)))
 
 
+# 300: more streams than the projection kernel takes; with a rank of 22 and two heads the stacked rows are whole 16-byte units,
+# with 20 they are not
 @pytest.mark.parametrize('gate', ['scalar', 'vector', 'none'])
 @pytest.mark.parametrize('dk,dv', SIZES)
-def test_projections_follow_data_writes(gate, dk, dv):
+@pytest.mark.parametrize('streams,rank', [(3, 20), (300, 22), (300, 20)])
+def test_projections_follow_data_writes(gate, dk, dv, streams, rank):
     """On the CPU: the decode step's inputs before and after the change."""
-    m = _layer(gate, dk, dv, torch.float32, 'cpu')
-    x = torch.randn(3, 1, 256, generator=torch.Generator().manual_seed(1))
+    m = _layer(gate, dk, dv, torch.float32, 'cpu', rank=rank)
+    x = torch.randn(streams, 1, 256, generator=torch.Generator().manual_seed(1))
     with torch.no_grad():
         m._decode_inputs(x)
         _rewrite(m, 2)
         got = m._decode_inputs(x)
         for y, w in zip(got, (m.wq, m.wk, m.wv, m.wg)):
             assert torch.allclose(y, w(x), atol=1e-5, rtol=1e-5)
-        assert torch.allclose(got[5].float(), m.wb(x), atol=1e-5, rtol=1e-5)
+        if got[6] is None:                                      # else the decode kernel forms it from the parameters
+            assert torch.allclose(got[5].float(), m.wb(x), atol=1e-5, rtol=1e-5)
+        else:
+            assert gate == 'scalar' and all(a is b for a, b in zip(got[6], (x, m.wa.weight, m.wb.weight, m.A_log, m.dt_bias)))
+        if gate == 'vector':
+            assert torch.allclose(got[4].flatten(2), m.wa2(m.wa1(x)), atol=1e-5, rtol=1e-5)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize('gate,delta', [('scalar', True), ('scalar', False), ('vector', True), ('none', True)])
-@pytest.mark.parametrize('dk,dv', SIZES)
-def test_decode_step_follows_data_writes(dtype, gate, delta, dk, dv):
-    m = _layer(gate, dk, dv, dtype, 'cuda', delta=delta)
-    x = torch.randn(3, 4, 256, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
-    m.reset_cache(3)
+@pytest.mark.parametrize('dk,dv,streams', [(*s, 3) for s in SIZES] + [(128, 128, 300)])
+def test_decode_step_follows_data_writes(dtype, gate, delta, dk, dv, streams):
+    m = _layer(gate, dk, dv, dtype, 'cuda', delta=delta, rank=22)
+    x = torch.randn(streams, 4, 256, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+    m.reset_cache(streams)
     m.decode_step(x[:, :1])
     for t in range(1, 4):
         _rewrite(m, t)
@@ -66,6 +74,25 @@ def test_decode_step_follows_data_writes(dtype, gate, delta, dk, dv):
             del fresh.__dict__[k]                               # nothing that an earlier step left
         assert torch.equal(m.decode_step(x[:, t:t + 1]), fresh.decode_step(x[:, t:t + 1])), t
         assert torch.equal(m.state, fresh.state)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('gate', ['scalar', 'vector', 'none'])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_large_batches_step_as_small_ones(gate, dtype):
+    """More streams than the projection kernel takes, against the same streams in two batches."""
+    m = _layer(gate, 128, 128, dtype, 'cuda', rank=22)
+    x = torch.randn(300, 3, 256, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+
+    def steps(x):
+        m.reset_cache(x.shape[0])
+        y = torch.cat([m.decode_step(x[:, t:t + 1]) for t in range(3)], 1)
+        return y, m.state.clone()
+
+    tol = 1e-5 if dtype == torch.float32 else 2e-2
+    halves = [steps(h) for h in (x[:150], x[150:])]
+    for a, b in zip(steps(x), (torch.cat(t) for t in zip(*halves))):
+        assert ((a.double() - b.double()).norm() / b.double().norm()).item() < tol
 
 
 @pytest.mark.gpu

@@ -51,7 +51,7 @@ _DTYPES = {torch.float32: _lib.VGDR_F32, torch.bfloat16: _lib.VGDR_BF16, torch.f
 _CHUNK_TILE_DV = 16          # the chunk kernel takes dv in multiples of 16
 _REC_DVS = (64, 128)         # the recurrent kernel's column widths
 _DEC_DVS = (64, 128, 256)    # the one-token decode step with the short conv (one kernel)
-_PROJECT_ROWS = 256          # rows that project_rows takes
+_PROJECT_ROWS = 256          # rows that project_rows takes: above, the library's GEMM makes up for stacking the weights
 
 
 def _ptr(t):
