@@ -656,7 +656,7 @@ def write_traffic(run_dir):
 # stamps s_memtime around the state kernel's product stages for eight
 # workgroups: the chain wave's P = K S stage (16 MFMAs, up to X), its TE X
 # stage (6, up to the bf16 W), its state update (16, up to a read of S), and
-# the first output wave's products (22 with 32-column tiles, 11 with 16).
+# the first output wave's products (22 with 32-column tiles).
 # Empty asm statements pin each stage's operands after its first stamp and
 # consume its results before its last, so the products cannot move across the
 # stamps.  A stage's MFMA utilisation is (its MFMAs x 16 cycles) over its
@@ -724,41 +724,49 @@ extern "C" int vgdr_probe_calib(void *dst) {
     return (int)e;
 }
 namespace vgdr {"""),
-    ("""            f32x4 U[NB];
+    ("""            f32x4 U[NS][NB];
             if constexpr (DELTA) {
-                // P = K S (C layout), NB independent accumulation chains""", """            f32x4 U[NB];
-            const int gps = gp_slot(blockIdx.x);
+                // P = K S (C layout), NB independent accumulation chains per strip""", """            f32x4 U[NS][NB];
+            const int gps = WALK ? -1 : gp_slot(blockIdx.x);
             unsigned long long gt0 = 0, gt1 = 0, gt2 = 0, gt3 = 0;
             gt0 = gp_time();
 #pragma unroll
-            for (int q = 0; q < NKB / 2; ++q) asm volatile("" : "+v"(Sb[q]));
+            for (int q = 0; q < NKB / 2; ++q) asm volatile("" : "+v"(Sb[0][q]));
             if constexpr (DELTA) {
-                // P = K S (C layout), NB independent accumulation chains"""),
+                // P = K S (C layout), NB independent accumulation chains per strip"""),
     ("""#pragma unroll
-                for (int I = 0; I < NB; ++I) {
-                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};""", """#pragma unroll
-                for (int q = 0; q < NB / 2; ++q) asm volatile("" :: "v"(Xb[q]));
+                for (int I = 0; I < NB; ++I)
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) {
+                        f32x4 acc = {0.f, 0.f, 0.f, 0.f};""", """#pragma unroll
+                for (int q = 0; q < NB / 2; ++q) asm volatile("" :: "v"(Xb[0][q]));
                 gt1 = gp_time();
 #pragma unroll
-                for (int q = 0; q < NB / 2; ++q) asm volatile("" : "+v"(Xb[q]));
+                for (int q = 0; q < NB / 2; ++q) asm volatile("" : "+v"(Xb[0][q]));
 #pragma unroll
-                for (int I = 0; I < NB; ++I) {
-                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};"""),
+                for (int I = 0; I < NB; ++I)
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) {
+                        f32x4 acc = {0.f, 0.f, 0.f, 0.f};"""),
     ("""            // S <- Gc S + (K*Gend)^T U~
-            if constexpr (VEC) {""", """#pragma unroll
-            for (int q = 0; q < NB / 2; ++q) asm volatile("" :: "v"(Wb[q]));
+#pragma unroll
+            for (int t = 0; t < NS; ++t)""", """#pragma unroll
+            for (int q = 0; q < NB / 2; ++q) asm volatile("" :: "v"(Wb[0][q]));
             gt2 = gp_time();
 #pragma unroll
-            for (int q = 0; q < NB / 2; ++q) asm volatile("" : "+v"(Wb[q]));
+            for (int q = 0; q < NB / 2; ++q) asm volatile("" : "+v"(Wb[0][q]));
             // S <- Gc S + (K*Gend)^T U~
-            if constexpr (VEC) {"""),
-    ("""                                                    Ktr + (32 * q + 16) * PK + KQ::col(16 * kt)), Wb[q], S[kt]);
+#pragma unroll
+            for (int t = 0; t < NS; ++t)"""),
+    ("""                    for (int t = 0; t < NS; ++t) S[t][kt] = mfma_pair(k, Wb[t][q], S[t][kt]);
+                }
         }
-        if (nchunks > 0) lds_barrier();                       // barrier n""", """                                                    Ktr + (32 * q + 16) * PK + KQ::col(16 * kt)), Wb[q], S[kt]);
+        if (nchunks > 0) lds_barrier();                       // barrier n""", """                    for (int t = 0; t < NS; ++t) S[t][kt] = mfma_pair(k, Wb[t][q], S[t][kt]);
+                }
             {
                 float tmp = 0.f;
 #pragma unroll
-                for (int kt = 0; kt < NKB; ++kt) tmp += S[kt][0];
+                for (int kt = 0; kt < NKB; ++kt) tmp += S[0][kt][0];
                 asm volatile("" :: "v"(tmp));
             }
             gt3 = gp_time();
@@ -800,9 +808,18 @@ namespace vgdr {"""),
 ]
 
 
+def probe_source():
+    """gdr_chunk.hip with PROBE_PATCHES applied: each anchor must occur once in the current source."""
+    from vagus_amd import build as b
+    src = open(os.path.join(b.CSRC, 'gdr_chunk.hip')).read()
+    for anchor, repl in PROBE_PATCHES:
+        assert src.count(anchor) == 1, f'probe anchor not found once: {anchor[:60]!r}'
+        src = src.replace(anchor, repl)
+    return src
+
+
 def build_phase_probe(outdir):
-    """The instrumented library: gdr_chunk.hip with PROBE_PATCHES applied (each
-    anchor must occur once in the current source), written to outdir beside
+    """The instrumented library: probe_source() written to outdir beside
     copies of the headers, and the other sources as they are, compiled with
     the library's flags.  Returns the library path."""
     import concurrent.futures as cf
@@ -814,11 +831,7 @@ def build_phase_probe(outdir):
         if f.endswith('.hpp'):
             shutil.copy(os.path.join(b.CSRC, f), os.path.join(outdir, f))
     path = os.path.join(outdir, 'gdr_chunk.hip')
-    src = open(os.path.join(b.CSRC, 'gdr_chunk.hip')).read()
-    for anchor, repl in PROBE_PATCHES:
-        assert src.count(anchor) == 1, f'probe anchor not found once: {anchor[:60]!r}'
-        src = src.replace(anchor, repl)
-    open(path, 'w').write(src)
+    open(path, 'w').write(probe_source())
     # the instrumented file from outdir (beside the headers), every other file from the package
     srcs = [path] + [s for s in b.sources() if os.path.basename(s) != 'gdr_chunk.hip']
     objs = [os.path.join(outdir, os.path.basename(s)[:-4] + '.o') for s in srcs]
@@ -877,6 +890,8 @@ def gemm_phase(torch, workloads, lib_path, name):
         _lib._lib = prev
     a = np.frombuffer(buf, dtype=np.uint64).reshape(8, 128, 8).astype(np.int64)
     nsteps = xs[0].q.shape[1] // CHUNK
+    if gate == 'vector':
+        nsteps //= 2                                           # kda_prefill's sequences are walked in two segments
     a = a[:, :nsteps]
     ok = (a[:, :, 0] > 0) & (a[:, :, 3] > a[:, :, 0]) & (a[:, :, 5] > a[:, :, 4])
     p_st, te_st = (a[:, :, 1] - a[:, :, 0])[ok], (a[:, :, 2] - a[:, :, 1])[ok]
@@ -884,7 +899,7 @@ def gemm_phase(torch, workloads, lib_path, name):
     out = (a[:, :, 5] - a[:, :, 4])[ok]
     step = np.diff(a[:, :, 0], axis=1)[:, 1:-1]
     n = int(ok.sum())
-    n_chain, n_out = 38, (22 if gate == 'scalar' else 11)      # 32-column tiles (gdn_340m) or 16 (kda_prefill)
+    n_chain, n_out = 38, 22                                    # 32-column tiles
     c = 16.0
     frac = lambda m, d: round(m * c * n / float(d.sum()), 4)
     return {'workload': name, 'instrumented_state_us': round(state_us, 1), 'samples': n,
