@@ -1579,7 +1579,7 @@ chunk_pipe_kernel(const ChunkParams p) {
     int64_t cbase = chunk_base(p.geo, seq);
     const int col0 = tile * DVT;
     bool split = p.n_segs > 0;
-    if (!WALK && p.n_segs > 2) {                              // columns that chunk_segment_kernel could not chain
+    if (!WALK && __builtin_expect(p.n_segs > 2, 0)) {         // columns that chunk_segment_kernel could not chain
         const int *fl = p.seg_whole + ((int64_t)seq * H + h) * (DV / 16) + col0 / 16;
         int whole = 0;
 #pragma unroll
