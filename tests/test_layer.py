@@ -14,8 +14,8 @@ GPU:
     reproduces forward; export / load mid-stream is exact; L == 0 is a no-op;
     the layer is causal;
   * ragged packed prefill into cache rows against each sequence alone;
-  * the one-token step's regrouped weight copies follow in-place parameter
-    changes (bit-equal to a layer rebuilt from the changed state);
+  * the one-token step follows in-place parameter changes (bit-equal to a
+    layer rebuilt from the changed state);
   * the explicit-write route (_write returning w) into chunk_scan_vec.
 Bars: rel-L2 <= 2e-2 for bf16 modules, <= 1e-4 for fp32 modules (fp32
 projections and fp32 kernels against the fp64 oracle).
@@ -186,9 +186,8 @@ def test_decode_matches_forward(gate, delta, conv, dtype, dk, dv):
 @pytest.mark.parametrize('gate', ['scalar', 'vector'])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
 def test_decode_weight_copies_follow_the_parameters(gate, dtype):
-    """The one-token decode step reads regrouped copies of its projection
-    weights (and the scalar gate's constants); an in-place change of a
-    parameter between steps must reach the next step.  Two identical layers
+    """An in-place change of a parameter between one-token decode steps must
+    reach the next step.  Two identical layers
     step through the same tokens; one has W_q, W_a (or W_a2), A_log and dt_bias
     changed in place after its first step, the other is rebuilt from that
     state: their later outputs and states are equal."""
@@ -299,8 +298,8 @@ def test_explicit_write_routes_to_chunk_scan_vec(dtype):
 
 @pytest.mark.gpu
 def test_training_forward_differentiates():
-    """With grads, the scan runs its HIP backward and the conv and epilogue
-    their torch expressions: every parameter receives a gradient, and the
+    """With grads, the scan, the conv and the epilogue run their HIP
+    backwards: every parameter receives a gradient, and the
     input gradient matches torch autograd through the oracle composition."""
     m = make('scalar', True, 4, dtype=torch.float32, device='cuda').train()
     x = torch.randn(1, 40, 256, generator=torch.Generator().manual_seed(7)).cuda().requires_grad_(True)
