@@ -413,10 +413,14 @@ _VEC_BWD_CHUNK = 64
 def _workspace(c: _Call, gate_kind, chunk_size, *, bwd: bool, whole: bool):
     """(a workspace, its bytes) of a chunked call; whole: without room for split
     sequences' states, so that no sequence is split."""
-    fn = f'vgdr_chunk{"_bwd" if bwd else ""}{"_whole" if whole else ""}_workspace_size'
-    with torch.cuda.device(c.device):
-        nbytes = getattr(_lib.load(), fn)(_DTYPES[c.dtype], gate_kind, c.B, c.T, c.H, c.dkp, *([c.dvp] if bwd else []),
-                                          c.N, int(c.cu is not None), int(chunk_size))
+    L = _lib.load()
+    head = (_DTYPES[c.dtype], gate_kind, c.B, c.T, c.H, c.dkp)
+    tail = (c.N, int(c.cu is not None), int(chunk_size))
+    if bwd:
+        size = L.vgdr_chunk_bwd_whole_workspace_size if whole else L.vgdr_chunk_bwd_workspace_size
+        nbytes = size(*head, c.dvp, *tail)
+    else:
+        nbytes = (L.vgdr_chunk_whole_workspace_size if whole else L.vgdr_chunk_workspace_size)(*head, *tail)
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=c.device), nbytes
 
 
