@@ -736,7 +736,8 @@ chunk_prep_kernel(const ChunkParams p) {
             // pair each from LDS and Q from global memory, 4 channels at a time, with
             // nothing in flight).  KDA scan of 4 x 8192 tokens, 8 heads, dk = dv = 128, most
             // chunks flagged: bf16 480 -> 449 us, fp16 921 -> 574 us; 1000 tokens, 4 heads:
-            // prep 48 -> 27 to 38 us.  (The tiles below the diagonal on gated operands too,
+            // prep 55 -> 36 us in a kernel trace, while the eager call takes 48 either way
+            // (the host's issue).  (The tiles below the diagonal on gated operands too,
             // as in the fast form, spilled registers: 472 us, and 332 against 305 us
             // for a call with no flagged block.)
             const int sub = r16 >> 2, r0 = 16 * I + 4 * sub;
